@@ -366,7 +366,10 @@ struct Buffers {
     uint16_t* row_part;      // N x kRowPartners: each row's partners ascending, upper then lower
     float4* mf_u;            // terms: u_t of the matrix-free apply
     float4* mf_g;            // 2 per term: J_t^T u_t of the recomputing matrix-free apply
-    float* n2t_w;            // kv1: slot weight of each Node2Term entry's node (sign: several slots)
+    float* n2t_w;            // kv1: slot weight of each Node2Term entry's node (sign: several slots; FP32 recompute)
+    uint2* mf_ent;           // kv1: (term | several slots, slot weight) of each Node2Term entry (mixed mode)
+    float4* mf_edge;         // edges: lever arm of the second end (mixed mode, recomputing apply)
+    float* mf_rec[2];        // 16 N: s, d, node of the matrix-free PCG, read and written in turn (mixed mode)
     // assembly partials of runs crossing 64-entry chunk boundaries
     float* part_diag;        // (kv1 / 64 + 1) x 2 x 27
     float* part_pair;        // (kv2 / 64 + 1) x 2 x 36

@@ -639,94 +639,625 @@ __global__ void __launch_bounds__(256) mfr_coords_kernel(const Buffers* __restri
     }
 }
 
+// ------------------------------------------------------------- mixed mode
+// The same PCG with FP64 sums, three launches per iteration: terms, gather,
+// update.  What bounds them is gathers of a few words per lane, so the data is
+// laid out for wide loads:
+//   terms  : a knn slot's source is one 64-byte record (s, d_prev, node) -- four
+//            16-byte loads where separate arrays took 13 dwords -- and the
+//            direction is formed from it as before;
+//   gather : one wave per node over its Node2Term list, an entry being one 8-byte
+//            record (term, sign bit set when the term names the node in several
+//            slots, and the slot weight) and the term's J and u (stored J) or
+//            g_t (recomputed J); the six sums of a row by a reduce-scatter.  With
+//            16 lanes a row of 450 entries was 28 dependent rounds on 125
+//            workgroups;
+//   update : eight lanes per node, a lane reading its row of M^-1 (48 contiguous
+//            bytes) where a thread per node read 288 on 64 workgroups.
+// Every 32-bit value (d, q, x, r, s, and a term's u, g and products) is rounded
+// where it was, and only FP64 sums are reordered, so the iterates keep their bits.
+// 2k nodes, 220k terms, stored J: gather 127 -> 22 us, terms 14 -> 9, update 8.9 ->
+// 4.8 (10 PCG x 5 GN: 8.2 -> 2.55 ms a frame); 8k nodes, 163k terms, recomputed J:
+// gather 28 -> 14 us, terms 27 -> 20, update 8.9 -> 5.1 (15 x 5: 5.3 -> 3.45 ms).
+// The FP32 mode keeps the kernels above: its sums are 32-bit, their order is part
+// of its results.
+constexpr uint32_t kMfWaves = 8;                      // rows (waves) per gather workgroup
+constexpr uint32_t kMfGroups = kPartialStride;        // partial sums of the gather, at most
+constexpr uint32_t kMfLanes = 8;                      // lanes per node in the update
+constexpr uint32_t kMfNodes = 256 / kMfLanes;         // nodes per update workgroup
+constexpr uint32_t kManySlots = 0x80000000u;
+
+// Partial sums of a frame of N nodes, functions of N alone (a member of a batch
+// sums as it does alone): one per gather workgroup of kMfWaves rows, the rows
+// past kMfGroups of them wrapping around, and one per update workgroup.
+__host__ __device__ inline uint32_t mf_partials(uint32_t nodes) {
+    const uint32_t g = (nodes + kMfWaves - 1) / kMfWaves;
+    return g < kMfGroups ? g : kMfGroups;
+}
+__host__ __device__ inline uint32_t mf_delta_partials(uint32_t nodes) { return (nodes + kMfNodes - 1) / kMfNodes; }
+
+// Value a (lanes 8 k + a, a < 6) of one node's 6-vector, seen by its lanes.
+__device__ inline double node_lane(double v, uint32_t a) { return __shfl(v, (int)((threadIdx.x & 56u) + a), 64); }
+
+// Lane a's component of M^-1 v for the 32-bit vector v.
+__device__ inline float lane_minv(const Buffers& b, uint32_t n, float v, uint32_t a) {
+    const double* M = b.diag_inv64 + 36 * (size_t)n + 6 * (a < 6 ? a : 0);
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s += M[k] * node_lane(v, k);
+    return (float)s;
+}
+
+// The node records read by the terms of iteration k (k & 1): s 0..5, d_{k-1}
+// 6..11, node 12..14; the other set receives d_k and s_{k+1}.
+constexpr uint32_t kNodeRec = 16;
+__device__ inline float* node_recs(const Buffers& b, uint32_t set) { return set & 1 ? b.mf_rec[1] : b.mf_rec[0]; }
+
+// kStart: r = b, d_0 = M^-1 b, x = 0, delta_0.  Otherwise iteration k:
+// alpha = delta_k / dot(d, q); x += alpha d; r -= alpha q; s = M^-1 r; delta_{k+1}.
+template <bool kStart>
+__global__ void __launch_bounds__(256) mf_update_kernel(const Buffers* __restrict__ bs, uint32_t k) {
+    const Buffers b = frame_buffers(bs);
+    const FrameDev& f = *b.frame;
+    double alpha = 0.0;
+    if (!kStart) {
+        double delta, dq;
+        reduce_partials2<double>(slot_ptr(b, kSlotDelta + k), mf_delta_partials(f.N), slot_ptr(b, kSlotDQ + k),
+                                 mf_partials(f.N), delta, dq);
+        alpha = dq != 0.0 ? delta / dq : 0.0;
+    }
+    const uint32_t first = blockIdx.x * kMfNodes;
+    if (b.counts->error || first >= f.N) return;
+    const uint32_t a = threadIdx.x % kMfLanes, n = first + threadIdx.x / kMfLanes;
+    const bool own = n < f.N && a < 6;
+    const uint32_t nn = n < f.N ? n : f.N - 1;
+    const size_t i = 6 * (size_t)nn + (a < 6 ? a : 0);
+    float t;
+    if (kStart) {
+        t = b.jtr[i];
+        if (own) b.x[i] = 0.f;
+    } else {
+        const float x = (float)((double)b.x[i] + alpha * (double)b.d1[i]);
+        t = (float)((double)b.r[i] - alpha * (double)b.q[i]);
+        if (own) b.x[i] = x;
+    }
+    const float s = lane_minv(b, nn, t, a);
+    if (own) {
+        b.r[i] = t;
+        if (kStart) {
+            node_recs(b, 0)[kNodeRec * (size_t)nn + 6 + a] = s;
+            if (a < 3) {
+                const float4 g = f.nodes[nn];
+                const float ga = a == 0 ? g.x : a == 1 ? g.y : g.z;
+                node_recs(b, 0)[kNodeRec * (size_t)nn + 12 + a] = ga;
+                node_recs(b, 1)[kNodeRec * (size_t)nn + 12 + a] = ga;
+            }
+        } else {
+            node_recs(b, k + 1)[kNodeRec * (size_t)nn + a] = s;
+        }
+    }
+    write_partial<double>(b, kStart ? kSlotDelta : kSlotDelta + k + 1, own ? (double)t * (double)s : 0.0);
+}
+
+// x += (num / den) z of a refinement step.
+__global__ void __launch_bounds__(256) mf_refine_step_kernel(const Buffers* __restrict__ bs) {
+    const Buffers b = frame_buffers(bs);
+    const FrameDev& f = *b.frame;
+    double num, den;
+    const uint32_t parts = mf_partials(f.N);
+    reduce_partials2<double>(slot_ptr(b, kSlotRefNum), parts, slot_ptr(b, kSlotRefDen), parts, num, den);
+    if (b.counts->error) return;
+    const double a = den > 0.0 ? num / den : 0.0;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 6 * f.N; i += gridDim.x * blockDim.x)
+        b.x[i] = (float)((double)b.x[i] + a * (double)b.d1[i]);
+}
+
+// Node2Term entries as (term | kManySlots, slot weight of the entry's node; an
+// edge's entries 1 at its first node, 0 at its second).
+__global__ void __launch_bounds__(256) mf_entries_kernel(const Buffers* __restrict__ bs) {
+    const Buffers b = frame_buffers(bs);
+    const FrameDev& f = *b.frame;
+    const Counts& c = *b.counts;
+    if (c.error) return;
+    const TermBounds tb(c);
+    const uint32_t lane = threadIdx.x & 63, waves = gridDim.x * (blockDim.x / 64);
+    for (uint32_t i = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); i < f.N; i += waves) {
+        const uint32_t beg = b.n2t_offset[i], end = b.n2t_offset[i + 1];
+        for (uint32_t e = beg + lane; e < end; e += 64) {
+            const uint32_t t = b.n2t_index[e];
+            uint32_t kk, many;
+            float wi;
+            const int type = type_of(tb, t, kk);
+            if (type == kSmooth) {
+                const ushort2 ij = f.graph[kk];
+                wi = ij.x == i ? 1.f : 0.f;
+                many = ij.x == ij.y ? kManySlots : 0u;
+            } else {
+                ushort4 knn;
+                float4 wk;
+                term_knn(b, type, kk, knn, wk);
+                wi = slot_weight(knn, wk, i);
+                many = (knn.x == i) + (knn.y == i) + (knn.z == i) + (knn.w == i) > 1 ? kManySlots : 0u;
+            }
+            b.mf_ent[e] = make_uint2(t | many, __float_as_uint(wi));
+        }
+    }
+}
+
+// J rows and lambda^2 of a knn term from its record.
+__device__ inline int stored_rows(const Buffers& b, int type, uint32_t kk, const MfLambda2& l2, bool density, float J[3][6],
+                                  float lam[3]) {
+    if (type == kDense || type == kForeground) {
+        const ScalarRec& rec = type == kDense ? b.dense[kk] : b.fg[kk];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) J[0][q] = rec.J[q];
+        lam[0] = type == kDense ? 1.f : l2.foreground;
+        if (type == kDense && density) {
+            const ScalarRec& d = b.density[kk];
+#pragma unroll
+            for (int q = 0; q < 6; ++q) J[1][q] = d.J[q];
+            lam[1] = l2.density;
+            return 2;
+        }
+        return 1;
+    }
+    const P2PRec& rec = type == kFeature ? b.feat[kk] : b.cross[kk];
+    float res[3];
+    p2p_rows(rec, J, res);
+    const uint32_t mask = type == kFeature ? 0xFFFFFFFFu : 0u;
+    lam[0] = lam[1] = lam[2] = __uint_as_float((__float_as_uint(l2.feature) & mask) | (__float_as_uint(l2.cross) & ~mask));
+    return 3;
+}
+
+// kSrc kSrcDir: V from the direction of iteration k, also stored (d1, and the
+// records of the next iteration); kSrcX, kSrcZ: from x or d1; kSrcRows: u_t from
+// mf_u (debug).  Stored J: u_t to mf_u.  Recomputed J: kOutG g_t, kOutRows u_t.
+// An edge of the recomputing apply leaves lambda^2 u and its two lever arms
+// (zero when it is not valid) for the gather: mf_g = (u, valid; a), mf_edge = b.
+template <bool kRecompute, int kSrc, int kOut>
+__global__ void __launch_bounds__(256) mf_apply_terms_kernel(const Buffers* __restrict__ bs, uint32_t k, Penalty pen,
+                                                             uint32_t which) {
+    const Buffers b = frame_buffers(bs);
+    const FrameDev& f = *b.frame;
+    const Counts& c = *b.counts;
+    if (c.error) return;
+    double beta = 0.0, num = 0.0, den = 0.0;
+    if (kSrc == kSrcDir && k > 0) {
+        const uint32_t parts = mf_delta_partials(f.N);
+        partials_sum2<double>(slot_ptr(b, kSlotDelta + k), parts, slot_ptr(b, kSlotDelta + k - 1), parts, num, den);
+    }
+    const DQ* __restrict__ se3 = which ? b.se3[1] : b.se3[0];
+    const float4* __restrict__ recs = reinterpret_cast<const float4*>(node_recs(b, k));
+    const float* __restrict__ vec = kSrc == kSrcX ? b.x : b.d1;
+    // the source vector at node n, node-centred
+    auto source = [&](uint32_t n, float v[6], float4& g) {
+        if (kSrc == kSrcDir) {
+            const float4 q0 = recs[4 * (size_t)n], q1 = recs[4 * (size_t)n + 1], q2 = recs[4 * (size_t)n + 2];
+            g = recs[4 * (size_t)n + 3];
+            const float sv[6] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y};
+            const float pv[6] = {q1.z, q1.w, q2.x, q2.y, q2.z, q2.w};
+#pragma unroll
+            for (int a = 0; a < 6; ++a) v[a] = k > 0 ? (float)((double)sv[a] + beta * (double)pv[a]) : pv[a];
+        } else {
+            g = f.nodes[n];
+            const float2* p = reinterpret_cast<const float2*>(vec + 6 * (size_t)n);
+            const float2 p0 = p[0], p1 = p[1], p2 = p[2];
+            v[0] = p0.x; v[1] = p0.y; v[2] = p1.x; v[3] = p1.y; v[4] = p2.x; v[5] = p2.y;
+        }
+    };
+    const TermBounds tb(c);
+    const MfLambda2 l2 = mf_lambda2(pen);
+    const bool density = b.density && pen.density != 0.f;
+    const uint32_t total = c.off[4];
+    const uint32_t stride = gridDim.x * blockDim.x;
+    // a term's rows, which do not depend on the source ...
+    struct Rows {
+        int type, rows;
+        uint32_t kk;
+        ushort4 knn;
+        float4 wk;
+        float J[3][6], lam[3];
+        SmoothRec sm;
+    };
+    auto rows_of = [&](uint32_t t, Rows& r) {
+        r.type = type_of(tb, t, r.kk);
+        if (r.type == kSmooth) {
+            r.sm = kRecompute ? eval_smooth<double>(f, se3, r.kk) : b.smooth[r.kk];
+        } else {
+            term_knn(b, r.type, r.kk, r.knn, r.wk);
+            r.rows = kRecompute ? knn_term_rows<double>(b, f, se3, r.type, r.kk, l2, density, r.J, r.lam)
+                                : stored_rows(b, r.type, r.kk, l2, density, r.J, r.lam);
+        }
+    };
+    // ... and their product with it
+    auto apply_rows = [&](uint32_t t, const Rows& r) {
+        float u[3] = {0.f, 0.f, 0.f};
+        float4 g0 = make_float4(0.f, 0.f, 0.f, 0.f), g1 = g0;
+        if (kSrc == kSrcRows) {
+            const float4 ut = b.mf_u[t];
+            u[0] = ut.x;
+            u[1] = ut.y;
+            u[2] = ut.z;
+        }
+        if (r.type == kSmooth) {
+            const SmoothRec& sm = r.sm;
+            const float l = kSrc == kSrcRows ? 1.f : l2.smooth;
+            if (kSrc != kSrcRows) {
+                const uint32_t n1 = sm.ij & 0xFFFF, n2 = sm.ij >> 16;
+                float J1[3][6], J2[3][6], res[3], v[6], w1[6], w2[6];
+                float4 g;
+                smooth_rows(sm, true, J1, res);
+                smooth_rows(sm, n2 == n1, J2, res);
+                source(n1, v, g);
+                node_to_ref(g, v, w1);
+                source(n2, v, g);
+                node_to_ref(g, v, w2);
+                if (kRecompute) {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) u[q] = dot6(J1[q], w1) + dot6(J2[q], w2);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) u[q] = l * (dot6(J1[q], w1) + dot6(J2[q], w2));
+                }
+            }
+            if (kRecompute && kOut == kOutG) {
+                const float on = sm.valid ? 1.f : 0.f;
+                g0 = make_float4(l * u[0], l * u[1], l * u[2], on);
+                g1 = make_float4(on * sm.Ti_xj[0], on * sm.Ti_xj[1], on * sm.Ti_xj[2], 0.f);
+                b.mf_edge[r.kk] = make_float4(on * (sm.Ti_xj[0] - sm.r[0]), on * (sm.Ti_xj[1] - sm.r[1]),
+                                              on * (sm.Ti_xj[2] - sm.r[2]), 0.f);
+            }
+        } else {
+            if (kSrc != kSrcRows) {
+                // sum_k w_k T_k v_k over the knn slots (slot-rule weights)
+                float V[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                const uint32_t n[4] = {r.knn.x, r.knn.y, r.knn.z, r.knn.w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float v[6], w6[6];
+                    float4 g;
+                    source(n[q], v, g);
+                    node_to_ref(g, v, w6);
+                    const float ws = slot_weight(r.knn, r.wk, n[q]);
+#pragma unroll
+                    for (int a = 0; a < 6; ++a) V[a] += ws * w6[a];
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    if (q < r.rows) u[q] = kRecompute ? dot6(r.J[q], V) : r.lam[q] * dot6(r.J[q], V);
+            }
+            if (kRecompute && kOut == kOutG) {
+                float g[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    if (q < r.rows) {
+                        const float s = (kSrc == kSrcRows ? 1.f : r.lam[q]) * u[q];
+#pragma unroll
+                        for (int a = 0; a < 6; ++a) g[a] += s * r.J[q][a];
+                    }
+                }
+                g0 = make_float4(g[0], g[1], g[2], g[3]);
+                g1 = make_float4(g[4], g[5], 0.f, 0.f);
+            }
+        }
+        if (kRecompute && kOut == kOutG) {
+            b.mf_g[2 * (size_t)t] = g0;
+            b.mf_g[2 * (size_t)t + 1] = g1;
+        } else {
+            b.mf_u[t] = make_float4(u[0], u[1], u[2], 0.f);
+        }
+    };
+    uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    Rows rows;
+    if (t < total) rows_of(t, rows);  // the first term's rows overlap the reduction
+    if (kSrc == kSrcDir && k > 0) {
+        double s0, s1;
+        partials_finish2<double>(num, den, s0, s1);
+        beta = s1 != 0.0 ? s0 / s1 : 0.0;
+    }
+    while (t < total) {
+        apply_rows(t, rows);
+        t += stride;
+        if (t < total) rows_of(t, rows);
+    }
+    if (kSrc == kSrcDir) {
+        float* next = node_recs(b, k + 1);
+        for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < f.N; n += stride) {
+            float v[6];
+            float4 g;
+            source(n, v, g);
+#pragma unroll
+            for (int a = 0; a < 6; ++a) {
+                b.d1[6 * (size_t)n + a] = v[a];
+                next[kNodeRec * (size_t)n + 6 + a] = v[a];
+            }
+        }
+    }
+}
+
+// One step of a wave's reduction of 2 kHalf values: the lane keeps the half
+// its lane bit names and adds the other lane's copies of it.
+template <int kHalf>
+__device__ inline void reduce_half(double (&v)[8]) {
+    const bool upper = (threadIdx.x & kHalf) != 0;
+#pragma unroll
+    for (int k = 0; k < kHalf; ++k) {
+        const double keep = upper ? v[k + kHalf] : v[k], send = upper ? v[k] : v[k + kHalf];
+        v[k] = keep + __shfl_xor(send, kHalf, 64);
+    }
+}
+
+// y_i over the Node2Term list of row i, then the epilogue: kEpiSpmv (v = d):
+// q and dot(d, q) of iteration k; kEpiResidual (v = x): r = b - A x, z = M^-1 r to
+// d1, (r, z); kEpiCurvature (v = z): (z, A z); kEpiAdjoint: the gather's sum to q.
+template <bool kRecompute, int kEpi>
+__global__ void __launch_bounds__(64 * kMfWaves) mf_apply_gather_kernel(const Buffers* __restrict__ bs, uint32_t k, Penalty pen) {
+    const Buffers b = frame_buffers(bs);
+    const FrameDev& f = *b.frame;
+    const Counts& c = *b.counts;
+    // XCD-aware rows: neighbouring rows share terms and stay in one L2
+    const uint32_t group = xcd_remap(blockIdx.x, gridDim.x, mf_partials(f.N));
+    if (c.error || group == 0xFFFFFFFFu) return;
+    const uint32_t lane = threadIdx.x & 63, a = threadIdx.x % kMfLanes;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const float* __restrict__ vec = kEpi == kEpiResidual ? b.x : b.d1;
+    constexpr bool correct = kEpi != kEpiAdjoint;
+    const TermBounds tb(c);
+    const MfLambda2 l2 = mf_lambda2(pen);
+    const bool density = b.density && pen.density != 0.f;
+    double acc = 0.0;
+    for (uint32_t i = group * kMfWaves + wave; i < f.N; i += kMfGroups * kMfWaves) {
+        const uint32_t beg = b.n2t_offset[i], end = b.n2t_offset[i + 1];
+        const float4 g = f.nodes[i];
+        float vi[6], tv[6];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) vi[q] = correct ? vec[6 * (size_t)i + q] : 0.f;
+        node_to_ref(g, vi, tv);
+        double y[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // kRecompute: in reference coordinates until the row is complete
+        // the next round's entries load while this round's terms do
+        uint2 next = beg + lane < end ? b.mf_ent[beg + lane] : make_uint2(0u, 0u);
+        for (uint32_t e = beg + lane; e < end; e += 64) {
+            const uint2 ent = next;
+            if (e + 64 < end) next = b.mf_ent[e + 64];
+            const uint32_t t = ent.x & ~kManySlots;
+            const bool many = (ent.x & kManySlots) != 0;
+            const float wi = __uint_as_float(ent.y);
+            uint32_t kk;
+            const int type = type_of(tb, t, kk);
+            if (kRecompute) {
+                const float4 g0 = b.mf_g[2 * (size_t)t], g1 = b.mf_g[2 * (size_t)t + 1];
+                if (type == kSmooth) {
+                    // J^T u of one end: rotation p x u, translation u, opposite signs
+                    const bool first = wi != 0.f;
+                    const float4 p = first ? g1 : b.mf_edge[kk];
+                    const float sg = first ? 1.f : -1.f;
+                    const float J[3][6] = {{0.f, sg * p.z, -sg * p.y, g0.w * sg, 0.f, 0.f},
+                                           {-sg * p.z, 0.f, sg * p.x, 0.f, g0.w * sg, 0.f},
+                                           {sg * p.y, -sg * p.x, 0.f, 0.f, 0.f, g0.w * sg}};
+                    const float u[3] = {g0.x, g0.y, g0.z};
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) {
+                        float s = u[r];
+                        if (correct && many) s -= l2.smooth * dot6(J[r], tv);
+#pragma unroll
+                        for (int q = 0; q < 6; ++q) y[q] += (double)(s * J[r][q]);
+                    }
+                } else {
+                    const float gv[6] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y};
+#pragma unroll
+                    for (int q = 0; q < 6; ++q) y[q] += (double)(wi * gv[q]);
+                    if (correct && many) {
+                        // (m - 1) w^2 J^T J v less, J as the evaluation pass stored it
+                        ushort4 knn;
+                        float4 wk;
+                        term_knn(b, type, kk, knn, wk);
+                        const uint32_t mult = (knn.x == i) + (knn.y == i) + (knn.z == i) + (knn.w == i);
+                        float J[3][6], lam[3];
+                        const int rows = stored_rows(b, type, kk, l2, density, J, lam);
+#pragma unroll
+                        for (int r = 0; r < 3; ++r) {
+                            if (r < rows) {
+                                const float s = -(float)(mult - 1) * lam[r] * wi * wi * dot6(J[r], tv);
+#pragma unroll
+                                for (int q = 0; q < 6; ++q) y[q] += (double)(s * J[r][q]);
+                            }
+                        }
+                    }
+                }
+            } else {
+                const float4 ut = b.mf_u[t];
+                const float u[3] = {ut.x, ut.y, ut.z};
+                float J[3][6], lam[3], w = 1.f;
+                uint32_t mult = 1;
+                int rows = 3;
+                if (type == kSmooth) {
+                    float res[3];
+                    smooth_rows(b.smooth[kk], wi != 0.f, J, res);
+                    lam[0] = lam[1] = lam[2] = l2.smooth;
+                    if (many) mult = 2;
+                } else {
+                    rows = stored_rows(b, type, kk, l2, density, J, lam);
+                    w = wi;
+                    if (many) {
+                        ushort4 knn;
+                        float4 wk;
+                        term_knn(b, type, kk, knn, wk);
+                        mult = (knn.x == i) + (knn.y == i) + (knn.z == i) + (knn.w == i);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    if (r < rows) {
+                        to_node_frame(J[r], g);
+                        float s = w * u[r];
+                        if (mult > 1) s -= (float)(mult - 1) * lam[r] * w * w * dot6(J[r], vi);
+#pragma unroll
+                        for (int q = 0; q < 6; ++q) y[q] += (double)(s * J[r][q]);
+                    }
+                }
+            }
+        }
+        reduce_half<4>(y);
+        reduce_half<2>(y);
+        reduce_half<1>(y);
+        double ya = y[0];  // component a over the lanes 8 k + a
+#pragma unroll
+        for (int o = 8; o < 64; o <<= 1) ya += __shfl_xor(ya, o, 64);
+        if (kRecompute) {
+            // to node-centred coordinates: T^T (r, t) = (r + t x g, t)
+            const double t0 = node_lane(ya, 3), t1 = node_lane(ya, 4), t2 = node_lane(ya, 5);
+            ya += a == 0 ? t1 * g.z - t2 * g.y : a == 1 ? t2 * g.x - t0 * g.z : a == 2 ? t0 * g.y - t1 * g.x : 0.0;
+        }
+        if (correct) {
+            // damping 1e-2 T^T T v: T v = (w, v + g x w), T^T (a, b) = (a + b x g, b)
+            const float bx = tv[4] * g.z - tv[5] * g.y, by = tv[5] * g.x - tv[3] * g.z, bz = tv[3] * g.y - tv[4] * g.x;
+            const float damp[6] = {tv[0] + bx, tv[1] + by, tv[2] + bz, tv[3], tv[4], tv[5]};
+            const float da = a == 0 ? damp[0] : a == 1 ? damp[1] : a == 2 ? damp[2] : a == 3 ? damp[3] : a == 4 ? damp[4] : damp[5];
+            ya += (double)(1e-2f * da);
+        }
+        const float va = a == 0 ? vi[0] : a == 1 ? vi[1] : a == 2 ? vi[2] : a == 3 ? vi[3] : a == 4 ? vi[4] : vi[5];
+        const size_t ka = 6 * (size_t)i + (a < 6 ? a : 0);
+        const bool own = lane < 6;
+        if (kEpi == kEpiSpmv || kEpi == kEpiAdjoint) {
+            if (own) b.q[ka] = (float)ya;
+            acc += own ? (double)va * ya : 0.0;
+        } else if (kEpi == kEpiResidual) {
+            const float rr = (float)((double)b.jtr[ka] - ya), z = lane_minv(b, i, rr, a);
+            if (own) {
+                b.r[ka] = rr;
+                b.d1[ka] = z;
+            }
+            acc += own ? (double)rr * (double)z : 0.0;
+        } else {
+            acc += own ? (double)va * ya : 0.0;
+        }
+    }
+    if (kEpi == kEpiAdjoint) return;
+    // the waves' sums in order
+    __shared__ double part[kMfWaves];
+    acc = wave_sum(acc);
+    if (lane == 0) part[wave] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < (int)kMfWaves; ++w) s += part[w];
+        slot_ptr(b, kEpi == kEpiSpmv ? kSlotDQ + k : kEpi == kEpiResidual ? kSlotRefNum : kSlotRefDen)[group] = s;
+    }
+}
+
 // ------------------------------------------------------------- host launch
-void launch_pcg_init(const Batch& B, bool fp64, hipStream_t stream);
-void launch_pcg_update(const Batch& B, bool fp64, uint32_t k, uint32_t spmv_blocks, uint32_t dsel, hipStream_t stream);
-void launch_refine_step(const Batch& B, bool fp64, uint32_t spmv_blocks, hipStream_t stream);
+void launch_pcg_init(const Batch& B, hipStream_t stream);
+void launch_pcg_update(const Batch& B, uint32_t k, uint32_t spmv_blocks, uint32_t dsel, hipStream_t stream);
+void launch_refine_step(const Batch& B, uint32_t spmv_blocks, hipStream_t stream);
 uint32_t row_group_grid(uint32_t nodes);
 
 static uint32_t term_grid(const Batch& B) { return std::min<uint32_t>(std::max<uint32_t>(64 * B.nodes / 256, 64), 2048); }
+// Gather workgroups: one per partial of the largest frame, a multiple of the XCD count.
+static uint32_t gather_grid(const Batch& B) { return (mf_partials(B.nodes) + kXcds - 1) / kXcds * kXcds; }
 
-template <typename Acc>
+// ------------------------------------------------ FP32 mode
 static void mf_apply(const Batch& B, int src_epi, uint32_t k, uint32_t cur, const Penalty& pen, hipStream_t stream) {
-    const uint32_t tg = term_grid(B), sg = row_group_grid(B.nodes);
+    const dim3 tg(term_grid(B), B.frames), sg(row_group_grid(B.nodes), B.frames), wg(256);
     if (src_epi == 0) {
-        hipLaunchKernelGGL((mf_terms_kernel<Acc, kSrcDir>), dim3(tg, B.frames), dim3(256), 0, stream, B.dev, k, cur, pen);
-        hipLaunchKernelGGL((mf_gather_kernel<Acc, kEpiSpmv>), dim3(sg, B.frames), dim3(256), 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_terms_kernel<float, kSrcDir>), tg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_gather_kernel<float, kEpiSpmv>), sg, wg, 0, stream, B.dev, k, cur, pen);
     } else if (src_epi == 1) {
-        hipLaunchKernelGGL((mf_terms_kernel<Acc, kSrcX>), dim3(tg, B.frames), dim3(256), 0, stream, B.dev, k, cur, pen);
-        hipLaunchKernelGGL((mf_gather_kernel<Acc, kEpiResidual>), dim3(sg, B.frames), dim3(256), 0, stream, B.dev, k, cur,
-                           pen);
+        hipLaunchKernelGGL((mf_terms_kernel<float, kSrcX>), tg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_gather_kernel<float, kEpiResidual>), sg, wg, 0, stream, B.dev, k, cur, pen);
     } else {
-        hipLaunchKernelGGL((mf_terms_kernel<Acc, kSrcZ>), dim3(tg, B.frames), dim3(256), 0, stream, B.dev, k, cur, pen);
-        hipLaunchKernelGGL((mf_gather_kernel<Acc, kEpiCurvature>), dim3(sg, B.frames), dim3(256), 0, stream, B.dev, k,
-                           cur, pen);
+        hipLaunchKernelGGL((mf_terms_kernel<float, kSrcZ>), tg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_gather_kernel<float, kEpiCurvature>), sg, wg, 0, stream, B.dev, k, cur, pen);
     }
 }
 
-template <typename Acc, typename R>
 static void mfr_apply(const Batch& B, int src_epi, uint32_t k, uint32_t cur, const Penalty& pen, uint32_t which,
                       hipStream_t stream) {
-    const uint32_t tg = term_grid(B), sg = row_group_grid(B.nodes);
+    const dim3 tg(term_grid(B), B.frames), sg(row_group_grid(B.nodes), B.frames), wg(256);
     if (src_epi == 0) {
-        hipLaunchKernelGGL((mfr_terms_kernel<Acc, R, kSrcDir, kOutG>), dim3(tg, B.frames), dim3(256), 0, stream, B.dev, k,
-                           cur, pen, which);
-        hipLaunchKernelGGL((mfr_gather_kernel<Acc, R, kEpiSpmv>), dim3(sg, B.frames), dim3(256), 0, stream, B.dev, k, cur,
-                           pen, which);
+        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcDir, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiSpmv>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
     } else if (src_epi == 1) {
-        hipLaunchKernelGGL((mfr_terms_kernel<Acc, R, kSrcX, kOutG>), dim3(tg, B.frames), dim3(256), 0, stream, B.dev, k,
-                           cur, pen, which);
-        hipLaunchKernelGGL((mfr_gather_kernel<Acc, R, kEpiResidual>), dim3(sg, B.frames), dim3(256), 0, stream, B.dev, k,
-                           cur, pen, which);
+        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcX, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiResidual>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
     } else {
-        hipLaunchKernelGGL((mfr_terms_kernel<Acc, R, kSrcZ, kOutG>), dim3(tg, B.frames), dim3(256), 0, stream, B.dev, k,
-                           cur, pen, which);
-        hipLaunchKernelGGL((mfr_gather_kernel<Acc, R, kEpiCurvature>), dim3(sg, B.frames), dim3(256), 0, stream, B.dev, k,
-                           cur, pen, which);
+        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcZ, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiCurvature>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
     }
 }
 
-// One apply of either form: fp64 selects FP64 sums and FP64 term geometry
-// (the mixed precision mode), as the evaluation pass.
-static void apply_any(const Batch& B, bool recompute, bool fp64, int src_epi, uint32_t k, uint32_t cur,
-                      const Penalty& pen, uint32_t which, hipStream_t stream) {
+static void apply_fp32(const Batch& B, bool recompute, int src_epi, uint32_t k, uint32_t cur, const Penalty& pen,
+                       uint32_t which, hipStream_t stream) {
+    if (recompute) mfr_apply(B, src_epi, k, cur, pen, which, stream);
+    else mf_apply(B, src_epi, k, cur, pen, stream);
+}
+
+// ------------------------------------------------ mixed mode
+template <int kSrc, int kEpi>
+static void apply_mixed(const Batch& B, bool recompute, uint32_t k, const Penalty& pen, uint32_t which,
+                        hipStream_t stream) {
+    const dim3 tg(std::max<uint32_t>(term_grid(B), 1024), B.frames), gg(gather_grid(B), B.frames), wg(256), ww(64 * kMfWaves);
     if (recompute) {
-        if (fp64) mfr_apply<double, double>(B, src_epi, k, cur, pen, which, stream);
-        else mfr_apply<float, float>(B, src_epi, k, cur, pen, which, stream);
+        hipLaunchKernelGGL((mf_apply_terms_kernel<true, kSrc, kOutG>), tg, wg, 0, stream, B.dev, k, pen, which);
+        hipLaunchKernelGGL((mf_apply_gather_kernel<true, kEpi>), gg, ww, 0, stream, B.dev, k, pen);
     } else {
-        if (fp64) mf_apply<double>(B, src_epi, k, cur, pen, stream);
-        else mf_apply<float>(B, src_epi, k, cur, pen, stream);
+        hipLaunchKernelGGL((mf_apply_terms_kernel<false, kSrc, kOutG>), tg, wg, 0, stream, B.dev, k, pen, which);
+        hipLaunchKernelGGL((mf_apply_gather_kernel<false, kEpi>), gg, ww, 0, stream, B.dev, k, pen);
     }
 }
 
-// Block-Jacobi PCG with the matrix-free apply: per iteration the term pass,
-// the gather (q = A d, dot(d, q)) and the update of the materialized path.
+// Block-Jacobi PCG with the matrix-free apply.
 void launch_pcg_matrix_free(const Batch& B, uint32_t iters, uint32_t refine, bool fp64, const Penalty& pen,
                             bool recompute, uint32_t which, hipStream_t stream) {
-    const uint32_t sg = row_group_grid(B.nodes);
     iters = std::min(iters, kMaxIters);
-    launch_pcg_init(B, fp64, stream);
+    if (fp64) {
+        const dim3 ug(mf_delta_partials(B.nodes), B.frames);
+        hipLaunchKernelGGL(mf_update_kernel<true>, ug, dim3(256), 0, stream, B.dev, 0u);
+        for (uint32_t k = 0; k < iters; ++k) {
+            apply_mixed<kSrcDir, kEpiSpmv>(B, recompute, k, pen, which, stream);
+            hipLaunchKernelGGL(mf_update_kernel<false>, ug, dim3(256), 0, stream, B.dev, k);
+        }
+        for (uint32_t r = 0; r < refine; ++r) {
+            apply_mixed<kSrcX, kEpiResidual>(B, recompute, 0, pen, which, stream);
+            apply_mixed<kSrcZ, kEpiCurvature>(B, recompute, 0, pen, which, stream);
+            hipLaunchKernelGGL(mf_refine_step_kernel, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev);
+        }
+        return;
+    }
+    // FP32: per iteration the term pass, the gather (q = A d, dot(d, q)) and
+    // the update of the materialized path
+    const uint32_t sg = row_group_grid(B.nodes);
+    launch_pcg_init(B, stream);
     uint32_t cur = 0;
     for (uint32_t k = 0; k < iters; ++k) {
-        apply_any(B, recompute, fp64, 0, k, cur, pen, which, stream);
+        apply_fp32(B, recompute, 0, k, cur, pen, which, stream);
         cur ^= 1;
-        launch_pcg_update(B, fp64, k, sg, cur, stream);
+        launch_pcg_update(B, k, sg, cur, stream);
     }
     for (uint32_t r = 0; r < refine; ++r) {
-        apply_any(B, recompute, fp64, 1, 0, 0, pen, which, stream);
-        apply_any(B, recompute, fp64, 2, 0, 0, pen, which, stream);
-        launch_refine_step(B, fp64, sg, stream);
+        apply_fp32(B, recompute, 1, 0, 0, pen, which, stream);
+        apply_fp32(B, recompute, 2, 0, 0, pen, which, stream);
+        launch_refine_step(B, sg, stream);
     }
 }
 
-// One matrix-free apply q = A d (stage timing).
+// One matrix-free apply q = A d (stage timing), d as the last PCG left it.
 void launch_mf_apply_once(const Batch& B, bool fp64, const Penalty& pen, bool recompute, uint32_t which,
                           hipStream_t stream) {
-    apply_any(B, recompute, fp64, 0, 0, 0, pen, which, stream);
+    if (fp64) apply_mixed<kSrcDir, kEpiSpmv>(B, recompute, 0, pen, which, stream);
+    else apply_fp32(B, recompute, 0, 0, 0, pen, which, stream);
 }
 
-void launch_mf_entry_weights(const Batch& B, hipStream_t stream) {
-    hipLaunchKernelGGL(mf_entry_weights_kernel, dim3(row_group_grid(B.nodes), B.frames), dim3(256), 0, stream, B.dev);
+// One PCG update of the mixed matrix-free solve (stage timing).
+void launch_mf_update_once(const Batch& B, hipStream_t stream) {
+    hipLaunchKernelGGL(mf_update_kernel<false>, dim3(mf_delta_partials(B.nodes), B.frames), dim3(256), 0, stream, B.dev, 0u);
+}
+
+// The entry weights the matrix-free applies read (fixed by the index build).
+void launch_mf_entries(const Batch& B, bool fp64, bool recompute, hipStream_t stream) {
+    const dim3 sg(row_group_grid(B.nodes), B.frames);
+    if (fp64) hipLaunchKernelGGL(mf_entries_kernel, dim3((B.nodes + 3) / 4, B.frames), dim3(256), 0, stream, B.dev);
+    else if (recompute) hipLaunchKernelGGL(mf_entry_weights_kernel, sg, dim3(256), 0, stream, B.dev);
 }
 
 // The term Jacobian at se3[which] with unit weights, recomputed from the maps:
@@ -734,29 +1265,27 @@ void launch_mf_entry_weights(const Batch& B, hipStream_t stream) {
 // transpose 1: q = J^T y (reference twists) for y in mf_u.
 void launch_debug_jacobian(const Batch& B, bool fp64, bool transpose, uint32_t which, hipStream_t stream) {
     const Penalty unit{1.f, 1.f, 1.f, 1.f, 1.f};
-    const uint32_t tg = term_grid(B), sg = row_group_grid(B.nodes), vg = (B.nodes + 255) / 256;
-    if (!transpose) {
-        hipLaunchKernelGGL(mfr_coords_kernel, dim3(vg, B.frames), dim3(256), 0, stream, B.dev, 0);
-        if (fp64)
-            hipLaunchKernelGGL((mfr_terms_kernel<double, double, kSrcZ, kOutRows>), dim3(tg, B.frames), dim3(256), 0, stream,
-                               B.dev, 0u, 0u, unit, which);
-        else
-            hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcZ, kOutRows>), dim3(tg, B.frames), dim3(256), 0, stream,
-                               B.dev, 0u, 0u, unit, which);
+    const dim3 tg(term_grid(B), B.frames), sg(row_group_grid(B.nodes), B.frames), vg((B.nodes + 255) / 256, B.frames), wg(256);
+    if (fp64) {
+        if (!transpose) {
+            hipLaunchKernelGGL(mfr_coords_kernel, vg, wg, 0, stream, B.dev, 0);
+            hipLaunchKernelGGL((mf_apply_terms_kernel<true, kSrcZ, kOutRows>), tg, wg, 0, stream, B.dev, 0u, unit, which);
+        } else {
+            hipLaunchKernelGGL((mf_apply_terms_kernel<true, kSrcRows, kOutG>), tg, wg, 0, stream, B.dev, 0u, unit, which);
+            hipLaunchKernelGGL((mf_apply_gather_kernel<true, kEpiAdjoint>), dim3(gather_grid(B), B.frames),
+                               dim3(64 * kMfWaves), 0, stream, B.dev, 0u, unit);
+            hipLaunchKernelGGL(mfr_coords_kernel, vg, wg, 0, stream, B.dev, 1);
+        }
         return;
     }
-    if (fp64) {
-        hipLaunchKernelGGL((mfr_terms_kernel<double, double, kSrcRows, kOutG>), dim3(tg, B.frames), dim3(256), 0, stream,
-                           B.dev, 0u, 0u, unit, which);
-        hipLaunchKernelGGL((mfr_gather_kernel<double, double, kEpiAdjoint>), dim3(sg, B.frames), dim3(256), 0, stream,
-                           B.dev, 0u, 0u, unit, which);
-    } else {
-        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcRows, kOutG>), dim3(tg, B.frames), dim3(256), 0, stream,
-                           B.dev, 0u, 0u, unit, which);
-        hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiAdjoint>), dim3(sg, B.frames), dim3(256), 0, stream,
-                           B.dev, 0u, 0u, unit, which);
+    if (!transpose) {
+        hipLaunchKernelGGL(mfr_coords_kernel, vg, wg, 0, stream, B.dev, 0);
+        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcZ, kOutRows>), tg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
+        return;
     }
-    hipLaunchKernelGGL(mfr_coords_kernel, dim3(vg, B.frames), dim3(256), 0, stream, B.dev, 1);
+    hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcRows, kOutG>), tg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
+    hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiAdjoint>), sg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
+    hipLaunchKernelGGL(mfr_coords_kernel, vg, wg, 0, stream, B.dev, 1);
 }
 
 }  // namespace mvdr

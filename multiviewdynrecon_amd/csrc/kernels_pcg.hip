@@ -945,25 +945,18 @@ void launch_pair_blocks(const Batch& B, const Penalty& pen, hipStream_t stream) 
     hipLaunchKernelGGL(pair_blocks_kernel, dim3(grid, B.frames), dim3(256), 0, stream, B.dev, pen);
 }
 
-void launch_pcg_init(const Batch& B, bool fp64, hipStream_t stream) {
-    if (fp64) hipLaunchKernelGGL(pcg_init_kernel<double>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev);
-    else hipLaunchKernelGGL(pcg_init_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev);
+// Steps of the FP32 matrix-free PCG.
+void launch_pcg_init(const Batch& B, hipStream_t stream) {
+    hipLaunchKernelGGL(pcg_init_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev);
 }
 
-void launch_pcg_update(const Batch& B, bool fp64, uint32_t k, uint32_t spmv_blocks, uint32_t dsel, hipStream_t stream) {
-    if (fp64)
-        hipLaunchKernelGGL(pcg_update_kernel<double>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, k,
-                           spmv_blocks, dsel);
-    else
-        hipLaunchKernelGGL(pcg_update_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, k,
-                           spmv_blocks, dsel);
+void launch_pcg_update(const Batch& B, uint32_t k, uint32_t spmv_blocks, uint32_t dsel, hipStream_t stream) {
+    hipLaunchKernelGGL(pcg_update_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, k, spmv_blocks,
+                       dsel);
 }
 
-void launch_refine_step(const Batch& B, bool fp64, uint32_t spmv_blocks, hipStream_t stream) {
-    if (fp64)
-        hipLaunchKernelGGL(refine_step_kernel<double>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, spmv_blocks);
-    else
-        hipLaunchKernelGGL(refine_step_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, spmv_blocks);
+void launch_refine_step(const Batch& B, uint32_t spmv_blocks, hipStream_t stream) {
+    hipLaunchKernelGGL(refine_step_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, spmv_blocks);
 }
 
 // The CG transform alone (launch tuning).

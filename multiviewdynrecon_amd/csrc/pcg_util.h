@@ -30,12 +30,18 @@ __device__ inline double* slot_ptr(const Buffers& b, uint32_t slot) { return b.p
 // by every block (fixed order: strided per-thread sums, a wave butterfly, the
 // waves in order).  One workgroup barrier; at most one call per kernel (the
 // LDS is not reused).
+// partials_sum2 / partials_finish2 are its two halves: work between them overlaps
+// the partials' loads.
 template <typename Acc>
-__device__ inline void reduce_partials2(const double* p0, uint32_t n0, const double* p1, uint32_t n1, Acc& s0, Acc& s1) {
-    __shared__ Acc sh[2][4];
-    Acc v0 = 0, v1 = 0;
+__device__ inline void partials_sum2(const double* p0, uint32_t n0, const double* p1, uint32_t n1, Acc& v0, Acc& v1) {
+    v0 = 0;
+    v1 = 0;
     for (uint32_t i = threadIdx.x; i < n0; i += blockDim.x) v0 += (Acc)p0[i];
     for (uint32_t i = threadIdx.x; i < n1; i += blockDim.x) v1 += (Acc)p1[i];
+}
+template <typename Acc>
+__device__ inline void partials_finish2(Acc v0, Acc v1, Acc& s0, Acc& s1) {
+    __shared__ Acc sh[2][4];
     v0 = wave_sum(v0);
     v1 = wave_sum(v1);
     if ((threadIdx.x & 63) == 0) {
@@ -49,6 +55,12 @@ __device__ inline void reduce_partials2(const double* p0, uint32_t n0, const dou
         s0 += sh[0][w];
         s1 += sh[1][w];
     }
+}
+template <typename Acc>
+__device__ inline void reduce_partials2(const double* p0, uint32_t n0, const double* p1, uint32_t n1, Acc& s0, Acc& s1) {
+    Acc v0, v1;
+    partials_sum2<Acc>(p0, n0, p1, n1, v0, v1);
+    partials_finish2<Acc>(v0, v1, s0, s1);
 }
 
 // Block sum of per-thread values, stored as this block's partial of `slot`

@@ -28,7 +28,8 @@ void launch_pcg_matrix_free(const Batch& B, uint32_t iters, uint32_t refine, boo
 void launch_mf_apply_once(const Batch& B, bool fp64, const Penalty& pen, bool recompute, uint32_t which,
                           hipStream_t stream);
 void launch_debug_jacobian(const Batch& B, bool fp64, bool transpose, uint32_t which, hipStream_t stream);
-void launch_mf_entry_weights(const Batch& B, hipStream_t stream);
+void launch_mf_entries(const Batch& B, bool fp64, bool recompute, hipStream_t stream);
+void launch_mf_update_once(const Batch& B, hipStream_t stream);
 void launch_spmv_once(const Batch& B, bool fp64, hipStream_t stream);
 void launch_pcg_update_once(const Batch& B, bool fp64, hipStream_t stream);
 uint32_t launch_cost(const Batch& B, const Penalty& pen, bool density_in_jtj, hipStream_t stream);
@@ -193,7 +194,7 @@ void enqueue_batch(const Batch& B, const mvdr_solver_config& c, hipStream_t stre
         launch_copy_se3(B, stream);
         launch_index_build(B, c.use_foreground != 0, c.use_cross_view != 0,
                            mf ? kIndexNodes : (fp64 ? kIndexGram : kIndexLists), stream);
-        if (c.jtj_mode == MVDR_JTJ_RECOMPUTE) launch_mf_entry_weights(B, stream);
+        if (mf) launch_mf_entries(B, fp64, c.jtj_mode == MVDR_JTJ_RECOMPUTE, stream);
     }
     for (uint32_t k = first_iter; k < first_iter + iters; ++k) {
         const Penalty pen = kernel_penalty(c, k);
@@ -435,22 +436,31 @@ static size_t layout_buffers(const mvdr_solver_config& c, Buffers& b, FrameDev*&
     A(b.n2t_count, N1);
     A(b.n2t_offset, N1);
     A(b.n2t_index, b.cap_kv1);
-    A(b.n2t_node, b.cap_kv1);
+    const bool mf = matrix_free(c), mixed = c.precision == MVDR_PRECISION_MIXED;
+    if (!mf) A(b.n2t_node, b.cap_kv1);
     A(b.row_up, N1);
     A(b.row_low, N1);
     A(b.row_kv2, N1);
     A(b.pair_offset, N1);
     A(b.kv2_offset, N1);
-    A(b.pair_key, b.cap_pairs);
-    A(b.pair_range, b.cap_pairs);
-    A(b.pair_terms, b.cap_kv2);
-    A(b.kv2_pair, b.cap_kv2);
-    const bool mf = matrix_free(c);
+    if (!mf) {  // the matrix-free solve has no pair index and no off-diagonal blocks
+        A(b.pair_key, b.cap_pairs);
+        A(b.pair_range, b.cap_pairs);
+        A(b.pair_terms, b.cap_kv2);
+        A(b.kv2_pair, b.cap_kv2);
+        A(b.low_ent, b.cap_pairs);
+        A(b.offdiag, 36 * (size_t)b.cap_pairs);
+    }
     if (mf) {
+        const bool recompute = c.jtj_mode == MVDR_JTJ_RECOMPUTE;
         A(b.mf_u, knn_terms + b.cap_edges);
-        if (c.jtj_mode == MVDR_JTJ_RECOMPUTE) {
-            A(b.mf_g, 2 * (knn_terms + b.cap_edges));
-            A(b.n2t_w, b.cap_kv1);
+        if (recompute) A(b.mf_g, 2 * (knn_terms + b.cap_edges));
+        if (recompute && !mixed) A(b.n2t_w, b.cap_kv1);
+        if (mixed) {
+            A(b.mf_ent, b.cap_kv1);
+            if (recompute) A(b.mf_edge, b.cap_edges);
+            A(b.mf_rec[0], 16 * (size_t)c.max_nodes);
+            A(b.mf_rec[1], 16 * (size_t)c.max_nodes);
         }
     } else if (c.precision == MVDR_PRECISION_MIXED) {
         A(b.n2t_col, b.cap_kv1);
@@ -462,14 +472,12 @@ static size_t layout_buffers(const mvdr_solver_config& c, Buffers& b, FrameDev*&
         A(b.part_pair, ((size_t)b.cap_kv2 / 64 + 1) * 2 * 36);
     }
     A(b.low_offset, N1);
-    A(b.low_ent, b.cap_pairs);
     A(b.diag, 36 * (size_t)c.max_nodes);
     A(b.diag_inv, 36 * (size_t)c.max_nodes);
     // FP64 factors: the mixed mode, and the row Gram assembly of the matrix-free solve
     const bool factors64 = c.precision == MVDR_PRECISION_MIXED || mf;
     if (factors64) A(b.diag_inv64, 36 * (size_t)c.max_nodes);
     A(b.jtr, 6 * (size_t)c.max_nodes);
-    A(b.offdiag, 36 * (size_t)b.cap_pairs);
     for (float** v : {&b.x, &b.r, &b.s, &b.q, &b.d0, &b.d1}) A(*v, 6 * (size_t)c.max_nodes);
     if (factors64) A(b.linv64, kTri * (size_t)c.max_nodes);
     if (c.precision == MVDR_PRECISION_MIXED && !mf) {
@@ -880,7 +888,10 @@ static mvdr_status bench_stage_impl(const Batch& B, const mvdr_solver_config& c,
         switch (stage) {
             case MVDR_STAGE_EVAL_TERMS: launch_eval_terms(B, k & 1, fp64, st); break;
             case MVDR_STAGE_ASSEMBLE: launch_assemble(B, pen, fp64 || mf, mf, st); break;
-            case MVDR_STAGE_PCG_UPDATE: launch_pcg_update_once(B, fp64, st); break;
+            case MVDR_STAGE_PCG_UPDATE:
+                if (mf && fp64) launch_mf_update_once(B, st);
+                else launch_pcg_update_once(B, fp64, st);
+                break;
             case MVDR_STAGE_SPMV:
                 if (mf) launch_mf_apply_once(B, fp64, pen, c.jtj_mode == MVDR_JTJ_RECOMPUTE, k & 1, st);
                 else launch_spmv_once(B, fp64, st);
