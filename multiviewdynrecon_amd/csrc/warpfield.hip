@@ -1,13 +1,25 @@
 // Warp-field maintenance kernels (include/mvdr/warpfield.h): node graph,
 // skinning, forward and inverse warps.
 //
-// The two searches are all-pairs scans over the canonical nodes: each
-// workgroup stages the nodes through LDS in tiles of kNodeTile (every node is
-// read from HBM once per workgroup, the tile by all 256 threads), so the
-// searches run at the VALU rate of ~7 flops per (point, node) pair -- about
-// 1.2 G pairs for 150k surfels x 4k nodes.  The warps are streaming passes
-// bound by HBM (a 16-32 B read and write per point plus the L2-resident
-// warp-field gathers).
+// The two searches scan the canonical nodes in index order (the slots of a
+// result record the order of the insertions, so the order is part of it).
+// Both skip most of them by boxes around 8 consecutive nodes (built by every
+// workgroup): a box no nearer than the farthest result slot holds nothing that
+// could be inserted.
+//   vertices  : a thread per vertex.  A wave tests 64 boxes at a time against the
+//               box of its vertices, a lane per box; the nodes of a box pass through
+//               scalar registers (every lane looks at the same node; from LDS the
+//               reads alone took as long as the arithmetic), asked for one box ahead.
+//   nodes     : a wave per node, in the graph and in the skinning; a lane per box and
+//               then per node of the next eight near boxes; the few that beat the
+//               worst slot are inserted one after another.  (A thread per node filled
+//               16 workgroups of 256.)
+// Bound by the chain of insertions and the arithmetic around it (the memory traffic
+// is 8 MB).  159k surfels and 4018 nodes of the body scene: skinning 441 -> 198 us,
+// graph 791 -> 90 us; surfels in no order, whose boxes exclude nothing, 540 -> 494 us.
+//
+// The warps are streaming passes bound by HBM (a 16-32 B read and write per point plus
+// the L2-resident warp-field gathers).
 //
 // Distances are evaluated without contraction except where the reference
 // fuses explicitly (the skinning distance), so that they round like the
@@ -25,113 +37,300 @@
 namespace mvdr {
 namespace {
 
-constexpr uint32_t kNodeTile = 1024;
-constexpr int kGraphNeighbours = 8;   // nodesGraphNeigboursNum
+constexpr uint32_t kBoxNodes = 8;       // nodes per box
+constexpr uint32_t kBoxes = 512;        // boxes in LDS at a time (4096 nodes, 16 KB)
+constexpr int kGraphNeighbours = 8;     // nodesGraphNeigboursNum
+constexpr uint32_t kGraphWaves = 8;     // nodes per workgroup of the graph search
+
+// Squared distances are compared by their bits: at least +0, they are ordered alike (a
+// not-a-number comes last), and integer minima and maxima need no canonical operands.
+__device__ inline uint32_t bits(float d) { return __float_as_uint(d); }
 
 // The reference's 4-slot heap update (brute_foce_knn.cuh:17-39): slot x holds
-// the current worst; a closer node replaces it and sifts once.
-__device__ inline void heap_update(float d[4], uint32_t id[4], uint32_t idx, float dist) {
-    if (!(dist < d[0])) return;
-    d[0] = dist;
-    id[0] = idx;
-    if (d[1] < d[2]) {
-        if (d[0] < d[2]) {
-            const float t = d[0]; d[0] = d[2]; d[2] = t;
-            const uint32_t u = id[0]; id[0] = id[2]; id[2] = u;
+// the current worst; a closer node replaces it and sifts once.  Minima, maxima and
+// selects, no branches: the slots always form a heap (0 over 1 and 2, 1 over 3), so a
+// node that is not closer leaves them as they are.
+__device__ inline void heap_update(uint32_t d[4], uint32_t id[4], uint32_t idx, uint32_t dist) {
+    const uint32_t m = dist < d[0] ? idx : id[0], n = min(dist, d[0]);
+    const bool right = d[1] < d[2];
+    const uint32_t c = max(d[1], d[2]), ic = right ? id[2] : id[1];
+    const bool sift = n < c, to2 = sift & right, to1 = sift & !right;
+    const uint32_t e = to1 ? n : d[1], ie = to1 ? m : id[1];  // at slot 1 before the look at slot 3
+    const bool to3 = e < d[3];
+    d[0] = max(n, c);
+    id[0] = sift ? ic : m;
+    d[2] = to2 ? n : d[2];
+    id[2] = to2 ? m : id[2];
+    d[1] = max(e, d[3]);
+    id[1] = to3 ? id[3] : ie;
+    d[3] = min(e, d[3]);
+    id[3] = to3 ? ie : id[3];
+}
+
+// Maximum over each eight lanes, and over the wave (from lane 63, without LDS).
+template <int kCtrl, int kRows = 0xF>
+__device__ inline float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), kCtrl, kRows, 0xF, false));
+}
+__device__ inline float wave_max(float v) {
+    v = fmaxf(v, dpp<0xB1>(v));        // lane ^ 1
+    v = fmaxf(v, dpp<0x4E>(v));        // lane ^ 2
+    v = fmaxf(v, dpp<0x141>(v));       // the other four of eight
+    v = fmaxf(v, dpp<0x140>(v));       // the other eight of a row
+    v = fmaxf(v, dpp<0x142, 0xA>(v));  // rows 1 and 3: lane 15 of the row before
+    v = fmaxf(v, dpp<0x143, 0xC>(v));  // rows 2 and 3: lane 31
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// The same for the bits of squared distances (one instruction a step).
+template <int kCtrl, int kRows = 0xF>
+__device__ inline uint32_t max_dpp(uint32_t v) {
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xF, false));
+}
+__device__ inline uint32_t eight_max(uint32_t v) { return max_dpp<0x141>(max_dpp<0x4E>(max_dpp<0xB1>(v))); }
+__device__ inline uint32_t wave_max(uint32_t v) {
+    v = max_dpp<0x143, 0xC>(max_dpp<0x142, 0xA>(max_dpp<0x140>(eight_max(v))));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The boxes of nodes [base, base + n), n <= kBoxes * kBoxNodes, by the workgroup.
+struct NodeBoxes {
+    float4 lo[kBoxes], hi[kBoxes];
+};
+__device__ inline uint32_t build_boxes(const float4* __restrict__ nodes, uint32_t base, uint32_t n, NodeBoxes& x) {
+    const uint32_t boxes = (n + kBoxNodes - 1) / kBoxNodes;
+    __syncthreads();
+    for (uint32_t t = threadIdx.x; t < 2 * boxes; t += blockDim.x) {  // two lanes per box, four nodes each
+        float4 l, h;
+#pragma unroll
+        for (uint32_t j = 0; j < kBoxNodes / 2; ++j) {
+            const float4 q = nodes[base + min(t * (kBoxNodes / 2) + j, n - 1)];  // the last node repeats past the end
+            l = j == 0 ? q : make_float4(fminf(l.x, q.x), fminf(l.y, q.y), fminf(l.z, q.z), 0.f);
+            h = j == 0 ? q : make_float4(fmaxf(h.x, q.x), fmaxf(h.y, q.y), fmaxf(h.z, q.z), 0.f);
         }
-    } else if (d[0] < d[1]) {
-        float t = d[0]; d[0] = d[1]; d[1] = t;
-        uint32_t u = id[0]; id[0] = id[1]; id[1] = u;
-        if (d[1] < d[3]) {
-            t = d[1]; d[1] = d[3]; d[3] = t;
-            u = id[1]; id[1] = id[3]; id[3] = u;
+        l = make_float4(fminf(l.x, dpp<0xB1>(l.x)), fminf(l.y, dpp<0xB1>(l.y)), fminf(l.z, dpp<0xB1>(l.z)), 0.f);
+        h = make_float4(fmaxf(h.x, dpp<0xB1>(h.x)), fmaxf(h.y, dpp<0xB1>(h.y)), fmaxf(h.z, dpp<0xB1>(h.z)), 0.f);
+        if (t % 2 == 0)
+            x.lo[t / 2] = l;
+        else
+            x.hi[t / 2] = h;
+    }
+    __syncthreads();
+    return boxes;
+}
+
+// Eight nodes at a wave-uniform index in scalar registers (nothing writes the nodes
+// during the call, so the constant address space may serve them).  Volatile: the
+// compiler would move the loads down to their first use, and the wave would wait there.
+typedef float float16 __attribute__((ext_vector_type(16), aligned(16)));
+struct NodeGroup {
+    float16 q[2];
+    __device__ void load(const float4* nodes, uint32_t k) {
+#if __HIP_DEVICE_COMPILE__
+        const auto* p = (const volatile __attribute__((address_space(4))) float16*)(nodes + k);
+        q[0] = p[0];
+        q[1] = p[1];
+#endif
+    }
+    __device__ float4 node(uint32_t j) const {
+        const float16& h = q[j / 4];
+        return make_float4(h[j % 4 * 4], h[j % 4 * 4 + 1], h[j % 4 * 4 + 2], 0.f);
+    }
+};
+
+__device__ inline float skin_distance(float4 pt, float4 q) {
+    const float dx = pt.x - q.x, dy = pt.y - q.y, dz = pt.z - q.z;
+    return __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+}
+
+// Squared distance of two boxes (a point is a box of no extent).
+__device__ inline float box_distance(float4 alo, float4 ahi, float4 lo, float4 hi) {
+    const float dx = fmaxf(fmaxf(lo.x - ahi.x, alo.x - hi.x), 0.f);
+    const float dy = fmaxf(fmaxf(lo.y - ahi.y, alo.y - hi.y), 0.f);
+    const float dz = fmaxf(fmaxf(lo.z - ahi.z, alo.z - hi.z), 0.f);
+    return __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+}
+
+// Whether a distance below d0 may hide behind a box distance.  Box distances and
+// distances carry at most 5 roundings each way; 2e-6 below a box distance no
+// distance can fall (above the denormal range).  Not-a-number answers true.
+__device__ inline bool may_be_nearer(float box, float d0) { return !(box * 0.999998f >= d0 && box > 1e-30f); }
+
+// Passes the nodes that may enter the slots of one point `me` (the wave's), in index
+// order: a lane per box, then per node of the next eight near boxes.
+//   slots.bound()             the farthest slot
+//   slots.distance(me, q)     slots.wants(d): whether a distance may be inserted
+//   slots.insert(k, d)        one node, k and d wave-uniform
+template <class Slots>
+__device__ inline void scan_for_point(const float4* __restrict__ nodes, uint32_t num_nodes, float4 me, NodeBoxes& box,
+                                      Slots& slots) {
+    const uint32_t lane = threadIdx.x & 63, part = lane / kBoxNodes;
+    for (uint32_t base = 0; base < num_nodes; base += kBoxes * kBoxNodes) {
+        const uint32_t boxes = build_boxes(nodes, base, min(kBoxes * kBoxNodes, num_nodes - base), box);
+        for (uint32_t b0 = 0; b0 < boxes; b0 += 64) {
+            const uint32_t mine = min(b0 + lane, boxes - 1);
+            const float away = box_distance(me, me, box.lo[mine], box.hi[mine]);
+            uint64_t left = b0 + 64 <= boxes ? ~0ull : (1ull << (boxes - b0)) - 1;  // boxes not yet passed
+            for (;;) {
+                // the next eight near boxes, one to eight lanes (a box passed over
+                // is no nearer than the farthest slot, which only gets nearer)
+                uint64_t near = left & __ballot(may_be_nearer(away, slots.bound()));
+                if (!near) break;
+                uint32_t x = 0xFFFFFFFFu, last = 0;
+#pragma unroll
+                for (uint32_t r = 0; r < 64 / kBoxNodes; ++r) {
+                    if (near) {
+                        last = (uint32_t)__builtin_ctzll(near);
+                        near &= near - 1;
+                        if (part == r) x = last;
+                    }
+                }
+                left = last == 63 ? 0 : left & (~0ull << (last + 1));
+                const uint32_t k = base + (b0 + x) * kBoxNodes + lane % kBoxNodes;
+                const bool live = x != 0xFFFFFFFFu && k < num_nodes;
+                const float d = slots.distance(me, nodes[live ? k : 0]);
+                uint64_t hits = __ballot(live && slots.wants(d));
+                while (hits) {
+                    const int l = __builtin_ctzll(hits);
+                    slots.insert((uint32_t)__builtin_amdgcn_readlane((int)k, l),
+                                 __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d), l)));
+                    // later hits that still beat the farthest slot
+                    hits &= __ballot(d < slots.bound()) & (l == 63 ? 0ull : ~0ull << (l + 1));
+                }
+            }
         }
     }
 }
 
-// One workgroup of 256 threads per 256 points; the nodes pass through LDS.
-// Points [0, num_vertices) are vertices, [num_vertices, + num_nodes) nodes.
-__global__ void __launch_bounds__(256) skin_kernel(const float4* __restrict__ vertices, uint32_t num_vertices,
-                                                   const float4* __restrict__ nodes, uint32_t num_nodes,
-                                                   float radius, ushort4* __restrict__ vknn, float4* __restrict__ vw,
-                                                   ushort4* __restrict__ nknn, float4* __restrict__ nw) {
-    __shared__ float4 tile[kNodeTile];
-    const uint32_t total = num_vertices + num_nodes;
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    float4 pt = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (p < num_vertices) pt = vertices[p];
-    else if (p < total) pt = nodes[p - num_vertices];
-    float d[4] = {1e6f, 1e6f, 1e6f, 1e6f};
-    uint32_t id[4] = {0, 0, 0, 0};
-    for (uint32_t base = 0; base < num_nodes; base += kNodeTile) {
-        const uint32_t n = min(kNodeTile, num_nodes - base);
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) tile[k] = nodes[base + k];
-        __syncthreads();
-        for (uint32_t k = 0; k < n; ++k) {
-            const float4 q = tile[k];
-            const float dx = pt.x - q.x, dy = pt.y - q.y, dz = pt.z - q.z;
-            const float dist = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-            heap_update(d, id, base + k, dist);
+struct SkinSlots {
+    uint32_t d[4], id[4] = {0, 0, 0, 0};
+    __device__ SkinSlots() { d[0] = d[1] = d[2] = d[3] = bits(1e6f); }
+    __device__ float bound() const { return __uint_as_float(d[0]); }
+    __device__ static float distance(float4 pt, float4 q) { return skin_distance(pt, q); }
+    __device__ bool wants(float dist) const { return bits(dist) < d[0]; }
+    __device__ void insert(uint32_t k, float dist) { heap_update(d, id, k, bits(dist)); }
+    // nodes k .. k + 8, each lane's point its own; whether any entered
+    __device__ bool pass(float4 pt, const NodeGroup& g, uint32_t k) {
+        uint32_t dist[kBoxNodes], nearest;
+#pragma unroll
+        for (uint32_t j = 0; j < kBoxNodes; ++j) {
+            dist[j] = bits(skin_distance(pt, g.node(j)));
+            nearest = j == 0 ? dist[0] : min(nearest, dist[j]);
         }
+        if (!__any(nearest < d[0])) return false;
+#pragma unroll
+        for (uint32_t j = 0; j < kBoxNodes; ++j)
+            if (__any(dist[j] < d[0])) heap_update(d, id, k + j, dist[j]);
+        return true;
     }
-    if (p >= total) return;
+};
+
+// Weights of the four slots (skinningVertexAndNodeKernel).
+__device__ inline void put_skin(float4 pt, const SkinSlots& slots, const float4* __restrict__ nodes, float radius,
+                                ushort4* __restrict__ knn, float4* __restrict__ weight) {
     float w[4];
     const float den = (2.0f * radius) * radius;
     for (int s = 0; s < 4; ++s) {
-        const float4 q = nodes[id[s]];
+        const float4 q = nodes[slots.id[s]];
         const float dx = pt.x - q.x, dy = pt.y - q.y, dz = pt.z - q.z;
         w[s] = expf(-(dx * dx + dy * dy + dz * dz) / den);
     }
     const float inv = 1.0f / (fabsf(w[0]) + fabsf(w[1]) + fabsf(w[2]) + fabsf(w[3]));
-    const ushort4 k4 = make_ushort4(id[0], id[1], id[2], id[3]);
-    const float4 w4 = make_float4(w[0] * inv, w[1] * inv, w[2] * inv, w[3] * inv);
-    if (p < num_vertices) {
-        vknn[p] = k4;
-        vw[p] = w4;
-    } else {
-        nknn[p - num_vertices] = k4;
-        nw[p - num_vertices] = w4;
-    }
+    *knn = make_ushort4(slots.id[0], slots.id[1], slots.id[2], slots.id[3]);
+    *weight = make_float4(w[0] * inv, w[1] * inv, w[2] * inv, w[3] * inv);
 }
 
-// BuildNodesGraphKernel: 8 slots, the worst replaced (WarpField.cu:15-59).
-__global__ void __launch_bounds__(256) node_graph_kernel(const float4* __restrict__ nodes, uint32_t num_nodes,
-                                                         ushort2* __restrict__ graph) {
-    __shared__ float4 tile[kNodeTile];
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const float4 me = i < num_nodes ? nodes[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    float dist[kGraphNeighbours];
-    int idx[kGraphNeighbours];
-    for (int k = 0; k < kGraphNeighbours; ++k) {
-        dist[k] = 1e5f;
-        idx[k] = -1;
+constexpr uint32_t kSkinWaves = 4;  // waves per workgroup of the skinning
+
+// The first workgroups skin 256 vertices each, the others a node per wave.  (64 nodes
+// in a row lie too far apart for boxes common to them.)  All waves are resident at
+// once, a few per SIMD, and the longest of them set the time: vertices before nodes
+// (198 us; nodes first 226) and four waves a workgroup (eight of them 219 nodes first,
+// one 202) spread them best.
+__global__ void __launch_bounds__(64 * kSkinWaves)
+    skin_kernel(const float4* __restrict__ vertices, uint32_t num_vertices, const float4* __restrict__ nodes,
+                uint32_t num_nodes, float radius, ushort4* __restrict__ vknn, float4* __restrict__ vw,
+                ushort4* __restrict__ nknn, float4* __restrict__ nw) {
+    __shared__ NodeBoxes box;
+    SkinSlots slots;
+    const uint32_t vertex_blocks = (num_vertices + blockDim.x - 1) / blockDim.x, lane = threadIdx.x & 63;
+    if (blockIdx.x >= vertex_blocks) {
+        const uint32_t i = (blockIdx.x - vertex_blocks) * kSkinWaves + (threadIdx.x >> 6);
+        const float4 me = nodes[min(i, num_nodes - 1)];
+        scan_for_point(nodes, num_nodes, me, box, slots);
+        if (i < num_nodes && lane == 0) put_skin(me, slots, nodes, radius, nknn + i, nw + i);
+        return;
     }
-    int worst = 0;
-    for (uint32_t base = 0; base < num_nodes; base += kNodeTile) {
-        const uint32_t n = min(kNodeTile, num_nodes - base);
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) tile[k] = nodes[base + k];
-        __syncthreads();
-        for (uint32_t k = 0; k < n; ++k) {
-            const float4 q = tile[k];
-            const float d = (me.x - q.x) * (me.x - q.x) + (me.y - q.y) * (me.y - q.y) + (me.z - q.z) * (me.z - q.z);
-            if (d > 1e-6f && d < dist[worst]) {
-                dist[worst] = d;
-                idx[worst] = (int)(base + k);
-                worst = 0;
-                float mx = 0.f;
-                for (int j = 0; j < kGraphNeighbours; ++j)
-                    if (dist[j] > mx) {
-                        worst = j;
-                        mx = dist[j];
-                    }
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    const float4 pt = vertices[min(p, num_vertices - 1)];  // idle lanes repeat the last vertex
+    const float4 whi = make_float4(wave_max(pt.x), wave_max(pt.y), wave_max(pt.z), 0.f);
+    const float4 wlo = make_float4(-wave_max(-pt.x), -wave_max(-pt.y), -wave_max(-pt.z), 0.f);
+    float worst = 1e6f;  // the farthest fourth neighbour of the wave's points
+    for (uint32_t base = 0; base < num_nodes; base += kBoxes * kBoxNodes) {
+        const uint32_t n = min(kBoxes * kBoxNodes, num_nodes - base);
+        build_boxes(nodes, base, n, box);
+        const uint32_t whole = n / kBoxNodes;  // whole boxes; the rest comes last in any case
+        for (uint32_t b0 = 0; b0 < whole; b0 += 64) {
+            const uint32_t mine = min(b0 + lane, whole - 1);
+            const float coarse = box_distance(wlo, whi, box.lo[mine], box.hi[mine]);
+            uint64_t left = b0 + 64 <= whole ? ~0ull : (1ull << (whole - b0)) - 1;  // boxes not yet passed
+            uint64_t near = left & __ballot(may_be_nearer(coarse, worst));
+            if (!near) continue;
+            const float4* first = nodes + base + b0 * kBoxNodes;
+            uint32_t x = (uint32_t)__builtin_ctzll(near);
+            NodeGroup here, next;
+            here.load(first, x * kBoxNodes);
+            for (;;) {
+                // the next box's nodes are asked for before this one's are worked on
+                left &= ~((2ull << x) - 1);
+                near &= left;
+                const uint32_t y = near ? (uint32_t)__builtin_ctzll(near) : x;
+                next.load(first, y * kBoxNodes);
+                if (slots.pass(pt, here, base + (b0 + x) * kBoxNodes)) {
+                    worst = __uint_as_float(wave_max(slots.d[0]));
+                    near = left & __ballot(may_be_nearer(coarse, worst));
+                }
+                if (y == x) break;
+                x = y;
+                here = next;
             }
         }
+        for (uint32_t k = base + whole * kBoxNodes; k < base + n; ++k) slots.insert(k, skin_distance(pt, nodes[k]));
     }
-    if (i >= num_nodes) return;
-    for (int k = 0; k < kGraphNeighbours; ++k)
-        graph[(size_t)i * kGraphNeighbours + k] = make_ushort2((uint16_t)i, (uint16_t)idx[k]);
+    if (p < num_vertices) put_skin(pt, slots, nodes, radius, vknn + p, vw + p);
+}
+
+// BuildNodesGraphKernel: 8 slots, the worst replaced (WarpField.cu:15-59).  Lane
+// j < 8 holds slot j.
+struct GraphSlots {
+    float dist = (threadIdx.x & 63) < kGraphNeighbours ? 1e5f : 0.f;
+    int idx = -1;
+    float worst_d = 1e5f;
+    uint32_t worst = 0;
+    __device__ float bound() const { return worst_d; }
+    __device__ static float distance(float4 me, float4 q) {
+        return (me.x - q.x) * (me.x - q.x) + (me.y - q.y) * (me.y - q.y) + (me.z - q.z) * (me.z - q.z);
+    }
+    __device__ bool wants(float d) const { return d > 1e-6f && d < worst_d; }
+    __device__ void insert(uint32_t k, float d) {
+        if ((threadIdx.x & 63) == worst) {
+            dist = d;
+            idx = (int)k;
+        }
+        // the new worst slot: the first of the largest 
+        worst_d = __int_as_float(__builtin_amdgcn_readfirstlane((int)eight_max(bits(dist))));
+        worst = (uint32_t)__builtin_ctzll(__ballot(dist == worst_d));
+    }
+};
+__global__ void __launch_bounds__(64 * kGraphWaves) node_graph_kernel(const float4* __restrict__ nodes, uint32_t num_nodes,
+                                                                      ushort2* __restrict__ graph) {
+    __shared__ NodeBoxes box;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t i = blockIdx.x * kGraphWaves + (threadIdx.x >> 6);
+    GraphSlots slots;
+    scan_for_point(nodes, num_nodes, nodes[min(i, num_nodes - 1)], box, slots);
+    if (i < num_nodes && lane < (uint32_t)kGraphNeighbours)
+        graph[(size_t)i * kGraphNeighbours + lane] = make_ushort2((uint16_t)i, (uint16_t)slots.idx);
 }
 
 __device__ inline bool knn_in_range(ushort4 k, uint32_t n) { return k.x < n && k.y < n && k.z < n && k.w < n; }
@@ -363,8 +562,8 @@ mvdr_status mvdr_warp_build_node_graph(const void* nodes, uint32_t num_nodes, vo
     if (num_nodes == 0) return MVDR_OK;
     if (!nodes || !graph) return MVDR_E_INVALID;
     if (num_nodes > 65535) return MVDR_E_SHAPE;
-    hipLaunchKernelGGL(node_graph_kernel, dim3((num_nodes + 255) / 256), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const float4*>(nodes), num_nodes, static_cast<ushort2*>(graph));
+    hipLaunchKernelGGL(node_graph_kernel, dim3((num_nodes + kGraphWaves - 1) / kGraphWaves), dim3(64 * kGraphWaves), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const float4*>(nodes), num_nodes, static_cast<ushort2*>(graph));
     return hipGetLastError() == hipSuccess ? MVDR_OK : MVDR_E_HIP;
 }
 
@@ -376,7 +575,8 @@ mvdr_status mvdr_warp_skin(const void* vertices, uint32_t num_vertices, const vo
     if (!nknn || !nw) return MVDR_E_INVALID;
     const uint64_t total = (uint64_t)num_vertices + num_nodes;
     if (total > 0xFFFFFFFFull - 255) return MVDR_E_SHAPE;
-    hipLaunchKernelGGL(skin_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
+    const uint32_t blocks = (num_vertices + 64 * kSkinWaves - 1) / (64 * kSkinWaves) + (num_nodes + kSkinWaves - 1) / kSkinWaves;
+    hipLaunchKernelGGL(skin_kernel, dim3(blocks), dim3(64 * kSkinWaves), 0, static_cast<hipStream_t>(stream),
                        static_cast<const float4*>(vertices), num_vertices, static_cast<const float4*>(nodes), num_nodes,
                        node_radius, static_cast<ushort4*>(vknn), static_cast<float4*>(vw), static_cast<ushort4*>(nknn),
                        static_cast<float4*>(nw));
