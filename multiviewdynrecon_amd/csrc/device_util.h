@@ -167,14 +167,6 @@ __device__ inline void bitonic_sort_lds(K* keys, uint32_t m) {
 }
 
 // Map fetches with the reference textures' border addressing: zero outside.
-__device__ inline float4 fetch4(const FrameDev& f, const float4* map, int x, int y) {
-    if (x < 0 || y < 0 || x >= (int)f.W || y >= (int)f.H) return make_float4(0.f, 0.f, 0.f, 0.f);
-    return map[y * (int)f.W + x];
-}
-__device__ inline uint32_t fetch_index(const FrameDev& f, uint32_t v, int x, int y) {
-    if (x < 0 || y < 0 || x >= (int)f.W || y >= (int)f.H) return 0u;
-    return f.index[v][y * (int)f.W + x];
-}
 __device__ inline uint8_t fetch_edge(const FrameDev& f, uint32_t v, int x, int y) {
     if (x < 0 || y < 0 || x >= (int)f.W || y >= (int)f.H) return 0;
     return f.edge[v][y * (int)f.W + x];
