@@ -578,8 +578,8 @@ static_assert(4 * kBigChunkTerms <= 0xFFFFu && kBigChunkTerms % kChunkTerms == 0
 // LDS node tile of the counting-sort kernels (dynamic shared memory).
 uint32_t hist_tile(uint32_t nodes) { return std::min<uint32_t>(nodes, kHistNodes); }
 size_t hist_tile_bytes(uint32_t tile) { return (size_t)(tile + 1) / 2 * sizeof(uint32_t); }
-// Chunk workgroups (over all frames of a launch) up to which the placement
-// keeps u32 counters: what the chip holds at once with 16 KB tiles (9 per CU).
+// Chunk workgroups (over all frames of a launch) up to which the chunks are small: what
+// the chip holds at once (9 per CU).
 constexpr size_t kPlaceResident = 2304;
 
 __device__ inline uint32_t num_chunks(const Counts& c, uint32_t chunk) { return (c.off[4] + chunk - 1) / chunk; }
@@ -670,44 +670,141 @@ __global__ void __launch_bounds__(64 * kScanWaves) n2t_colscan_kernel(const Buff
     if (w == kScanWaves - 1) b.n2t_count[n] = total;
 }
 
+// The value of lane ^ kMask, in the vector unit (an exchange through LDS costs a wave
+// ~120 cycles, and the sort below is a chain of 21 of them).
+template <int kCtrl, int kRows = 0xF>
+__device__ inline uint32_t lane_dpp(uint32_t v, uint32_t old = 0) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, kCtrl, kRows, 0xF, false);
+}
+template <int kMask>
+__device__ inline uint32_t lane_xor(uint32_t v) {
+#if __HIP_DEVICE_COMPILE__
+    if constexpr (kMask == 1) return lane_dpp<0xB1>(v);
+    if constexpr (kMask == 2) return lane_dpp<0x4E>(v);
+    if constexpr (kMask == 4) return lane_dpp<0x141>(lane_dpp<0x1B>(v));   // 3 and 7
+    if constexpr (kMask == 8) return lane_dpp<0x140>(lane_dpp<0x141>(v));  // 7 and 15
+    if constexpr (kMask == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return threadIdx.x & 16 ? r[0] : r[1];
+    }
+    if constexpr (kMask == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return threadIdx.x & 32 ? r[0] : r[1];
+    }
+#endif
+    return v;
+}
+
 // Bitonic sort of a wave's 256 keys, ascending; key e sits in lane e / 4,
 // register e % 4.  Pairs 4 or more keys apart are exchanged across lanes.
-__device__ inline void wave_sort256(uint32_t k[4]) {
+template <uint32_t kSize, uint32_t kD>
+__device__ inline void sort_step(uint32_t k[4]) {
     const uint32_t lane = threadIdx.x & 63;
+    if constexpr (kD >= 4) {
+        // bits kD and kSize of e = 4 lane + j come from the lane
+        const bool keep_min = (((4 * lane) & kSize) == 0) == (((4 * lane) & kD) == 0);
 #pragma unroll
-    for (uint32_t size = 2; size <= 256; size <<= 1) {
-#pragma unroll
-        for (uint32_t d = size >> 1; d > 0; d >>= 1) {
-            if (d >= 4) {
-                // bits d and size of e = 4 lane + j come from the lane
-                const bool keep_min = (((4 * lane) & size) == 0) == (((4 * lane) & d) == 0);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t o = (uint32_t)__shfl_xor((int)k[j], (int)(d >> 2), 64);
-                    k[j] = keep_min ? min(k[j], o) : max(k[j], o);
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (j & d) continue;
-                    const bool up = ((4 * lane + j) & size) == 0;
-                    const uint32_t lo = min(k[j], k[j ^ d]), hi = max(k[j], k[j ^ d]);
-                    k[j] = up ? lo : hi;
-                    k[j ^ d] = up ? hi : lo;
-                }
-            }
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t o = lane_xor<(int)(kD >> 2)>(k[j]);
+            k[j] = keep_min ? min(k[j], o) : max(k[j], o);
         }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (j & kD) continue;
+            const bool up = ((4 * lane + j) & kSize) == 0;
+            const uint32_t lo = min(k[j], k[j ^ kD]), hi = max(k[j], k[j ^ kD]);
+            k[j] = up ? lo : hi;
+            k[j ^ kD] = up ? hi : lo;
+        }
+    }
+    if constexpr (kD > 1) sort_step<kSize, kD / 2>(k);
+    else if constexpr (kSize < 256) sort_step<2 * kSize, kSize>(k);
+}
+__device__ inline void wave_sort256(uint32_t k[4]) { sort_step<2, 1>(k); }
+
+// For the lane's entries n[0..3] (0xFFFFFFFF: none): their rank among the wave's entries
+// of the same node in (lane, slot) order, and whether an entry is its node's last.
+struct RankTable {
+    uint4 rank[64];
+};
+__device__ inline void rank_entries(RankTable& table, const uint32_t n[4], uint32_t n0, uint32_t rank[4], bool last[4]) {
+    const uint32_t lane = threadIdx.x & 63;
+    // the round's 256 entries sorted by (node, term, slot): key = local
+    // node << 8 | 4 lane + slot; entries not placed here sort last
+    uint32_t k[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) k[q] = n[q] == 0xFFFFFFFFu ? 0xFFFFFFFFu : ((n[q] - n0) << 8) | (4 * lane + q);
+    wave_sort256(k);
+    // runs of equal nodes: rank = sorted position - start of the run
+    uint32_t nd[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) nd[j] = k[j] >> 8;
+    const uint32_t prev = lane_dpp<0x138>(nd[3], nd[3]), next = lane_dpp<0x130>(nd[0], nd[0]);  // lanes before and after
+    uint32_t start[4], run = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const bool head = j == 0 ? (lane == 0 || prev != nd[0]) : nd[j - 1] != nd[j];
+        if (head) run = 4 * lane + j;
+        start[j] = run;  // start of the run within this lane (0 if it began earlier)
+    }
+    // inclusive max-scan of the lanes' last run starts (along the rows of 16, then from
+    // each row to those after it), then exclusive
+    uint32_t scan = run;
+    scan = max(scan, lane_dpp<0x111>(scan));
+    scan = max(scan, lane_dpp<0x112>(scan));
+    scan = max(scan, lane_dpp<0x114>(scan));
+    scan = max(scan, lane_dpp<0x118>(scan));
+    scan = max(scan, lane_dpp<0x142, 0xA>(scan));
+    scan = max(scan, lane_dpp<0x143, 0xC>(scan));
+    const uint32_t before = lane_dpp<0x138>(scan);
+    uint32_t* rk = reinterpret_cast<uint32_t*>(table.rank);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const bool tail = j < 3 ? nd[j + 1] != nd[j] : (lane == 63 || next != nd[3]);
+        if (k[j] != 0xFFFFFFFFu) rk[k[j] & 255] = (4 * lane + j - max(start[j], before)) | (tail ? 0x80000000u : 0u);
+    }
+    wave_lds_sync();
+    const uint4 r4 = table.rank[lane];
+    const uint32_t mine[4] = {r4.x, r4.y, r4.z, r4.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        rank[q] = mine[q] & 0x7FFFFFFFu;
+        last[q] = n[q] != 0xFFFFFFFFu && (mine[q] >> 31) != 0;
     }
 }
 
+// The node words of term t, read and not yet looked at (term_nodes would wait for them
+// in each of its branches): two packed node numbers each, the second unused by an edge.
+struct TermWords {
+    uint32_t lo, hi;
+    bool edge;
+};
+__device__ inline TermWords term_words(const Buffers& b, const FrameDev& f, const uint32_t off[5], uint32_t t) {
+    TermWords w;
+    w.edge = t >= off[0] && t < off[1];
+    const void* p = b.dense_knn + t;
+    if (t >= off[0]) p = f.graph + (t - off[0]);
+    if (t >= off[1]) p = &b.fg[t - off[1]].knn;
+    if (t >= off[2]) p = &b.feat[t - off[2]].knn;
+    if (t >= off[3]) p = &b.cross[t - off[3]].knn;
+    const uint32_t* q = static_cast<const uint32_t*>(p);
+    w.lo = q[0];
+    w.hi = q[w.edge ? 0 : 1];
+    return w;
+}
+
+// Places a chunk's entries: an entry goes to its node's list offset plus the node's
+// entries in earlier chunks, in earlier rounds of 64 terms (cur) and in earlier lanes of
+// the round (its rank).  The nodes and list positions of kPlaceRounds rounds are read
+// before the first of them is placed: reads after a round's stores wait for those as
+// well.  The ranks come from a sort, whose time does not depend on how many nodes a
+// round names (a hash table of lane masks took 19 us where neighbouring pixels share
+// nodes, 41 where feature pixels do not).  Bound by the sort, a chain in the vector unit:
+// a lone frame of 190k terms and 4k nodes 34 -> 21.5 us, 16 frames 213 -> 160 us.
 // with_nodes: also each entry's node (n2t_node), which only the segmented
 // assembly of the plain path reads.
-// kLdsBase: the tile's u32 LDS counters start at each node's list offset plus
-// its entries in earlier chunks (loaded once per tile: a small grid, all of it
-// resident at once); otherwise u16 counters start at zero and each entry loads
-// that base while its round sorts (half the LDS: twice the resident
-// workgroups of a large grid).  Both place every entry at the same position.
-template <bool kLdsBase>
+constexpr uint32_t kPlaceRounds = kChunkTerms / 64;
 __global__ void __launch_bounds__(64) n2t_place_kernel(const Buffers* __restrict__ bs, uint32_t tile, int with_nodes, uint32_t chunk) {
     const Buffers b = frame_buffers(bs);
     const FrameDev& f = *b.frame;
@@ -720,96 +817,58 @@ __global__ void __launch_bounds__(64) n2t_place_kernel(const Buffers* __restrict
     const uint32_t lane = threadIdx.x;
     extern __shared__ uint32_t cur_words[];
     using u16_lds = uint16_t __attribute__((may_alias));
-    u16_lds* cur16 = reinterpret_cast<u16_lds*>(cur_words);
-    __shared__ uint4 rank_of[64];  // rank of entry (lane, slot) among the round's entries of its node
+    u16_lds* cur = reinterpret_cast<u16_lds*>(cur_words);
+    __shared__ RankTable table;
     const uint32_t* H = b.n2t_hist + (size_t)blockIdx.x * N;
+    uint32_t off[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) off[k] = c.off[k];
     for (uint32_t n0 = 0; n0 < N; n0 += tile) {
         const uint32_t span = min(tile, N - n0);
-        if (kLdsBase) {
-#pragma unroll 8
-            for (uint32_t k = lane; k < span; k += 64) cur_words[k] = b.n2t_offset[n0 + k] + H[n0 + k];
-        } else {
-            for (uint32_t k = lane; k < (span + 1) / 2; k += 64) cur_words[k] = 0;
-        }
-        // the next round's term nodes load while this round sorts
-        ushort4 kn_next = make_ushort4(0, 0, 0, 0);
-        int m_next = t0 + lane < t1 ? term_nodes(b, f, c.off, t0 + lane, kn_next) : 0;
-        for (uint32_t tb = t0; tb < t1; tb += 64) {
-            const uint32_t t = tb + lane;
-            const ushort4 kn = kn_next;
-            const int m = m_next;
-            if (t + 64 < t1) m_next = term_nodes(b, f, c.off, t + 64, kn_next);
-            else m_next = 0;
-            uint32_t n[4] = {kn.x, kn.y, kn.z, kn.w};
+        for (uint32_t k = lane; k < (span + 1) / 2; k += 64) cur_words[k] = 0;
+        wave_lds_sync();
+        for (uint32_t tb = t0; tb < t1; tb += 64 * kPlaceRounds) {
+            uint32_t lo[kPlaceRounds], hi[kPlaceRounds];  // packed nodes, 0xFFFF: not placed here
+            uint32_t base[kPlaceRounds][4];
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (!(q < m && n[q] >= n0 && n[q] - n0 < span)) n[q] = 0xFFFFFFFFu;  // not placed here
-            // where this chunk's entries of each node start: the node's list
-            // offset plus its entries in earlier chunks (in flight during the sort)
-            uint32_t base[4] = {0u, 0u, 0u, 0u};
-            if (!kLdsBase) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (n[q] != 0xFFFFFFFFu) base[q] = b.n2t_offset[n[q]] + H[n[q]];
+            for (uint32_t r = 0; r < kPlaceRounds; ++r) {
+                const TermWords w = term_words(b, f, off, min(tb + 64 * r + lane, t1 - 1));
+                lo[r] = w.lo;
+                hi[r] = w.edge ? 0xFFFFFFFFu : w.hi;
             }
-            // the round's 256 entries sorted by (node, term, slot): key = local
-            // node << 8 | 4 lane + slot; entries not placed here sort last
-            uint32_t k[4];
+            auto node = [&](uint32_t r, uint32_t q) {
+                const uint32_t v = q < 2 ? (lo[r] >> (16 * q)) & 0xFFFFu : (hi[r] >> (16 * (q - 2))) & 0xFFFFu;
+                return tb + 64 * r + lane < t1 && v >= n0 && v - n0 < span ? v : 0xFFFFFFFFu;
+            };
 #pragma unroll
-            for (int q = 0; q < 4; ++q) k[q] = n[q] == 0xFFFFFFFFu ? 0xFFFFFFFFu : ((n[q] - n0) << 8) | (4 * lane + q);
-            wave_sort256(k);
-            // runs of equal nodes: rank = sorted position - start of the run
-            uint32_t nd[4];
+            for (uint32_t r = 0; r < kPlaceRounds; ++r)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) nd[j] = k[j] >> 8;
-            const uint32_t prev = (uint32_t)__shfl_up((int)nd[3], 1, 64);
-            const uint32_t next = (uint32_t)__shfl_down((int)nd[0], 1, 64);
-            uint32_t start[4], run = 0;
+                for (uint32_t q = 0; q < 4; ++q) {
+                    const uint32_t v = node(r, q), k = v == 0xFFFFFFFFu ? n0 : v;
+                    base[r][q] = b.n2t_offset[k] + H[k];
+                }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool head = j == 0 ? (lane == 0 || prev != nd[0]) : nd[j - 1] != nd[j];
-                if (head) run = 4 * lane + j;
-                start[j] = run;  // start of the run within this lane (0 if it began earlier)
-            }
-            // inclusive max-scan of the lanes' last run starts, then exclusive
-            uint32_t scan = run;
+            for (uint32_t r = 0; r < kPlaceRounds; ++r) {
+                const uint32_t t = tb + 64 * r + lane;
+                if (t - lane >= t1) break;
+                const uint32_t n[4] = {node(r, 0), node(r, 1), node(r, 2), node(r, 3)};
+                uint32_t rank[4];
+                bool last[4];
+                rank_entries(table, n, n0, rank, last);
 #pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t v = (uint32_t)__shfl_up((int)scan, o, 64);
-                if ((int)lane >= o) scan = max(scan, v);
-            }
-            uint32_t before = (uint32_t)__shfl_up((int)scan, 1, 64);
-            if (lane == 0) before = 0;
-            uint32_t rank[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) rank[j] = 4 * lane + j - max(start[j], before);
-            uint32_t* rk = reinterpret_cast<uint32_t*>(rank_of);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (k[j] != 0xFFFFFFFFu) rk[k[j] & 255] = rank[j];
-            wave_lds_sync();
-            const uint4 r4 = rank_of[lane];
-            const uint32_t mine[4] = {r4.x, r4.y, r4.z, r4.w};
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (n[q] != 0xFFFFFFFFu) {
-                    const uint32_t l = n[q] - n0;
-                    const uint32_t at = kLdsBase ? cur_words[l] + mine[q] : base[q] + cur16[l] + mine[q];
+                for (uint32_t q = 0; q < 4; ++q) {
+                    if (n[q] == 0xFFFFFFFFu) continue;
+                    const uint32_t at = base[r][q] + cur[n[q] - n0] + rank[q];
                     b.n2t_index[at] = t;
                     if (with_nodes) b.n2t_node[at] = (uint16_t)n[q];
                 }
-            }
-            wave_lds_sync();  // every lane has read cur before the updates
-            // the last entry of each run advances its node's counter
+                wave_lds_sync();  // every lane has read cur before the updates
+                // the node's last entry of the round advances its counter
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool tail = j < 3 ? nd[j + 1] != nd[j] : (lane == 63 || next != nd[3]);
-                if (k[j] != 0xFFFFFFFFu && tail) {
-                    if (kLdsBase) cur_words[nd[j]] += rank[j] + 1;
-                    else cur16[nd[j]] = (uint16_t)(cur16[nd[j]] + rank[j] + 1);
-                }
+                for (uint32_t q = 0; q < 4; ++q)
+                    if (last[q]) cur[n[q] - n0] = (uint16_t)(cur[n[q] - n0] + rank[q] + 1);
+                wave_lds_sync();
             }
-            wave_lds_sync();
         }
     }
 }
@@ -1268,12 +1327,8 @@ void launch_index_build(const Batch& B, bool use_foreground, bool use_cross, int
                        chunk);
     hipLaunchKernelGGL(node_scan_kernel, dim3(1, F), dim3(1024), 0, stream, B.dev, 0);
     const int with_nodes = mode == kIndexLists ? 1 : 0;
-    if (resident)
-        hipLaunchKernelGGL(n2t_place_kernel<true>, dim3(chunks, F), dim3(64), tile * sizeof(uint32_t), stream, B.dev,
-                           tile, with_nodes, chunk);
-    else
-        hipLaunchKernelGGL(n2t_place_kernel<false>, dim3(chunks, F), dim3(64), hist_tile_bytes(tile), stream, B.dev,
-                           tile, with_nodes, chunk);
+    hipLaunchKernelGGL(n2t_place_kernel, dim3(chunks, F), dim3(64), hist_tile_bytes(tile), stream, B.dev, tile, with_nodes,
+                       chunk);
     if (mode == kIndexNodes) return;
     const uint32_t row_grid = (B.nodes + kXcds - 1) / kXcds * kXcds;
     if (gram) {
