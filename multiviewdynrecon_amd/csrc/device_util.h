@@ -63,11 +63,48 @@ __device__ inline Buffers frame_buffers_at(const Buffers* bs, uint32_t frame) {
 #endif
 }
 
+// The value of lane ^ kMask, in the vector unit: an exchange through LDS costs a wave
+// ~120 cycles, and sums and sorts over a wave are chains of them.
+template <int kCtrl, int kRows = 0xF>
+__device__ inline uint32_t lane_dpp(uint32_t v, uint32_t old = 0) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, kCtrl, kRows, 0xF, false);
+}
+template <int kMask>
+__device__ inline uint32_t lane_xor(uint32_t v) {
+#if __HIP_DEVICE_COMPILE__
+    if constexpr (kMask == 1) return lane_dpp<0xB1>(v);
+    if constexpr (kMask == 2) return lane_dpp<0x4E>(v);
+    if constexpr (kMask == 4) return lane_dpp<0x141>(lane_dpp<0x1B>(v));   // 3 and 7
+    if constexpr (kMask == 8) return lane_dpp<0x140>(lane_dpp<0x141>(v));  // 7 and 15
+    if constexpr (kMask == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return threadIdx.x & 16 ? r[0] : r[1];
+    }
+    if constexpr (kMask == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return threadIdx.x & 32 ? r[0] : r[1];
+    }
+#endif
+    return v;
+}
+template <int kMask>
+__device__ inline float lane_xor(float v) { return __uint_as_float(lane_xor<kMask>(__float_as_uint(v))); }
+template <int kMask>
+__device__ inline double lane_xor(double v) {
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned long long lo = lane_xor<kMask>((uint32_t)u), hi = lane_xor<kMask>((uint32_t)(u >> 32));
+    return __longlong_as_double((long long)(lo | hi << 32));
+}
+
+// Sum over each kLanes lanes, in every one of them: partners kLanes / 2 away first.
+template <int kLanes, typename T>
+__device__ inline T lanes_sum(T v) {
+    if constexpr (kLanes == 1) return v;
+    else return lanes_sum<kLanes / 2>(v + lane_xor<kLanes / 2>(v));
+}
 template <typename T>
 __device__ inline T wave_sum(T v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return lanes_sum<64>(v);
 }
 
 template <typename T>

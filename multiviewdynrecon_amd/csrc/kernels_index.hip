@@ -670,31 +670,6 @@ __global__ void __launch_bounds__(64 * kScanWaves) n2t_colscan_kernel(const Buff
     if (w == kScanWaves - 1) b.n2t_count[n] = total;
 }
 
-// The value of lane ^ kMask, in the vector unit (an exchange through LDS costs a wave
-// ~120 cycles, and the sort below is a chain of 21 of them).
-template <int kCtrl, int kRows = 0xF>
-__device__ inline uint32_t lane_dpp(uint32_t v, uint32_t old = 0) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, kCtrl, kRows, 0xF, false);
-}
-template <int kMask>
-__device__ inline uint32_t lane_xor(uint32_t v) {
-#if __HIP_DEVICE_COMPILE__
-    if constexpr (kMask == 1) return lane_dpp<0xB1>(v);
-    if constexpr (kMask == 2) return lane_dpp<0x4E>(v);
-    if constexpr (kMask == 4) return lane_dpp<0x141>(lane_dpp<0x1B>(v));   // 3 and 7
-    if constexpr (kMask == 8) return lane_dpp<0x140>(lane_dpp<0x141>(v));  // 7 and 15
-    if constexpr (kMask == 16) {
-        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-        return threadIdx.x & 16 ? r[0] : r[1];
-    }
-    if constexpr (kMask == 32) {
-        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-        return threadIdx.x & 32 ? r[0] : r[1];
-    }
-#endif
-    return v;
-}
-
 // Bitonic sort of a wave's 256 keys, ascending; key e sits in lane e / 4,
 // register e % 4.  Pairs 4 or more keys apart are exchanged across lanes.
 template <uint32_t kSize, uint32_t kD>

@@ -248,9 +248,7 @@ __global__ void __launch_bounds__(256) mf_gather_kernel(const Buffers* __restric
                 }
             }
 #pragma unroll
-            for (int a = 0; a < 6; ++a)
-#pragma unroll
-                for (int o = kRowLanes / 2; o > 0; o >>= 1) y[a] += __shfl_xor(y[a], o, 64);
+            for (int a = 0; a < 6; ++a) y[a] = lanes_sum<kRowLanes>(y[a]);
             if (i < f.N && sub == 0) {
                 if (kEpi == kEpiSpmv) {
 #pragma unroll
@@ -562,9 +560,7 @@ __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restri
                 }
             }
 #pragma unroll
-            for (int a = 0; a < 6; ++a)
-#pragma unroll
-                for (int o = kRowLanes / 2; o > 0; o >>= 1) y[a] += __shfl_xor(y[a], o, 64);
+            for (int a = 0; a < 6; ++a) y[a] = lanes_sum<kRowLanes>(y[a]);
             if (i < f.N && sub == 0) {
                 // to node-centred coordinates: T^T (a, b) = (a + b x g, b)
                 y[0] += y[4] * (Acc)gi.z - y[5] * (Acc)gi.y;
@@ -983,7 +979,7 @@ __device__ inline void reduce_half(double (&v)[8]) {
 #pragma unroll
     for (int k = 0; k < kHalf; ++k) {
         const double keep = upper ? v[k + kHalf] : v[k], send = upper ? v[k] : v[k + kHalf];
-        v[k] = keep + __shfl_xor(send, kHalf, 64);
+        v[k] = keep + lane_xor<kHalf>(send);
     }
 }
 
@@ -1101,8 +1097,9 @@ __global__ void __launch_bounds__(64 * kMfWaves) mf_apply_gather_kernel(const Bu
         reduce_half<2>(y);
         reduce_half<1>(y);
         double ya = y[0];  // component a over the lanes 8 k + a
-#pragma unroll
-        for (int o = 8; o < 64; o <<= 1) ya += __shfl_xor(ya, o, 64);
+        ya += lane_xor<8>(ya);
+        ya += lane_xor<16>(ya);
+        ya += lane_xor<32>(ya);
         if (kRecompute) {
             // to node-centred coordinates: T^T (r, t) = (r + t x g, t)
             const double t0 = node_lane(ya, 3), t1 = node_lane(ya, 4), t2 = node_lane(ya, 5);

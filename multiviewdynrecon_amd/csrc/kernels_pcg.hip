@@ -66,9 +66,7 @@ __device__ inline void row_apply(const Buffers& b, uint32_t i, uint32_t sub, con
         block_mv<Acc>(B, tr, v, y);
     }
 #pragma unroll
-    for (int a = 0; a < 6; ++a)
-#pragma unroll
-        for (int o = kRowLanes / 2; o > 0; o >>= 1) y[a] += __shfl_xor(y[a], o, 64);
+    for (int a = 0; a < 6; ++a) y[a] = lanes_sum<kRowLanes>(y[a]);
 }
 
 // r = b, d = M^-1 b, x = 0, partials of delta_0 = dot(r, d)
@@ -498,9 +496,7 @@ __device__ inline void hat_row_apply(const Buffers& b, uint32_t i, uint32_t sub,
         block_mv<Acc>(b.offhat + 36 * (size_t)(s.y & 0x7FFFFFFFu), (s.y >> 31) != 0, v, y);
     }
 #pragma unroll
-    for (int a = 0; a < 6; ++a)
-#pragma unroll
-        for (int o = kHatLanes / 2; o > 0; o >>= 1) y[a] += __shfl_xor(y[a], o, 64);
+    for (int a = 0; a < 6; ++a) y[a] = lanes_sum<kHatLanes>(y[a]);
 }
 
 // w_0 = A^ r_0 (r_0 = b^), x^ = p_{-1} = s_{-1} = 0, partials of gamma_0, delta_0.

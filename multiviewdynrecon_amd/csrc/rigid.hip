@@ -68,7 +68,7 @@ __device__ inline void reduce_half(double (&v)[32], uint32_t lane) {
 #pragma unroll
     for (int k = 0; k < kHalf; ++k) {
         const double keep = upper ? v[k + kHalf] : v[k], send = upper ? v[k] : v[k + kHalf];
-        v[k] = keep + __shfl_xor(send, kHalf, 64);
+        v[k] = keep + lane_xor<kHalf>(send);
     }
 }
 __device__ inline double wave_sums32(double (&v)[32]) {
@@ -78,7 +78,7 @@ __device__ inline double wave_sums32(double (&v)[32]) {
     reduce_half<4>(v, lane);
     reduce_half<2>(v, lane);
     reduce_half<1>(v, lane);
-    return v[0] + __shfl_xor(v[0], 32, 64);
+    return v[0] + lane_xor<32>(v[0]);
 }
 
 __global__ void __launch_bounds__(kRigidBlock) rigid_rows_kernel(RigidViews r) {
