@@ -481,12 +481,11 @@ __global__ void __launch_bounds__(256) pair_blocks_kernel(const Buffers* __restr
     }
 }
 
-// y = sum over the off-diagonal blocks of row i of A^ v_j, with v_j = V(j)
-// supplied by the caller; split over the row's kHatLanes lanes and reduced.
+// y += the off-diagonal blocks of row i of A^ times v_j, with v_j = load(j) supplied by
+// the caller, from the lane's slot `sub` on; split over the row's kHatLanes lanes and
+// reduced.
 template <typename Load, typename Acc = double>
 __device__ inline void hat_row_apply(const Buffers& b, uint32_t i, uint32_t sub, const Load& load, Acc y[6]) {
-#pragma unroll
-    for (int a = 0; a < 6; ++a) y[a] = 0;
     const uint32_t beg = b.row_ptr[i], n = b.row_ptr[i + 1] - beg;
 #pragma unroll 2  // two slots of a lane in flight (a row has ~12 slots over 8 lanes)
     for (uint32_t e = sub; e < n; e += kHatLanes) {
@@ -525,7 +524,7 @@ __global__ void __launch_bounds__(256) cg_init_kernel(const Buffers* __restrict_
             const bool own = i < f.N && sub < 6;
             float* rec = RWS + kRws * (size_t)(i < f.N ? i : 0);
             const double r = own ? rec[sub] : 0.0;
-            double y[6];
+            double y[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
             hat_row_apply(b, i < f.N ? i : 0, sub, load, y);
             if (own) {
                 const double ya = sub == 0 ? y[0] : sub == 1 ? y[1] : sub == 2 ? y[2] : sub == 3 ? y[3] : sub == 4 ? y[4] : y[5];
@@ -543,18 +542,15 @@ __global__ void __launch_bounds__(256) cg_init_kernel(const Buffers* __restrict_
     }
 }
 
-// alpha_i, beta_i from the partials of gamma_i, delta_i and the stored
-// alpha_{i-1}, gamma_{i-1}; block 0 stores alpha_i, gamma_i for launch i + 1.
-__device__ inline void cg_scalars(const Buffers& b, uint32_t i, uint32_t blocks, double& alpha, double& beta,
-                                  uint32_t block) {
-    double gamma, delta;
-    reduce_partials2<double>(slot_ptr(b, kSlotCgGamma + i), blocks, slot_ptr(b, kSlotCgDelta + i), blocks, gamma, delta);
+// alpha_i, beta_i from gamma_i, delta_i and the stored alpha_{i-1}, gamma_{i-1} (prev);
+// block 0 stores alpha_i, gamma_i for launch i + 1.
+__device__ inline void cg_scalars(const Buffers& b, uint32_t i, double gamma, double delta, double2 prev, double& alpha,
+                                  double& beta, uint32_t block) {
     beta = 0.0;
     double den = delta;
     if (i > 0) {
-        const double alpha_prev = b.cg_scal[2 * (i - 1)], gamma_prev = b.cg_scal[2 * (i - 1) + 1];
-        beta = gamma_prev != 0.0 ? gamma / gamma_prev : 0.0;
-        den = alpha_prev != 0.0 ? delta - beta * gamma / alpha_prev : 0.0;
+        beta = prev.y != 0.0 ? gamma / prev.y : 0.0;
+        den = prev.x != 0.0 ? delta - beta * gamma / prev.x : 0.0;
     }
     alpha = den != 0.0 ? gamma / den : 0.0;
     if (block == 0 && threadIdx.x == 0) {
@@ -563,12 +559,42 @@ __device__ inline void cg_scalars(const Buffers& b, uint32_t i, uint32_t blocks,
     }
 }
 
+// The record (r_i, w_i, s_{i-1}) of a node, and r_{i+1} as its owner rounds and stores
+// it: FP32 vector updates, one rounding each, fused.
+struct RwsRecord {
+    float4 q0, q1, q2, q3;
+    float2 q4;
+    __device__ void load(const float* __restrict__ rws, uint32_t j) {
+        const float4* q = reinterpret_cast<const float4*>(rws + kRws * (size_t)j);
+        q0 = q[0];
+        q1 = q[1];
+        q2 = q[2];
+        q3 = q[3];
+        q4 = *reinterpret_cast<const float2*>(rws + kRws * (size_t)j + 16);
+    }
+    __device__ void next_r(float af, float bf, float v[6]) const {
+        const float r[6] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y};
+        const float w[6] = {q1.z, q1.w, q2.x, q2.y, q2.z, q2.w};
+        const float sp[6] = {q3.x, q3.y, q3.z, q3.w, q4.x, q4.y};
+#pragma unroll
+        for (int a = 0; a < 6; ++a) {
+            const float s_i = __builtin_fmaf(bf, sp[a], w[a]);
+            v[a] = __builtin_fmaf(-af, s_i, r[a]);
+        }
+    }
+};
+
 // The row kernels of the fused CG (init, iterations, refinement) keep every
 // workgroup of a frame on one XCD (frame_affine), so a frame's A^ blocks and
 // vectors stay in that XCD's L2 from one launch to the next.
 
 // Launch i of the fused CG (see above).  Reads r_i, w_i, s_{i-1}; writes
 // r_{i+1}, w_{i+1}, s_i, p_i, x^_{i+1}.
+// kDeep: a launch that leaves most of the chip idle (a lone frame) takes the time of one
+// wave, a chain of dependent reads.  Its first two slots per lane, their blocks and
+// records are then read before the scalars of the iteration are known (142 registers,
+// which a launch that fills the chip cannot spare): 6.85 -> 6.58 us for 4k nodes.
+template <bool kDeep>
 __global__ void __launch_bounds__(256) cg_iter_kernel(const Buffers* __restrict__ bs, uint32_t i) {
     const WorkItem wi = frame_affine();
     const Buffers b = frame_buffers_at(bs, wi.frame);
@@ -576,31 +602,47 @@ __global__ void __launch_bounds__(256) cg_iter_kernel(const Buffers* __restrict_
     const uint32_t sub = threadIdx.x % kHatLanes;
     __shared__ GroupSums sums;
     group_sums_init(sums);  // published by the barrier of the partial reduction
-    double alpha, beta;
-    cg_scalars(b, i, cg_partials(f.N), alpha, beta, wi.block);
-    uint32_t pass = 0;
-    if (!b.counts->error) {
-        // reads (r_i, w_i, s_{i-1}), writes (r_{i+1}, w_{i+1}, s_i)
-        // (selects, not an index into the by-value struct: that would move it to scratch)
-        const bool odd = (i & 1) != 0;
-        const float* RWS = odd ? b.cg_rws[1] : b.cg_rws[0];
-        float* RWSo = odd ? b.cg_rws[0] : b.cg_rws[1];
-        // r_{i+1} of node j, rounded as it is stored
-        // FP32 vector updates (one rounding each, fused): every row forms its
-        // columns' r_{i+1} exactly as their owners store it
-        const float af = (float)alpha, bf = (float)beta;
-        auto next_r = [&](uint32_t j, float v[6]) {
-            const float4* q = reinterpret_cast<const float4*>(RWS + kRws * (size_t)j);
-            const float4 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
-            const float2 q4 = *reinterpret_cast<const float2*>(RWS + kRws * (size_t)j + 16);
-            const float r[6] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y};
-            const float w[6] = {q1.z, q1.w, q2.x, q2.y, q2.z, q2.w};
-            const float sp[6] = {q3.x, q3.y, q3.z, q3.w, q4.x, q4.y};
+    // reads (r_i, w_i, s_{i-1}), writes (r_{i+1}, w_{i+1}, s_i)
+    // (selects, not an index into the by-value struct: that would move it to scratch)
+    const bool odd = (i & 1) != 0, good = !b.counts->error;
+    const float* RWS = odd ? b.cg_rws[1] : b.cg_rws[0];
+    float* RWSo = odd ? b.cg_rws[0] : b.cg_rws[1];
+    struct Slot {
+        uint2 s;
+        Block6 block;
+        RwsRecord rec;
+    } slot[2];
+    uint32_t row_slots = 0;
+    if (kDeep && good) {
+        const uint32_t row = wi.block * kHatRowsPerBlock + threadIdx.x / kHatLanes, n = row < f.N ? row : 0;
+        const uint32_t beg = b.row_ptr[n];
+        row_slots = b.row_ptr[n + 1] - beg;
 #pragma unroll
-            for (int a = 0; a < 6; ++a) {
-                const float s_i = __builtin_fmaf(bf, sp[a], w[a]);
-                v[a] = __builtin_fmaf(-af, s_i, r[a]);
+        for (uint32_t k = 0; k < 2; ++k)
+            if (sub + k * kHatLanes < row_slots) slot[k].s = b.row_ent[beg + sub + k * kHatLanes];
+    }
+    double gamma, delta, alpha, beta;
+    const uint32_t parts = cg_partials(f.N);
+    partials_sum2<double>(slot_ptr(b, kSlotCgGamma + i), parts, slot_ptr(b, kSlotCgDelta + i), parts, gamma, delta);
+    const double2 prev = i > 0 ? make_double2(b.cg_scal[2 * (i - 1)], b.cg_scal[2 * (i - 1) + 1]) : make_double2(0.0, 0.0);
+    if (kDeep && good) {
+#pragma unroll
+        for (uint32_t k = 0; k < 2; ++k)
+            if (sub + k * kHatLanes < row_slots) {
+                slot[k].block.load(b.offhat + 36 * (size_t)(slot[k].s.y & 0x7FFFFFFFu));
+                slot[k].rec.load(RWS, slot[k].s.x);
             }
+    }
+    partials_finish2<double>(gamma, delta, gamma, delta);
+    cg_scalars(b, i, gamma, delta, prev, alpha, beta, wi.block);
+    uint32_t pass = 0;
+    if (good) {
+        const float af = (float)alpha, bf = (float)beta;
+        // every row forms its columns' r_{i+1} exactly as their owners store it
+        auto next_r = [&](uint32_t j, float v[6]) {
+            RwsRecord rec;
+            rec.load(RWS, j);
+            rec.next_r(af, bf, v);
         };
         const uint32_t groups = gridDim.x * kHatRowsPerBlock;
         for (uint32_t base = wi.block * kHatRowsPerBlock; base < f.N; base += groups) {
@@ -619,8 +661,17 @@ __global__ void __launch_bounds__(256) cg_iter_kernel(const Buffers* __restrict_
                 pk = b.cg_p[ka];
                 xk = b.cg_x[ka];
             }
-            float y[6];
-            hat_row_apply(b, n < f.N ? n : 0, sub, next_r, y);
+            float y[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (kDeep && pass == 0) {
+#pragma unroll
+                for (uint32_t k = 0; k < 2; ++k)
+                    if (sub + k * kHatLanes < row_slots) {
+                        float v[6];
+                        slot[k].rec.next_r(af, bf, v);
+                        slot[k].block.template mv<float>((slot[k].s.y >> 31) != 0, v, y);
+                    }
+            }
+            hat_row_apply(b, n < f.N ? n : 0, sub + (kDeep && pass == 0 ? 2 * kHatLanes : 0u), next_r, y);
             if (own) {
                 const float ya = sub == 0 ? y[0] : sub == 1 ? y[1] : sub == 2 ? y[2] : sub == 3 ? y[3] : sub == 4 ? y[4] : y[5];
                 const float s_i = __builtin_fmaf(bf, sk, wk);
@@ -668,7 +719,7 @@ __global__ void __launch_bounds__(256) cg_refine_residual_kernel(const Buffers* 
             const bool own = n < f.N && sub < 6;
             const size_t k = 6 * (size_t)(n < f.N ? n : 0) + (sub < 6 ? sub : 0);
             const double bk = own ? (double)b.cg_b[k] : 0.0, xk = own ? (double)X[k] : 0.0;
-            double y[6];
+            double y[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
             hat_row_apply(b, n < f.N ? n : 0, sub, load, y);
             if (own) {
                 const double ya = sub == 0 ? y[0] : sub == 1 ? y[1] : sub == 2 ? y[2] : sub == 3 ? y[3] : sub == 4 ? y[4] : y[5];
@@ -704,7 +755,7 @@ __global__ void __launch_bounds__(256) cg_refine_curvature_kernel(const Buffers*
             double acc = 0.0;
             const bool own = n < f.N && sub < 6;
             const double q = own ? (double)Q[6 * (size_t)n + sub] : 0.0;
-            double y[6];
+            double y[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
             hat_row_apply(b, n < f.N ? n : 0, sub, load, y);
             if (own) {
                 const double ya = sub == 0 ? y[0] : sub == 1 ? y[1] : sub == 2 ? y[2] : sub == 3 ? y[3] : sub == 4 ? y[4] : y[5];
@@ -916,6 +967,16 @@ static uint32_t transform_grid(uint32_t nodes, uint32_t frames) {
 uint32_t cg_workgroups_for(uint32_t nodes, uint32_t frames) { return cg_grid(nodes, frames); }
 uint32_t transform_workgroups_for(uint32_t nodes, uint32_t frames) { return transform_grid(nodes, frames); }
 
+// Workgroups of a CG launch up to which all of them run at once with the deep reads'
+// registers, three to a CU (4k nodes: 6 frames 12.4 -> 12.1 us, 8 frames 12.3 -> 14.6).
+constexpr uint32_t kCgDeepWorkgroups = 3 * 256;
+static void launch_cg_iter(const Batch& B, uint32_t i, uint32_t grid, hipStream_t stream) {
+    if ((uint64_t)grid * B.frames <= kCgDeepWorkgroups)
+        hipLaunchKernelGGL(cg_iter_kernel<true>, dim3(grid, B.frames), dim3(256), 0, stream, B.dev, i);
+    else
+        hipLaunchKernelGGL(cg_iter_kernel<false>, dim3(grid, B.frames), dim3(256), 0, stream, B.dev, i);
+}
+
 void launch_cg_solve(const Batch& B, uint32_t iters, uint32_t refine, uint32_t k, const Penalty& pen,
                      hipStream_t stream) {
     const uint32_t sg = cg_grid(B.nodes, B.frames);
@@ -923,8 +984,7 @@ void launch_cg_solve(const Batch& B, uint32_t iters, uint32_t refine, uint32_t k
     hipLaunchKernelGGL(cg_transform_kernel, dim3(transform_grid(B.nodes, B.frames), B.frames), dim3(256), 0, stream,
                        B.dev, pen);
     hipLaunchKernelGGL(cg_init_kernel, dim3(sg, B.frames), dim3(256), 0, stream, B.dev);
-    for (uint32_t i = 0; i < iters; ++i)
-        hipLaunchKernelGGL(cg_iter_kernel, dim3(sg, B.frames), dim3(256), 0, stream, B.dev, i);
+    for (uint32_t i = 0; i < iters; ++i) launch_cg_iter(B, i, sg, stream);
     for (uint32_t r = 0; r < refine; ++r) {
         hipLaunchKernelGGL(cg_refine_residual_kernel, dim3(sg, B.frames), dim3(256), 0, stream, B.dev);
         hipLaunchKernelGGL(cg_refine_curvature_kernel, dim3(sg, B.frames), dim3(256), 0, stream, B.dev);
@@ -963,7 +1023,7 @@ void launch_cg_transform_once(const Batch& B, const Penalty& pen, hipStream_t st
 
 // One fused CG iteration (stage timing).
 void launch_cg_iter_once(const Batch& B, hipStream_t stream) {
-    hipLaunchKernelGGL(cg_iter_kernel, dim3(cg_grid(B.nodes, B.frames), B.frames), dim3(256), 0, stream, B.dev, 1u);
+    launch_cg_iter(B, 1, cg_grid(B.nodes, B.frames), stream);
 }
 
 void launch_copy_se3(const Batch& B, hipStream_t stream) {

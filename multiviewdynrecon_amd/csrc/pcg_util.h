@@ -98,25 +98,35 @@ __device__ inline void write_partials2(const Buffers& b, uint32_t slot0, Acc v0,
 }
 
 // 6x6 row-major block times a 6-vector (or its transpose), accumulated in Acc.
+struct Block6 {
+    float m[36];
+    __device__ void load(const float* __restrict__ B) {
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const float4 t = reinterpret_cast<const float4*>(B)[q];
+            m[4 * q] = t.x; m[4 * q + 1] = t.y; m[4 * q + 2] = t.z; m[4 * q + 3] = t.w;
+        }
+    }
+    template <typename Acc>
+    __device__ void mv(bool transposed, const float v[6], Acc y[6]) const {
+        if (!transposed) {
+#pragma unroll
+            for (int a = 0; a < 6; ++a)
+#pragma unroll
+                for (int k = 0; k < 6; ++k) y[a] += (Acc)m[6 * a + k] * (Acc)v[k];
+        } else {
+#pragma unroll
+            for (int a = 0; a < 6; ++a)
+#pragma unroll
+                for (int k = 0; k < 6; ++k) y[a] += (Acc)m[6 * k + a] * (Acc)v[k];
+        }
+    }
+};
 template <typename Acc>
 __device__ inline void block_mv(const float* __restrict__ B, bool transposed, const float v[6], Acc y[6]) {
-    float m[36];
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-        const float4 t = reinterpret_cast<const float4*>(B)[q];
-        m[4 * q] = t.x; m[4 * q + 1] = t.y; m[4 * q + 2] = t.z; m[4 * q + 3] = t.w;
-    }
-    if (!transposed) {
-#pragma unroll
-        for (int a = 0; a < 6; ++a)
-#pragma unroll
-            for (int k = 0; k < 6; ++k) y[a] += (Acc)m[6 * a + k] * (Acc)v[k];
-    } else {
-#pragma unroll
-        for (int a = 0; a < 6; ++a)
-#pragma unroll
-            for (int k = 0; k < 6; ++k) y[a] += (Acc)m[6 * k + a] * (Acc)v[k];
-    }
+    Block6 b;
+    b.load(B);
+    b.mv<Acc>(transposed, v, y);
 }
 
 // M^-1 v for node n: FP64 inverse in the mixed mode, FP32 otherwise.
