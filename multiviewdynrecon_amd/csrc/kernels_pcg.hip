@@ -20,53 +20,95 @@
 
 namespace mvdr {
 
-// Input vector entry of node j: prev_j, or s_j + beta * prev_j.
-template <typename Acc>
-__device__ inline void load_dir(const float* __restrict__ prev, const float* __restrict__ s, bool use_beta, Acc beta, uint32_t j,
-                                float v[6]) {
+// The input vector of node j: prev_j, or s_j + beta * prev_j (s not null).
+struct DirEntry {
+    float2 p[3], s[3];
+    __device__ void load(const float* __restrict__ prev, const float* __restrict__ sv, uint32_t j) {
 #pragma unroll
-    for (int a = 0; a < 6; ++a) {
-        const float p = prev[6 * j + a];
-        v[a] = use_beta ? (float)((Acc)s[6 * j + a] + beta * (Acc)p) : p;
+        for (int a = 0; a < 3; ++a) {
+            p[a] = reinterpret_cast<const float2*>(prev + 6 * (size_t)j)[a];
+            if (sv) s[a] = reinterpret_cast<const float2*>(sv + 6 * (size_t)j)[a];
+        }
     }
-}
-
-// y = (A v)_i over block row i: diagonal, lower entries (B_ki^T, k < i), upper
-// entries (B_ij, j > i), split over the kRowLanes lanes of the row group and
-// reduced across them.
-template <typename Acc>
-__device__ inline void row_apply(const Buffers& b, uint32_t i, uint32_t sub, const float* prev, const float* s, bool use_beta,
-                                 Acc beta, Acc y[6]) {
+    template <typename Acc>
+    __device__ void form(bool use_beta, Acc beta, float v[6]) const {
 #pragma unroll
-    for (int a = 0; a < 6; ++a) y[a] = 0;
-    const uint32_t lo_beg = b.low_offset[i], lo_n = b.low_offset[i + 1] - lo_beg;
-    const uint32_t up_beg = b.pair_offset[i], up_n = b.pair_offset[i + 1] - up_beg;
-    const uint32_t total = 1 + lo_n + up_n;
-    for (uint32_t e = sub; e < total; e += kRowLanes) {
+        for (int a = 0; a < 6; ++a) {
+            const float pa = a % 2 ? p[a / 2].y : p[a / 2].x, sa = a % 2 ? s[a / 2].y : s[a / 2].x;
+            v[a] = use_beta ? (float)((Acc)sa + beta * (Acc)pa) : pa;
+        }
+    }
+};
+
+// Block row i: diagonal, lower entries (B_ki^T, k < i), upper entries (B_ij, j > i),
+// split over the kRowLanes lanes of the row group.
+struct BlockRow {
+    uint32_t i, lo_beg, lo_n, up_beg, total;
+    __device__ BlockRow(const Buffers& b, uint32_t row) : i(row) {
+        lo_beg = b.low_offset[i];
+        lo_n = b.low_offset[i + 1] - lo_beg;
+        up_beg = b.pair_offset[i];
+        total = 1 + lo_n + b.pair_offset[i + 1] - up_beg;
+    }
+};
+// What a lane adds to (A v)_i from entry e, read before it is used.
+struct RowEntry {
+    Block6 block;
+    DirEntry dir;
+    bool has, transposed;
+    __device__ void load(const Buffers& b, const BlockRow& row, uint32_t e, const float* __restrict__ prev,
+                         const float* __restrict__ s) {
+        has = e < row.total;
+        if (!has) return;
         const float* B;
-        bool tr;
         uint32_t j;
+        transposed = e != 0 && e <= row.lo_n;
         if (e == 0) {
-            B = b.diag + 36 * (size_t)i;
-            tr = false;
-            j = i;
-        } else if (e <= lo_n) {
-            const uint2 le = b.low_ent[lo_beg + e - 1];
+            B = b.diag + 36 * (size_t)row.i;
+            j = row.i;
+        } else if (transposed) {
+            const uint2 le = b.low_ent[row.lo_beg + e - 1];
             B = b.offdiag + 36 * (size_t)le.y;
-            tr = true;
             j = le.x;
         } else {
-            const uint32_t p = up_beg + (e - 1 - lo_n);
+            const uint32_t p = row.up_beg + (e - 1 - row.lo_n);
             B = b.offdiag + 36 * (size_t)p;
-            tr = false;
             j = b.pair_key[p] & 0xFFFF;
         }
+        block.load(B);
+        dir.load(prev, s, j);
+    }
+    template <typename Acc>
+    __device__ void add(bool use_beta, Acc beta, Acc y[6]) const {
+        if (!has) return;
         float v[6];
-        load_dir<Acc>(prev, s, use_beta, beta, j, v);
-        block_mv<Acc>(B, tr, v, y);
+        dir.form<Acc>(use_beta, beta, v);
+        block.mv<Acc>(transposed, v, y);
+    }
+};
+// y = (A v)_i over the lane's entries, the first of them read already, reduced across
+// the row's lanes.
+template <typename Acc>
+__device__ inline void row_apply(const Buffers& b, const BlockRow& row, const RowEntry& first, uint32_t sub, const float* prev,
+                                 const float* s, bool use_beta, Acc beta, Acc y[6]) {
+#pragma unroll
+    for (int a = 0; a < 6; ++a) y[a] = 0;
+    first.add<Acc>(use_beta, beta, y);
+    for (uint32_t e = sub + kRowLanes; e < row.total; e += kRowLanes) {
+        RowEntry more;
+        more.load(b, row, e, prev, s);
+        more.add<Acc>(use_beta, beta, y);
     }
 #pragma unroll
     for (int a = 0; a < 6; ++a) y[a] = lanes_sum<kRowLanes>(y[a]);
+}
+// y = (A v)_i of a vector that is known.
+template <typename Acc>
+__device__ inline void row_apply(const Buffers& b, uint32_t i, uint32_t sub, const float* v, Acc y[6]) {
+    const BlockRow row(b, i);
+    RowEntry first;
+    first.load(b, row, sub, v, nullptr);
+    row_apply<Acc>(b, row, first, sub, v, nullptr, false, (Acc)0, y);
 }
 
 // r = b, d = M^-1 b, x = 0, partials of delta_0 = dot(r, d)
@@ -96,13 +138,24 @@ __global__ void __launch_bounds__(256) pcg_init_kernel(const Buffers* __restrict
 }
 
 // Iteration k: q = A d with d = s + beta d_prev (k > 0); partials of dot(d, q).
+// A launch is short against the chain of reads in it: a lane's first entry (of ~13 a row,
+// over 16 lanes) is read before the scalars of the iteration are known, as are the vectors
+// and M^-1 of a thread's first node in the update (which also stored x and r between its
+// reads).  4k nodes, FP32: 7.2 -> 5.5 us, update 6.2 -> 4.35 us.
 template <typename Acc>
 __global__ void __launch_bounds__(256) pcg_spmv_kernel(const Buffers* __restrict__ bs, uint32_t k, uint32_t cur) {
     const Buffers b = frame_buffers(bs);
-    const float* __restrict__ d_prev = cur ? b.d1 : b.d0;
-    float* __restrict__ d_out = cur ? b.d0 : b.d1;
+    const float* d_prev = cur ? b.d1 : b.d0;
+    float* d_out = cur ? b.d0 : b.d1;
+    const float* s = k > 0 ? b.s : nullptr;
     const FrameDev& f = *b.frame;
     const uint32_t sub = threadIdx.x % kRowLanes;
+    const bool good = !b.counts->error;
+    const uint32_t groups = gridDim.x * kRowsPerBlock;
+    uint32_t i = blockIdx.x * kRowsPerBlock + threadIdx.x / kRowLanes;
+    BlockRow row(b, good && i < f.N ? i : 0);
+    RowEntry entry;
+    if (good) entry.load(b, row, sub, d_prev, s);
     Acc beta = 0;
     if (k > 0) {
         Acc num, den;
@@ -110,15 +163,18 @@ __global__ void __launch_bounds__(256) pcg_spmv_kernel(const Buffers* __restrict
         beta = den != (Acc)0 ? num / den : (Acc)0;
     }
     Acc acc = 0;
-    if (!b.counts->error) {
-        const uint32_t groups = gridDim.x * kRowsPerBlock;
+    if (good) {
         for (uint32_t base = blockIdx.x * kRowsPerBlock; base < f.N; base += groups) {
-            const uint32_t i = base + threadIdx.x / kRowLanes;
+            if (base >= groups) {
+                i = base + threadIdx.x / kRowLanes;
+                row = BlockRow(b, i < f.N ? i : 0);
+                entry.load(b, row, sub, d_prev, s);
+            }
             Acc y[6];
-            row_apply<Acc>(b, i < f.N ? i : 0, sub, d_prev, b.s, k > 0, beta, y);
+            row_apply<Acc>(b, row, entry, sub, d_prev, s, k > 0, beta, y);
             if (i < f.N && sub == 0) {
-                float v[6];
-                load_dir<Acc>(d_prev, b.s, k > 0, beta, i, v);
+                float v[6];  // lane 0's first entry is the diagonal: its vector is the row's
+                entry.dir.form<Acc>(k > 0, beta, v);
 #pragma unroll
                 for (int a = 0; a < 6; ++a) {
                     d_out[6 * i + a] = v[a];
@@ -137,29 +193,51 @@ __global__ void __launch_bounds__(256) pcg_spmv_kernel(const Buffers* __restrict
 template <typename Acc>
 __global__ void __launch_bounds__(256) pcg_update_kernel(const Buffers* __restrict__ bs, uint32_t k, uint32_t spmv_blocks, uint32_t dsel) {
     const Buffers b = frame_buffers(bs);
-    const float* __restrict__ d = dsel ? b.d1 : b.d0;
+    const float* d = dsel ? b.d1 : b.d0;
     const FrameDev& f = *b.frame;
+    struct Node {
+        float2 x[3], d[3], r[3], q[3];
+        MinvBlock<Acc> minv;
+    } node;
+    auto load = [&](uint32_t n) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            node.x[a] = reinterpret_cast<const float2*>(b.x + 6 * (size_t)n)[a];
+            node.d[a] = reinterpret_cast<const float2*>(d + 6 * (size_t)n)[a];
+            node.r[a] = reinterpret_cast<const float2*>(b.r + 6 * (size_t)n)[a];
+            node.q[a] = reinterpret_cast<const float2*>(b.q + 6 * (size_t)n)[a];
+        }
+        node.minv.load(b, n);
+    };
+    const bool good = !b.counts->error;
+    uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t stride = gridDim.x * blockDim.x;
+    if (good && n < f.N) load(n);
     Acc delta, dq;
     reduce_partials2<Acc>(slot_ptr(b, kSlotDelta + k), kVecBlocks, slot_ptr(b, kSlotDQ + k), spmv_blocks, delta, dq);
     const Acc alpha = dq != (Acc)0 ? delta / dq : (Acc)0;
     Acc acc = 0;
-    if (!b.counts->error) {
-        const uint32_t stride = gridDim.x * blockDim.x;
-        for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < f.N; n += stride) {
-            float t[6], sv[6];
+    if (good) {
+        while (n < f.N) {
+            float x[6], t[6], sv[6];
 #pragma unroll
             for (int a = 0; a < 6; ++a) {
-                const uint32_t i = 6 * n + a;
-                b.x[i] = (float)((Acc)b.x[i] + alpha * (Acc)d[i]);
-                t[a] = (float)((Acc)b.r[i] - alpha * (Acc)b.q[i]);
-                b.r[i] = t[a];
+                const float xa = a % 2 ? node.x[a / 2].y : node.x[a / 2].x, da = a % 2 ? node.d[a / 2].y : node.d[a / 2].x;
+                const float ra = a % 2 ? node.r[a / 2].y : node.r[a / 2].x, qa = a % 2 ? node.q[a / 2].y : node.q[a / 2].x;
+                x[a] = (float)((Acc)xa + alpha * (Acc)da);
+                t[a] = (float)((Acc)ra - alpha * (Acc)qa);
             }
-            apply_minv<Acc>(b, n, t, sv);
+            node.minv.apply(t, sv);
 #pragma unroll
-            for (int a = 0; a < 6; ++a) {
-                b.s[6 * n + a] = sv[a];
-                acc += (Acc)t[a] * (Acc)sv[a];
+            for (int a = 0; a < 3; ++a) {
+                reinterpret_cast<float2*>(b.x + 6 * (size_t)n)[a] = make_float2(x[2 * a], x[2 * a + 1]);
+                reinterpret_cast<float2*>(b.r + 6 * (size_t)n)[a] = make_float2(t[2 * a], t[2 * a + 1]);
+                reinterpret_cast<float2*>(b.s + 6 * (size_t)n)[a] = make_float2(sv[2 * a], sv[2 * a + 1]);
             }
+#pragma unroll
+            for (int a = 0; a < 6; ++a) acc += (Acc)t[a] * (Acc)sv[a];
+            n += stride;
+            if (n < f.N) load(n);
         }
     }
     write_partial<Acc>(b, kSlotDelta + k + 1, acc);
@@ -178,7 +256,7 @@ __global__ void __launch_bounds__(256) refine_residual_kernel(const Buffers* __r
         for (uint32_t base = blockIdx.x * kRowsPerBlock; base < f.N; base += groups) {
             const uint32_t i = base + threadIdx.x / kRowLanes;
             Acc y[6];
-            row_apply<Acc>(b, i < f.N ? i : 0, sub, b.x, b.s, false, (Acc)0, y);
+            row_apply<Acc>(b, i < f.N ? i : 0, sub, b.x, y);
             if (i < f.N && sub == 0) {
                 float rr[6], z[6];
 #pragma unroll
@@ -210,7 +288,7 @@ __global__ void __launch_bounds__(256) refine_curvature_kernel(const Buffers* __
         for (uint32_t base = blockIdx.x * kRowsPerBlock; base < f.N; base += groups) {
             const uint32_t i = base + threadIdx.x / kRowLanes;
             Acc y[6];
-            row_apply<Acc>(b, i < f.N ? i : 0, sub, b.d1, b.s, false, (Acc)0, y);
+            row_apply<Acc>(b, i < f.N ? i : 0, sub, b.d1, y);
             if (i < f.N && sub == 0) {
 #pragma unroll
                 for (int a = 0; a < 6; ++a) acc += (Acc)b.d1[6 * i + a] * y[a];

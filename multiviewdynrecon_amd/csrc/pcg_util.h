@@ -129,28 +129,34 @@ __device__ inline void block_mv(const float* __restrict__ B, bool transposed, co
     b.mv<Acc>(transposed, v, y);
 }
 
-// M^-1 v for node n: FP64 inverse in the mixed mode, FP32 otherwise.
+// M^-1 of a node: FP64 inverse in the mixed mode, FP32 otherwise.
 template <typename Acc>
-__device__ inline void apply_minv(const Buffers& b, uint32_t n, const float v[6], float out[6]) {
-    if constexpr (sizeof(Acc) == 8) {
-        const double* M = b.diag_inv64 + 36 * (size_t)n;
+struct MinvBlock {
+    Acc m[36];
+    __device__ void load(const Buffers& b, uint32_t n) {
+        if constexpr (sizeof(Acc) == 8) {
 #pragma unroll
-        for (int a = 0; a < 6; ++a) {
-            double s = 0.0;
+            for (int q = 0; q < 36; ++q) m[q] = b.diag_inv64[36 * (size_t)n + q];
+        } else {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) s += M[6 * a + k] * (double)v[k];
-            out[a] = (float)s;
-        }
-    } else {
-        const float* M = b.diag_inv + 36 * (size_t)n;
-#pragma unroll
-        for (int a = 0; a < 6; ++a) {
-            float s = 0.f;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) s += M[6 * a + k] * v[k];
-            out[a] = s;
+            for (int q = 0; q < 36; ++q) m[q] = b.diag_inv[36 * (size_t)n + q];
         }
     }
+    __device__ void apply(const float v[6], float out[6]) const {
+#pragma unroll
+        for (int a = 0; a < 6; ++a) {
+            Acc s = 0;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) s += m[6 * a + k] * (Acc)v[k];
+            out[a] = (float)s;
+        }
+    }
+};
+template <typename Acc>
+__device__ inline void apply_minv(const Buffers& b, uint32_t n, const float v[6], float out[6]) {
+    MinvBlock<Acc> m;
+    m.load(b, n);
+    m.apply(v, out);
 }
 
 }  // namespace mvdr
