@@ -8,7 +8,7 @@ import ctypes as C
 import numpy as np
 
 from . import _abi
-from .solver import SolverError, _stream_handle, lib as _solver_lib
+from .solver import SolverError, _memcpy_d2h, _stream_handle, _synchronize, lib as _solver_lib
 
 _BOUND = False
 
@@ -94,20 +94,14 @@ class CrossViewEdgeCorrespondence:
             raise SolverError(rc, "mvdr_crossview_find failed")
 
     def _get(self, which):
-        import torch
-
         p, n = C.c_void_p(), C.c_uint32()
         rc = lib().mvdr_crossview_get_pairs(self.h, _abi.CROSSVIEW_LISTS[which], C.byref(p), C.byref(n))
         if rc not in (0, 3):
             raise SolverError(rc, "mvdr_crossview_get_pairs failed")
         out = np.empty((n.value, 6), np.uint16)
         if n.value:
-            torch.cuda.synchronize()
-            buf = (C.c_uint16 * (6 * n.value))()
-            from .solver import _memcpy_d2h
-
-            _memcpy_d2h(C.addressof(buf), p.value, 12 * n.value)
-            out[:] = np.frombuffer(buf, np.uint16).reshape(-1, 6)
+            _synchronize()
+            _memcpy_d2h(out.ctypes.data, p.value, 12 * n.value)
         if rc == 3:
             raise SolverError(rc, f"{which}: more pairs than max_pairs ({self.config.max_pairs})")
         return out

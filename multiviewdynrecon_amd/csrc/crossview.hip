@@ -59,7 +59,7 @@ struct CvBuffers {
     uint8_t* flags;              // per source pixel: 1 candidate, 2 unique, 4 back-traced
     uint32_t* tile_count;        // kCvLists x tiles
     uint32_t* tile_offset;       // kCvLists x tiles
-    uint32_t* counts;            // kCvLists totals (untruncated)
+    uint32_t* counts;            // kCvLists totals (untruncated), in host memory
     mvdr_cross_pair* out[kCvLists];
     uint32_t max_pairs;
     int radius, step, track;
@@ -352,6 +352,7 @@ struct mvdr_crossview {
     bool found = false;
     ~mvdr_crossview() {
         if (done) (void)hipEventDestroy(done);
+        if (b.counts) (void)hipHostFree(b.counts);
         if (block) (void)hipFree(block);
     }
 };
@@ -400,7 +401,6 @@ mvdr_status mvdr_crossview_create(const mvdr_crossview_config* config, mvdr_cros
         carve(h->b.flags, pixels, base);
         carve(h->b.tile_count, (size_t)kCvLists * h->tiles, base);
         carve(h->b.tile_offset, (size_t)kCvLists * h->tiles, base);
-        carve(h->b.counts, kCvLists, base);
         for (uint32_t l = 0; l < kCvLists; ++l) carve(h->b.out[l], c.max_pairs, base);
         return off;
     };
@@ -408,9 +408,12 @@ mvdr_status mvdr_crossview_create(const mvdr_crossview_config* config, mvdr_cros
     hipError_t e = hipMalloc(&h->block, bytes);
     if (e == hipSuccess) {
         lay(static_cast<char*>(h->block));
-        e = hipMemset(h->b.counts, 0, kCvLists * sizeof(uint32_t));
-        if (e == hipSuccess) e = hipMemset(h->b.num_edges, 0, sizeof(uint32_t));
+        e = hipMemset(h->b.num_edges, 0, sizeof(uint32_t));
     }
+    // the getters read the totals without a copy (~10 us each)
+    if (e == hipSuccess)
+        e = hipHostMalloc(reinterpret_cast<void**>(&h->b.counts), kCvLists * sizeof(uint32_t), hipHostMallocDefault);
+    if (e == hipSuccess) std::memset(h->b.counts, 0, kCvLists * sizeof(uint32_t));
     if (e == hipSuccess) e = hipEventCreateWithFlags(&h->done, hipEventDisableTiming);
     if (e != hipSuccess) {
         delete h;
@@ -475,11 +478,11 @@ mvdr_status mvdr_crossview_get_pairs(mvdr_crossview* h, int list, const void** p
     if (!h || !pairs || !count || list < 0 || list >= (int)kCvLists) return MVDR_E_INVALID;
     if (!h->found) return MVDR_E_STATE;
     if (hipEventSynchronize(h->done) != hipSuccess) return MVDR_E_HIP;
-    uint32_t n[kCvLists];
-    if (hipMemcpy(n, h->b.counts, sizeof(n), hipMemcpyDeviceToHost) != hipSuccess) return MVDR_E_HIP;
+    if (hipStreamSynchronize(nullptr) != hipSuccess) return MVDR_E_HIP;  // as a copy on it would
+    const uint32_t n = *static_cast<volatile const uint32_t*>(h->b.counts + list);
     *pairs = h->b.out[list];
-    *count = std::min(n[list], h->cfg.max_pairs);
-    return n[list] > h->cfg.max_pairs ? MVDR_E_CAPACITY : MVDR_OK;
+    *count = std::min(n, h->cfg.max_pairs);
+    return n > h->cfg.max_pairs ? MVDR_E_CAPACITY : MVDR_OK;
 }
 
 }  // extern "C"

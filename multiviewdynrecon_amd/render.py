@@ -7,7 +7,7 @@ import ctypes as C
 import numpy as np
 
 from . import _abi
-from .solver import SolverError, _stream_handle, lib as _solver_lib
+from .solver import SolverError, _stream_handle, _synchronize, lib as _solver_lib
 
 MAPS = ("reference_vertex", "reference_normal", "warp_vertex", "warp_normal", "index_map", "normalized_rgb")
 _BOUND = False
@@ -24,8 +24,9 @@ def lib():
 
 def mat34(m):
     out = _abi.Mat34()
-    out.rot[:] = [float(x) for x in m[:9]]
-    out.trans[:] = [float(x) for x in m[9:12]]
+    v = m.tolist() if getattr(m, "ndim", 0) == 1 else [float(x) for x in m[:12]]  # flat arrays in one step
+    out.rot[:] = v[:9]
+    out.trans[:] = v[9:12]
     return out
 
 
@@ -63,17 +64,19 @@ def RenderSolverMaps(views, width, height, surfels, stream=None, **kw):
     ri = render_input(views, width, height, surfels, ptr=ptr, **kw)
     ro = _abi.RenderOutput()
     maps = {name: [] for name in MAPS}
-    for v in range(len(views)):
-        for name in MAPS:
-            t = torch.empty((height, width) if name == "index_map" else (height, width, 4),
-                            dtype=torch.int32 if name == "index_map" else torch.float32, device="cuda")
+    # one z buffer for all views (host time: an allocation each was a third of the call's 64 us)
+    z = torch.empty((len(views), height, width), dtype=torch.int64, device="cuda")
+    for name in MAPS:
+        shape, dtype = ((height, width), torch.int32) if name == "index_map" else ((height, width, 4), torch.float32)
+        addresses = getattr(ro, name)
+        for v in range(len(views)):
+            t = torch.empty_like(t) if v else torch.empty(shape, dtype=dtype, device="cuda")
             maps[name].append(t)
-            getattr(ro, name)[v] = t.data_ptr()
-        z = torch.empty((height, width), dtype=torch.int64, device="cuda")
-        keep.append(z)
-        ro.zbuffer[v] = z.data_ptr()
+            addresses[v] = t.data_ptr()
+    for v in range(len(views)):
+        ro.zbuffer[v] = z.data_ptr() + 8 * height * width * v
     rc = lib().mvdr_render_solver_maps(C.byref(ri), C.byref(ro), _stream_handle(stream))
     if rc != 0:
         raise SolverError(rc, "mvdr_render_solver_maps failed")
-    torch.cuda.synchronize()
+    _synchronize()
     return maps

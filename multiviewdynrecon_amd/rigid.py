@@ -41,7 +41,7 @@ def rigid_input(views, width, height, ptr):
 
 
 def mat34_array(m):
-    return np.array(list(m.rot) + list(m.trans), np.float32)
+    return np.frombuffer(m, np.float32).copy()
 
 
 class RigidSolver:
@@ -85,4 +85,4 @@ class RigidSolver:
         rc = lib().mvdr_rigid_get_pose(self.h, poses, C.byref(avg))
         if rc != 0:
             raise SolverError(rc, "mvdr_rigid_get_pose failed")
-        return np.stack([mat34_array(poses[v]) for v in range(self._views)]), mat34_array(avg)
+        return np.frombuffer(poses, np.float32).reshape(3, 12)[:self._views].copy(), mat34_array(avg)

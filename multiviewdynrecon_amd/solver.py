@@ -91,9 +91,8 @@ def lib():
 _HIP = None
 
 
-def _memcpy_d2h(dst, src, nbytes):
-    """hipMemcpy device -> host through the process's HIP runtime (the one torch
-    loaded, found by its soname)."""
+def _hip():
+    """The process's HIP runtime (the one torch loaded, found by its soname)."""
     global _HIP
     if _HIP is None:
         import torch  # noqa: F401  (loads the runtime)
@@ -101,15 +100,31 @@ def _memcpy_d2h(dst, src, nbytes):
         _HIP = C.CDLL("libamdhip64.so.7")
         _HIP.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
         _HIP.hipMemcpy.restype = C.c_int
-    rc = _HIP.hipMemcpy(dst, src, nbytes, 2)  # hipMemcpyDeviceToHost
+    return _HIP
+
+
+def _memcpy_d2h(dst, src, nbytes):
+    """hipMemcpy device -> host."""
+    rc = _hip().hipMemcpy(dst, src, nbytes, 2)  # hipMemcpyDeviceToHost
     if rc != 0:
         raise SolverError(4, f"hipMemcpy failed ({rc})")
+
+
+def _synchronize():
+    """All work of the current device, without torch's checks around the call."""
+    rc = _hip().hipDeviceSynchronize()
+    if rc != 0:
+        raise SolverError(4, f"hipDeviceSynchronize failed ({rc})")
 
 
 def _stream_handle(stream):
     if stream is None:
         import torch
 
+        # the handle alone where torch offers it: a Stream object costs ~4 us to build
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None and torch.cuda.is_initialized():
+            return C.c_void_p(raw(torch.cuda.current_device()))
         return C.c_void_p(torch.cuda.current_stream().cuda_stream)
     if isinstance(stream, int):
         return C.c_void_p(stream)

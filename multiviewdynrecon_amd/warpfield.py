@@ -30,7 +30,7 @@ def lib():
 
 
 def _p(t):
-    return C.c_void_p(t.data_ptr()) if t is not None and t.numel() else None
+    return t.data_ptr() if t is not None and t.numel() else None
 
 
 def _check(rc, what):
