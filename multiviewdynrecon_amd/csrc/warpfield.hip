@@ -471,11 +471,19 @@ __device__ inline DQ dq_mul(const DQ& a, const DQ& b) {
 }
 
 // computeCorrespondenceGuidedNodesSE3 with computeSuitableCorrespondenceGuidedSe3
-// (NonRigidSolver.cu:100-138, :155-167): one thread per node.
+// (NonRigidSolver.cu:100-138, :155-167): 32 lanes per node, one per pixel of the 5 x 5
+// window (columns outer); the nearest of the suitable pixels wins, the first of equals.
+// Bound by two dependent reads (maps, then the winner's transform): 4018 nodes 7.6
+// us; a thread per node walked its 25 pixels one after another in 16 workgroups,
+// 33 us.
+constexpr uint32_t kCorrLanes = 32;
 __global__ void __launch_bounds__(256) correction_kernel(CorrViews r, const float4* __restrict__ nodes,
                                                          const float* __restrict__ error, uint32_t num_nodes,
                                                          DQ* __restrict__ correction) {
-    for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < num_nodes; n += gridDim.x * blockDim.x) {
+    constexpr uint32_t kSide = 2 * kCorrHalfWindow + 1;
+    const uint32_t lane = threadIdx.x % kCorrLanes, first = threadIdx.x & (64 - kCorrLanes);  // first: in the wave
+    for (uint32_t n = (blockIdx.x * blockDim.x + threadIdx.x) / kCorrLanes; n < num_nodes;
+         n += gridDim.x * blockDim.x / kCorrLanes) {
         const float e = error[n];
         DQ out;
         out.q0 = make_float4(0.f, 0.f, 0.f, 1.f);
@@ -490,14 +498,14 @@ __global__ void __launch_bounds__(256) correction_kernel(CorrViews r, const floa
             const bool room = r.W > 2 * kCorrHalfWindow && r.H > 2 * kCorrHalfWindow;  // the window fits the map
             if (room && !(u >= r.W - kCorrHalfWindow || u < kCorrHalfWindow || y >= r.H - kCorrHalfWindow ||
                           y < kCorrHalfWindow)) {
-                float best = 1e6f;
-                for (uint32_t i = u - kCorrHalfWindow; i <= u + kCorrHalfWindow; ++i)
-                    for (uint32_t j = y - kCorrHalfWindow; j <= y + kCorrHalfWindow; ++j) {
-                        const size_t o = (size_t)j * r.W + i;
-                        const float4 pv = r.prev[v][o];
-                        if (r.valid[v][o] != 1 || is_zero_vertex(pv)) continue;
-                        const float* g = r.guided[v] + 12 * o;
-                        Mat34 G;
+                uint32_t mine = 0xFFFFFFFFu;  // squared distance (its bits) of a suitable pixel
+                Mat34 G = sel;
+                if (lane < kSide * kSide) {
+                    const uint32_t column = u - kCorrHalfWindow + lane / kSide, row = y - kCorrHalfWindow + lane % kSide;
+                    const size_t o = (size_t)row * r.W + column;
+                    const float4 pv = r.prev[v][o];
+                    const float* g = r.guided[v] + 12 * o;
+                    if (r.valid[v][o] == 1 && !is_zero_vertex(pv)) {
                         G.c0 = mk(g[0], g[1], g[2]);
                         G.c1 = mk(g[3], g[4], g[5]);
                         G.c2 = mk(g[6], g[7], g[8]);
@@ -505,16 +513,25 @@ __global__ void __launch_bounds__(256) correction_kernel(CorrViews r, const floa
                         const f3 d = c - xyz(pv);
                         const float d2 = dot3(d, d);
                         const f3 m = G.apply(c) - c;
-                        if (best > d2 && d2 < 1e-4f && dot3(m, m) < 4 * (kNodeRadius * kNodeRadius)) {
-                            best = d2;
-                            sel = G;
-                        }
+                        if (d2 < 1e-4f && dot3(m, m) < 4 * (kNodeRadius * kNodeRadius)) mine = __float_as_uint(d2);
                     }
+                }
+                uint32_t best = mine;
+#pragma unroll
+                for (uint32_t s = 1; s < kCorrLanes; s *= 2) best = min(best, (uint32_t)__shfl_xor((int)best, s, 64));
+                if (best != 0xFFFFFFFFu) {
+                    const uint64_t winners = __ballot(mine == best) >> first;
+                    const int from = (int)first + __builtin_ctz((uint32_t)winners);
+                    sel.c0 = mk(__shfl(G.c0.x, from, 64), __shfl(G.c0.y, from, 64), __shfl(G.c0.z, from, 64));
+                    sel.c1 = mk(__shfl(G.c1.x, from, 64), __shfl(G.c1.y, from, 64), __shfl(G.c1.z, from, 64));
+                    sel.c2 = mk(__shfl(G.c2.x, from, 64), __shfl(G.c2.y, from, 64), __shfl(G.c2.z, from, 64));
+                    sel.t = mk(__shfl(G.t.x, from, 64), __shfl(G.t.y, from, 64), __shfl(G.t.z, from, 64));
+                }
                 sel = compose(compose(compose(compose(r.w2c_inv[v], r.init[v]), sel), r.init_inv[v]), r.w2c[v]);
             }
             out = dq_scale(dq_from_mat34(sel), e);
         }
-        correction[n] = out;
+        if (lane == 0) correction[n] = out;
     }
 }
 
@@ -646,7 +663,8 @@ mvdr_status mvdr_warp_correct_nodes(const mvdr_node_correction* in, void* stream
         r.valid[v] = static_cast<const uint8_t*>(in->guided_valid[v]);
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(correction_kernel, dim3(stream_grid(in->num_nodes)), dim3(256), 0, st, r,
+    constexpr uint32_t kCorrNodes = 256 / kCorrLanes;  // per workgroup
+    hipLaunchKernelGGL(correction_kernel, dim3((in->num_nodes + kCorrNodes - 1) / kCorrNodes), dim3(256), 0, st, r,
                        static_cast<const float4*>(in->live_nodes), static_cast<const float*>(in->node_error),
                        in->num_nodes, static_cast<DQ*>(in->correction));
     hipLaunchKernelGGL(apply_correction_kernel, dim3(stream_grid(in->num_surfels + in->num_nodes)), dim3(256), 0, st,
