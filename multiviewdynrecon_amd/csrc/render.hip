@@ -6,7 +6,9 @@
 // equal depths keep the lower surfel index, as the reference's depth test
 // does in draw order.  Both passes stream their arrays once (HBM bound:
 // 64 B of surfel attributes read per surfel, 8 B atomic per drawn surfel,
-// ~88 B written per pixel).
+// ~88 B written per pixel).  A workgroup draws one view (grid.y), whose camera and
+// addresses are scalars then.  159k surfels into three 640 x 480 views: clear 4 us, splat
+// 15.5 (the atomics: looking before them takes 17.6), resolve 19.3 (20.8 with plain stores).
 #pragma clang fp contract(off)
 
 #include <hip/hip_runtime.h>
@@ -42,20 +44,19 @@ struct RenderMaps {
     unsigned long long* z[kMaxViews];
 };
 
-__global__ void __launch_bounds__(256) zclear_kernel(RenderMaps m, uint32_t V, uint32_t pixels) {
-    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < V * pixels; p += gridDim.x * blockDim.x) {
-        const uint32_t v = p / pixels;
-        m.z[v][p - v * pixels] = ~0ull;
-    }
+__global__ void __launch_bounds__(256) zclear_kernel(RenderMaps m, uint32_t pixels) {
+    unsigned long long* z = m.z[blockIdx.y];
+    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < pixels; p += gridDim.x * blockDim.x) z[p] = ~0ull;
 }
 
 __global__ void __launch_bounds__(256) splat_kernel(RenderViews r, RenderMaps m) {
-    const uint32_t total = r.V * r.S;
-    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < total; g += gridDim.x * blockDim.x) {
-        const uint32_t v = g / r.S, s = g - v * r.S;
-        const f3 p = r.w2c[v].apply(xyz(r.warp_v[v][s]));
+    const uint32_t v = blockIdx.y;
+    for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < r.S; s += gridDim.x * blockDim.x) {
+        const float4 vertex = r.warp_v[v][s];
+        const float confidence = r.ref_v[v][s].w;
+        const f3 p = r.w2c[v].apply(xyz(vertex));
         if (p.z > r.max_depth + 0.05f || p.z < 0.f) continue;
-        if (r.ref_v[v][s].w < r.conf_thr && fabsf(r.color_time[s].z - r.now) >= r.time_thr) continue;
+        if (confidence < r.conf_thr && fabsf(r.color_time[s].z - r.now) >= r.time_thr) continue;
         const float u = (r.fx[v] * p.x) / p.z + r.cx[v];
         const float w = (r.fy[v] * p.y) / p.z + r.cy[v];
         if (!(u >= 0.f && w >= 0.f && u < (float)r.W && w < (float)r.H)) continue;
@@ -70,10 +71,15 @@ __device__ inline float4 decode_rgb(float4 ct) {
                        (float)(c & 0x000000FF) / 255.f, ct.y);
 }
 
+// The maps are 77 MB, no cache keeps them: streaming stores.
+__device__ inline void stream(float4* p, float4 v) {
+    typedef float vec4 __attribute__((ext_vector_type(4)));
+    __builtin_nontemporal_store(vec4{v.x, v.y, v.z, v.w}, reinterpret_cast<vec4*>(p));
+}
+
 __global__ void __launch_bounds__(256) resolve_kernel(RenderViews r, RenderMaps m) {
-    const uint32_t pixels = r.W * r.H;
-    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < r.V * pixels; g += gridDim.x * blockDim.x) {
-        const uint32_t v = g / pixels, o = g - v * pixels;
+    const uint32_t pixels = r.W * r.H, v = blockIdx.y;
+    for (uint32_t o = blockIdx.x * blockDim.x + threadIdx.x; o < pixels; o += gridDim.x * blockDim.x) {
         const unsigned long long key = m.z[v][o];
         const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
         float4 rv = zero, rn = zero, wv = zero, wn = zero, rgb = zero;
@@ -87,12 +93,12 @@ __global__ void __launch_bounds__(256) resolve_kernel(RenderViews r, RenderMaps 
             wn = make_float4(d.x, d.y, d.z, 0.f);
             rgb = decode_rgb(r.color_time[idx]);
         }
-        m.ref_v[v][o] = rv;
-        m.ref_n[v][o] = rn;
-        m.warp_v[v][o] = wv;
-        if (m.warp_n[v]) m.warp_n[v][o] = wn;
-        m.index[v][o] = idx;
-        if (m.rgb[v]) m.rgb[v][o] = rgb;
+        stream(m.ref_v[v] + o, rv);
+        stream(m.ref_n[v] + o, rn);
+        stream(m.warp_v[v] + o, wv);
+        if (m.warp_n[v]) stream(m.warp_n[v] + o, wn);
+        __builtin_nontemporal_store(idx, m.index[v] + o);
+        if (m.rgb[v]) stream(m.rgb[v] + o, rgb);
     }
 }
 
@@ -148,8 +154,8 @@ extern "C" mvdr_status mvdr_render_solver_maps(const mvdr_render_input* in, cons
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint32_t pixels = r.W * r.H;
-    hipLaunchKernelGGL(zclear_kernel, dim3(grid_for((uint64_t)r.V * pixels)), dim3(256), 0, st, m, r.V, pixels);
-    if (r.S) hipLaunchKernelGGL(splat_kernel, dim3(grid_for((uint64_t)r.V * r.S)), dim3(256), 0, st, r, m);
-    hipLaunchKernelGGL(resolve_kernel, dim3(grid_for((uint64_t)r.V * pixels)), dim3(256), 0, st, r, m);
+    hipLaunchKernelGGL(zclear_kernel, dim3(grid_for(pixels), r.V), dim3(256), 0, st, m, pixels);
+    if (r.S) hipLaunchKernelGGL(splat_kernel, dim3(grid_for(r.S), r.V), dim3(256), 0, st, r, m);
+    hipLaunchKernelGGL(resolve_kernel, dim3(grid_for(pixels), r.V), dim3(256), 0, st, r, m);
     return hipGetLastError() == hipSuccess ? MVDR_OK : MVDR_E_HIP;
 }
