@@ -553,6 +553,29 @@ __device__ inline int term_nodes(const Buffers& b, const FrameDev& f, const uint
     return 4;
 }
 
+// The node words of term t, read and not yet looked at (term_nodes would wait for them
+// in each of its branches): two packed node numbers each, the second unused by an edge.
+struct TermWords {
+    uint32_t lo, hi;
+    bool edge;
+};
+__device__ inline TermWords term_words(const Buffers& b, const FrameDev& f, const uint32_t off[5], uint32_t t) {
+    TermWords w;
+    w.edge = t >= off[0] && t < off[1];
+    const void* p = b.dense_knn + t;
+    if (t >= off[0]) p = f.graph + (t - off[0]);
+    if (t >= off[1]) p = &b.fg[t - off[1]].knn;
+    if (t >= off[2]) p = &b.feat[t - off[2]].knn;
+    if (t >= off[3]) p = &b.cross[t - off[3]].knn;
+    const uint32_t* q = static_cast<const uint32_t*>(p);
+    w.lo = q[0];
+    w.hi = q[w.edge ? 0 : 1];
+    return w;
+}
+__device__ inline ushort4 words_nodes(const TermWords& w) {
+    return make_ushort4((uint16_t)w.lo, (uint16_t)(w.lo >> 16), (uint16_t)w.hi, (uint16_t)(w.hi >> 16));
+}
+
 __device__ inline uint32_t slot(ushort4 k, int q) { return q == 0 ? k.x : (q == 1 ? k.y : (q == 2 ? k.z : k.w)); }
 
 // The reference builds Node2Term by a stable key sort of (node, term) pairs
@@ -571,6 +594,7 @@ __device__ inline uint32_t slot(ushort4 k, int q) { return q == 0 ? k.x : (q == 
 // counters, twice the resident workgroups).
 constexpr uint32_t kChunkTerms = 512;      // chunk of a launch the chip holds at once; the capacity unit
 constexpr uint32_t kBigChunkTerms = 2048;  // chunk of a larger launch (half the histogram rows)
+constexpr uint32_t kHistRounds = 8;
 constexpr uint32_t kHistNodes = 16384;  // largest LDS node tile (32 KB of u16 counters)
 static_assert(4 * kBigChunkTerms <= 0xFFFFu && kBigChunkTerms % kChunkTerms == 0,
               "per-chunk node counts must fit 16 bits");
@@ -604,22 +628,17 @@ __global__ void __launch_bounds__(64) n2t_hist_kernel(const Buffers* __restrict_
         const uint32_t span = min(tile, N - n0);
         for (uint32_t k = threadIdx.x; k < (span + 1) / 2; k += 64) hist[k] = 0;
         wave_lds_sync();
-        // four rounds of term nodes in flight, then their counts
-        for (uint32_t tb = t0 + threadIdx.x; tb < t1; tb += 4 * 64) {
-            ushort4 k[4];
-            int m[4];
+        // eight rounds of term nodes in flight, then their counts
+        for (uint32_t tb = t0 + threadIdx.x; tb < t1; tb += kHistRounds * 64) {
+            TermWords w[kHistRounds];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t t = tb + 64 * r;
-                k[r] = make_ushort4(0, 0, 0, 0);
-                m[r] = t < t1 ? term_nodes(b, f, off, t, k[r]) : 0;
-            }
+            for (uint32_t r = 0; r < kHistRounds; ++r) w[r] = term_words(b, f, off, min(tb + 64 * r, t1 - 1));
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+            for (uint32_t r = 0; r < kHistRounds; ++r)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const uint32_t n = slot(k[r], q);
-                    if (q >= m[r]) continue;
+                    const uint32_t n = slot(words_nodes(w[r]), q);
+                    if (tb + 64 * r >= t1 || (q >= 2 && w[r].edge)) continue;
                     if (n >= N) {
                         if (n0 == 0) atomicOr(&c.error, kErrNodes);
                     } else if (n >= n0 && n - n0 < span) {
@@ -749,26 +768,6 @@ __device__ inline void rank_entries(RankTable& table, const uint32_t n[4], uint3
     }
 }
 
-// The node words of term t, read and not yet looked at (term_nodes would wait for them
-// in each of its branches): two packed node numbers each, the second unused by an edge.
-struct TermWords {
-    uint32_t lo, hi;
-    bool edge;
-};
-__device__ inline TermWords term_words(const Buffers& b, const FrameDev& f, const uint32_t off[5], uint32_t t) {
-    TermWords w;
-    w.edge = t >= off[0] && t < off[1];
-    const void* p = b.dense_knn + t;
-    if (t >= off[0]) p = f.graph + (t - off[0]);
-    if (t >= off[1]) p = &b.fg[t - off[1]].knn;
-    if (t >= off[2]) p = &b.feat[t - off[2]].knn;
-    if (t >= off[3]) p = &b.cross[t - off[3]].knn;
-    const uint32_t* q = static_cast<const uint32_t*>(p);
-    w.lo = q[0];
-    w.hi = q[w.edge ? 0 : 1];
-    return w;
-}
-
 // Places a chunk's entries: an entry goes to its node's list offset plus the node's
 // entries in earlier chunks, in earlier rounds of 64 terms (cur) and in earlier lanes of
 // the round (its rank).  The nodes and list positions of kPlaceRounds rounds are read
@@ -887,6 +886,10 @@ __global__ void __launch_bounds__(1024) node_scan_kernel(const Buffers* __restri
 // single waves, so LDS traffic between lanes needs no workgroup barrier.
 constexpr uint32_t kRowHash = kRowPartners;  // partner set capacity per row
 
+// Where a partner's search in the set begins.
+__device__ inline uint32_t row_hash(uint32_t v) { return (v * 2654435761u) >> 23; }
+static_assert(kRowHash == 1u << 9, "9 hash bits");
+
 // Partners of node i in term t with the reference's pair multiplicity: every
 // knn slot q with knn[q] != i, or the other end of a non-loop graph edge.
 __device__ inline ushort4 partners_of(ushort4 k, int m, uint32_t i) {
@@ -962,32 +965,49 @@ __global__ void __launch_bounds__(64 * kWaves) pair_rows_kernel(const Buffers* _
         kq[u] = make_ushort4(0, 0, 0, 0);
         mq[u] = 0;
     }
-    for (uint32_t p0 = beg + tid; p0 < end; p0 += kBatch * 64 * kWaves) {
+    uint32_t off[5];
 #pragma unroll
-        for (int u = 0; u < (int)kBatch; ++u) {
-            const uint32_t p = p0 + u * 64 * kWaves;
-            kq[u] = make_ushort4(0, 0, 0, 0);
-            mq[u] = p < end ? term_nodes(b, f, c.off, b.n2t_index[p], kq[u]) : 0;
+    for (int k = 0; k < 5; ++k) off[k] = c.off[k];
+    auto batch_nodes = [&](uint32_t p0) {
+        uint32_t t[kBatch];
+        TermWords w[kBatch];
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) t[u] = b.n2t_index[min(p0 + u * 64 * kWaves, end - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) w[u] = term_words(b, f, off, t[u]);
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) {
+            kq[u] = words_nodes(w[u]);
+            mq[u] = p0 + u * 64 * kWaves >= end ? 0 : w[u].edge ? 2 : 4;
         }
+    };
+    for (uint32_t p0 = beg + tid; p0 < end; p0 += kBatch * 64 * kWaves) {
+        batch_nodes(p0);
         ushort4 oq[kBatch];
 #pragma unroll
         for (int u = 0; u < (int)kBatch; ++u)
             oq[u] = mq[u] ? partners_of(kq[u], mq[u], i) : make_ushort4(0xFFFF, 0xFFFF, 0xFFFF, 0xFFFF);
+        // most partners are present where they hash to: plain reads, all at once, settle
+        // them (one after another, here and in the column pass, they were a chain of 32
+        // LDS reads; 4k nodes 26 -> 22.5 us with the batch's term nodes read together)
+        uint32_t seen[4 * kBatch];
+#pragma unroll
+        for (int uq = 0; uq < (int)(4 * kBatch); ++uq) seen[uq] = set[row_hash(slot(oq[uq / 4], uq % 4))];
 #pragma unroll
         for (int uq = 0; uq < (int)(4 * kBatch); ++uq) {
             const uint32_t v = slot(oq[uq / 4], uq % 4);
             if (v == 0xFFFF) continue;
             upper_entries += v > i ? 1u : 0u;
-            uint32_t h = (v * 2654435761u) >> 23;  // 9 bits
+            if (seen[uq] == v) continue;
+            uint32_t h = row_hash(v);
             for (uint32_t probe = 0;; ++probe) {
                 if (probe == kRowHash) {
                     overflow = true;
                     break;
                 }
-                // most partners are already present: a plain read settles them
-                const uint32_t seen = set[h];
-                if (seen == v) break;
-                if (seen == 0xFFFFFFFFu) {
+                const uint32_t now = set[h];
+                if (now == v) break;
+                if (now == 0xFFFFFFFFu) {
                     const uint32_t old = atomicCAS(&set[h], 0xFFFFFFFFu, v);
                     if (old == 0xFFFFFFFFu || old == v) break;
                 }
@@ -1063,14 +1083,10 @@ __global__ void __launch_bounds__(64 * kWaves) pair_rows_kernel(const Buffers* _
         for (uint32_t u = tid; u < up; u += 64 * kWaves) rp[u] = (uint16_t)ul[u];
         for (uint32_t k = tid; k < low; k += 64 * kWaves) rp[up + k] = (uint16_t)ll[k];
         for (uint32_t p0 = beg + tid; p0 < end; p0 += kBatch * 64 * kWaves) {
-            if (!one_batch) {
+            if (!one_batch) batch_nodes(p0);
+            uint32_t seen[4 * kBatch];
 #pragma unroll
-                for (int u = 0; u < (int)kBatch; ++u) {
-                    const uint32_t p = p0 + u * 64 * kWaves;
-                    kq[u] = make_ushort4(0, 0, 0, 0);
-                    mq[u] = p < end ? term_nodes(b, f, c.off, b.n2t_index[p], kq[u]) : 0;
-                }
-            }
+            for (int uq = 0; uq < (int)(4 * kBatch); ++uq) seen[uq] = set[row_hash(slot(kq[uq / 4], uq % 4))];
 #pragma unroll
             for (int u = 0; u < (int)kBatch; ++u) {
                 const uint32_t p = p0 + u * 64 * kWaves;
@@ -1084,10 +1100,13 @@ __global__ void __launch_bounds__(64 * kWaves) pair_rows_kernel(const Buffers* _
                         uint32_t col = 0xFFu;
                         if (v != 0xFFFF && v > i) {
                             // v is in the set: its slot holds its column (above the node)
-                            uint32_t h = (v * 2654435761u) >> 23;
-                            for (uint32_t probe = 0; probe < kRowHash && (set[h] & 0xFFFFu) != v; ++probe)
+                            uint32_t entry = seen[4 * u + q];
+                            uint32_t h = row_hash(v);
+                            for (uint32_t probe = 1; probe < kRowHash && (entry & 0xFFFFu) != v; ++probe) {
                                 h = (h + 1) & (kRowHash - 1);
-                            col = (set[h] & 0xFFFFu) == v ? set[h] >> 16 : 0xFFu;
+                                entry = set[h];
+                            }
+                            col = (entry & 0xFFFFu) == v ? entry >> 16 : 0xFFu;
                         }
                         packed |= col << (8 * q);
                     }
