@@ -89,7 +89,8 @@ __device__ inline void tile_edges(const CvFrame& f, uint32_t base, uint8_t (&e)[
 }
 
 // The listed edge pixels with their candidates and minima cleared, and the flags
-// and tile counts of all pixels; one counter update per workgroup (one per wave and round took 50 us, all on one address).
+// and tile counts of all pixels; one counter update per workgroup (one per wave and
+// round took 50 us, all on one address).
 __global__ void __launch_bounds__(kCvThreads) cv_edges_kernel(CvFrame f, CvBuffers b, uint32_t tiles) {
     const uint32_t pixels = f.V * f.W * f.H, base = blockIdx.x * kCvTile;
     const uint32_t wave = threadIdx.x >> 6;

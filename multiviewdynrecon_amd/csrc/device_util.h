@@ -1,5 +1,5 @@
 // Wave64 / workgroup primitives used by the solver kernels: lane prefixes,
-// block sums and scans, LDS bitonic sort, bordered map fetches.
+// exchanges, sums and scans over lanes and blocks, bordered map fetches.
 #pragma once
 
 #include "common.h"
@@ -177,30 +177,6 @@ __device__ inline uint32_t block_exclusive_scan_1024(const uint32_t* in, uint32_
     if (max_out) *max_out = gmax;
     __syncthreads();
     return total;
-}
-
-__device__ inline uint32_t next_pow2(uint32_t v) {
-    uint32_t m = 1;
-    while (m < v) m <<= 1;
-    return m;
-}
-
-// Ascending bitonic sort of m (a power of two) keys in LDS by the whole block.
-template <typename K>
-__device__ inline void bitonic_sort_lds(K* keys, uint32_t m) {
-    for (uint32_t k = 2; k <= m; k <<= 1)
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t i = threadIdx.x; i < (m >> 1); i += blockDim.x) {
-                const uint32_t lo = ((i / j) * 2 * j) + (i % j), hi = lo + j;
-                const bool asc = (lo & k) == 0;
-                const K a = keys[lo], c = keys[hi];
-                if ((a > c) == asc) {
-                    keys[lo] = c;
-                    keys[hi] = a;
-                }
-            }
-            __syncthreads();
-        }
 }
 
 // Map fetches with the reference textures' border addressing: zero outside.

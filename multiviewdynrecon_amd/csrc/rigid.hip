@@ -13,8 +13,8 @@
 //                      the 6x6 system by an FP64 Cholesky in registers and
 //                      updates the pose in device memory -- the next iteration
 //                      reads it there, so the host never waits.
-// 3 views of 640x480, 3 iterations with the pose read back: 1116 -> 102 us (the
-// solve 293 -> 6 us an iteration, where 27 threads added 1200 partials one after
+// 3 views of 640x480, 3 iterations with the pose read back: 1116 -> 87 us (the
+// solve 293 -> 5.4 us an iteration, where 27 threads added 1200 partials one after
 // another; the rows 60 -> 11 us).
 #pragma clang fp contract(off)
 

@@ -322,8 +322,8 @@ struct GraphSlots {
         worst = (uint32_t)__builtin_ctzll(__ballot(dist == worst_d));
     }
 };
-__global__ void __launch_bounds__(64 * kGraphWaves) node_graph_kernel(const float4* __restrict__ nodes, uint32_t num_nodes,
-                                                                      ushort2* __restrict__ graph) {
+__global__ void __launch_bounds__(64 * kGraphWaves)
+    node_graph_kernel(const float4* __restrict__ nodes, uint32_t num_nodes, ushort2* __restrict__ graph) {
     __shared__ NodeBoxes box;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t i = blockIdx.x * kGraphWaves + (threadIdx.x >> 6);
@@ -580,7 +580,8 @@ mvdr_status mvdr_warp_build_node_graph(const void* nodes, uint32_t num_nodes, vo
     if (!nodes || !graph) return MVDR_E_INVALID;
     if (num_nodes > 65535) return MVDR_E_SHAPE;
     hipLaunchKernelGGL(node_graph_kernel, dim3((num_nodes + kGraphWaves - 1) / kGraphWaves), dim3(64 * kGraphWaves), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const float4*>(nodes), num_nodes, static_cast<ushort2*>(graph));
+                       static_cast<hipStream_t>(stream), static_cast<const float4*>(nodes), num_nodes,
+                       static_cast<ushort2*>(graph));
     return hipGetLastError() == hipSuccess ? MVDR_OK : MVDR_E_HIP;
 }
 
@@ -592,8 +593,9 @@ mvdr_status mvdr_warp_skin(const void* vertices, uint32_t num_vertices, const vo
     if (!nknn || !nw) return MVDR_E_INVALID;
     const uint64_t total = (uint64_t)num_vertices + num_nodes;
     if (total > 0xFFFFFFFFull - 255) return MVDR_E_SHAPE;
-    const uint32_t blocks = (num_vertices + 64 * kSkinWaves - 1) / (64 * kSkinWaves) + (num_nodes + kSkinWaves - 1) / kSkinWaves;
-    hipLaunchKernelGGL(skin_kernel, dim3(blocks), dim3(64 * kSkinWaves), 0, static_cast<hipStream_t>(stream),
+    constexpr uint32_t kSkinThreads = 64 * kSkinWaves;
+    const uint32_t blocks = (num_vertices + kSkinThreads - 1) / kSkinThreads + (num_nodes + kSkinWaves - 1) / kSkinWaves;
+    hipLaunchKernelGGL(skin_kernel, dim3(blocks), dim3(kSkinThreads), 0, static_cast<hipStream_t>(stream),
                        static_cast<const float4*>(vertices), num_vertices, static_cast<const float4*>(nodes), num_nodes,
                        node_radius, static_cast<ushort4*>(vknn), static_cast<float4*>(vw), static_cast<ushort4*>(nknn),
                        static_cast<float4*>(nw));
