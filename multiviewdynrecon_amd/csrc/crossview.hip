@@ -410,6 +410,8 @@ mvdr_status mvdr_crossview_create(const mvdr_crossview_config* config, mvdr_cros
     if (e == hipSuccess) {
         lay(static_cast<char*>(h->block));
         e = hipMemset(h->b.num_edges, 0, sizeof(uint32_t));
+        // the fill is done before a call on a stream that does not wait for the null stream
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     }
     // the getters read the totals without a copy (~10 us each)
     if (e == hipSuccess)
