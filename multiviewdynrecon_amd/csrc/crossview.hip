@@ -28,14 +28,12 @@
 
 #include "../../include/mvdr/crossview.h"
 #include "common.h"
+#include "crossview_tiles.h"
 #include "device_util.h"
 
 namespace mvdr {
 namespace {
 
-constexpr uint32_t kCvThreads = 256;
-constexpr uint32_t kCvRounds = 8;        // pixels per thread of a tile, their loads in flight together
-constexpr uint32_t kCvTile = kCvThreads * kCvRounds;  // source pixels per workgroup
 constexpr uint32_t kCvWaves = kCvThreads / 64;
 constexpr uint32_t kCvLists = 3;
 constexpr uint32_t kNoCandidate = 0xFFFFFFFFu;
@@ -189,7 +187,8 @@ __global__ void __launch_bounds__(256) cv_candidates_kernel(CvFrame f, CvBuffers
     const uint32_t plane = f.W * f.H;
     const uint32_t count = min(*b.num_edges, b.cap_edges);
     const uint32_t waves = gridDim.x * (blockDim.x / 64);
-    for (uint32_t w = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); w < count; w += waves) {
+    // 64-bit list positions here and in the flags: the step past the last may pass 2^32
+    for (uint64_t w = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); w < count; w += waves) {
         const uint32_t p = b.edges[w];
         const uint32_t v = p / plane;
         float4 src;
@@ -255,8 +254,8 @@ __device__ inline uint32_t pair_flags(const CvFrame& f, const CvBuffers& b, uint
 // wave's pixels mostly share a tile, so it adds once per tile it meets.
 __global__ void __launch_bounds__(kCvThreads) cv_flags_kernel(CvFrame f, CvBuffers b, uint32_t tiles) {
     const uint32_t count = min(*b.num_edges, b.cap_edges), pixels = f.V * f.W * f.H;
-    for (uint32_t base = blockIdx.x * kCvThreads; base < count; base += gridDim.x * kCvThreads) {
-        const uint32_t i = base + threadIdx.x;
+    for (uint64_t base = blockIdx.x * kCvThreads; base < count; base += gridDim.x * kCvThreads) {
+        const uint64_t i = base + threadIdx.x;
         uint32_t tile = 0xFFFFFFFFu, flag = 0;
         const uint32_t p = i < count ? b.edges[i] : pixels;
         if (p < pixels) {
@@ -385,7 +384,7 @@ mvdr_status mvdr_crossview_create(const mvdr_crossview_config* config, mvdr_cros
     if (pixels >= 0xFFFFFFFFull) return MVDR_E_SHAPE;
     auto* h = new mvdr_crossview();
     h->cfg = c;
-    h->tiles = (uint32_t)((pixels + kCvTile - 1) / kCvTile);
+    h->tiles = cv_tiles((uint32_t)pixels);
     size_t off = 0;
     auto carve = [&](auto*& p, size_t n, char* base) {
         using T = std::remove_reference_t<decltype(*p)>;
@@ -463,7 +462,7 @@ mvdr_status mvdr_crossview_find(mvdr_crossview* h, const mvdr_crossview_input* i
     }
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint32_t pixels = f.V * f.W * f.H;
-    const uint32_t tiles = (pixels + kCvTile - 1) / kCvTile;
+    const uint32_t tiles = cv_tiles(pixels);
     // candidates and flags loop over the edge list (its length is known on the
     // device alone)
     hipLaunchKernelGGL(cv_edges_kernel, dim3(tiles), dim3(kCvThreads), 0, st, f, h->b, tiles);

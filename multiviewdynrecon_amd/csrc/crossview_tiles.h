@@ -1,0 +1,14 @@
+// Split of the source pixels into workgroup tiles, for pixel counts up to 2^32 - 2.
+#pragma once
+
+namespace mvdr {
+
+constexpr uint32_t kCvThreads = 256;
+constexpr uint32_t kCvRounds = 8;        // pixels per thread of a tile, their loads in flight together
+constexpr uint32_t kCvTile = kCvThreads * kCvRounds;  // source pixels per workgroup
+static_assert((1ull << 32) % kCvTile == 0, "the last tile's pixel numbers fit 32 bits");
+
+// (Rounding up by a sum would pass 32 bits for the last counts.)
+__host__ __device__ inline uint32_t cv_tiles(uint32_t pixels) { return pixels / kCvTile + (pixels % kCvTile != 0); }
+
+}  // namespace mvdr
