@@ -187,8 +187,9 @@ __global__ void __launch_bounds__(256) cv_candidates_kernel(CvFrame f, CvBuffers
     const uint32_t plane = f.W * f.H;
     const uint32_t count = min(*b.num_edges, b.cap_edges);
     const uint32_t waves = gridDim.x * (blockDim.x / 64);
-    // 64-bit list positions here and in the flags: the step past the last may pass 2^32
-    for (uint64_t w = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6); w < count; w += waves) {
+    uint32_t w = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
+    if (w >= count) return;
+    do {
         const uint32_t p = b.edges[w];
         const uint32_t v = p / plane;
         float4 src;
@@ -213,7 +214,7 @@ __global__ void __launch_bounds__(256) cv_candidates_kernel(CvFrame f, CvBuffers
             const uint32_t t = cand.y * plane + (cand.x >> 16) * f.W + (cand.x & 0xFFFF);
             atomicMin(&b.best[t], ((unsigned long long)__float_as_uint(best) << 32) | p);
         }
-    }
+    } while (cv_step(w, waves, count));
 }
 
 __device__ inline uint32_t target_of(const CvFrame& f, uint2 c) {
@@ -254,8 +255,10 @@ __device__ inline uint32_t pair_flags(const CvFrame& f, const CvBuffers& b, uint
 // wave's pixels mostly share a tile, so it adds once per tile it meets.
 __global__ void __launch_bounds__(kCvThreads) cv_flags_kernel(CvFrame f, CvBuffers b, uint32_t tiles) {
     const uint32_t count = min(*b.num_edges, b.cap_edges), pixels = f.V * f.W * f.H;
-    for (uint64_t base = blockIdx.x * kCvThreads; base < count; base += gridDim.x * kCvThreads) {
-        const uint64_t i = base + threadIdx.x;
+    uint32_t base = blockIdx.x * kCvThreads;
+    if (base >= count) return;
+    do {
+        const uint32_t i = base + threadIdx.x;
         uint32_t tile = 0xFFFFFFFFu, flag = 0;
         const uint32_t p = i < count ? b.edges[i] : pixels;
         if (p < pixels) {
@@ -275,7 +278,7 @@ __global__ void __launch_bounds__(kCvThreads) cv_flags_kernel(CvFrame f, CvBuffe
             }
             left &= ~__ballot(mine);
         }
-    }
+    } while (cv_step(base, gridDim.x * kCvThreads, count));
 }
 
 __global__ void __launch_bounds__(1024) cv_scan_kernel(CvBuffers b, uint32_t tiles) {

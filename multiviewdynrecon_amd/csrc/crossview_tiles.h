@@ -1,4 +1,5 @@
-// Split of the source pixels into workgroup tiles, for pixel counts up to 2^32 - 2.
+// Split of the source pixels into workgroup tiles, and steps through their list, for
+// pixel counts up to 2^32 - 2.
 #pragma once
 
 namespace mvdr {
@@ -10,5 +11,14 @@ static_assert((1ull << 32) % kCvTile == 0, "the last tile's pixel numbers fit 32
 
 // (Rounding up by a sum would pass 32 bits for the last counts.)
 __host__ __device__ inline uint32_t cv_tiles(uint32_t pixels) { return pixels / kCvTile + (pixels % kCvTile != 0); }
+
+// The next list position of a strided loop, i < count; false past the end (i + step may
+// pass 32 bits there; with 64-bit positions the candidate search of 2 % edges took 98
+// us in place of 88, of all edges 3.66 ms in place of 2.45).
+__host__ __device__ inline bool cv_step(uint32_t& i, uint32_t step, uint32_t count) {
+    if (count - i <= step) return false;
+    i += step;
+    return true;
+}
 
 }  // namespace mvdr

@@ -1,6 +1,8 @@
-// csrc/crossview_tiles.h on the host: the tiles hold every pixel, and none is empty.
+// csrc/crossview_tiles.h on the host: the tiles hold every pixel, and none is empty; a
+// strided loop passes the positions below its count, and ends.
 #include <cstdint>
 #include <cstdio>
+#include <initializer_list>
 
 #define __device__
 #define __host__
@@ -19,5 +21,17 @@ int main() {
             return 1;
         }
     }
+    for (const uint32_t count : counts)
+        for (const uint32_t step : {8192u, 131072u, 0x40000000u}) {
+            // from the last positions, where the sum would pass 32 bits
+            const uint32_t first = count > 4 * step && step < 0x40000000u ? count - 4 * step : 0;
+            uint32_t i = first, steps = 1;
+            while (steps < 8 && cv_step(i, step, count)) ++steps;
+            const uint64_t want = (count - (uint64_t)first + step - 1) / step;
+            if (steps != want || i != first + (want - 1) * step) {
+                std::printf("count %u step %u: %u steps to %u\n", count, step, steps, i);
+                return 1;
+            }
+        }
     return 0;
 }
