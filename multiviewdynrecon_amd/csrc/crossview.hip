@@ -13,6 +13,12 @@
 // the first strict minimum of the scan).  With one thread per pixel the few
 // edge pixels of a wave walked 2 x 441 taps each in a chain, at one or two
 // active lanes: 493 us for three 640x480 views, 29 us now (all passes 525 -> 60 us).
+// With many edges the taps' arithmetic bounds it: the pixel and its views are the
+// wave's (scalars), a tap's place follows from the last one's by additions, and a
+// window inside the image needs no bounds.  All passes, 2 / 10 / 50 / 100 % edge
+// pixels of three 640x480 views: 70 / 192 / 773 / 1557 us; a division per tap and
+// addresses per lane 87 / 297 / 1291 / 2442; a thread per pixel 641 / 1129 / 1469 /
+// 1436 (its taps lie side by side, a wave's lie `step` apart: from ~90 % on it wins).
 // The list's order is arbitrary and no result depends on it: candidates and the
 // per-target 64-bit minimum (squared-distance bits << 32 | source pixel) are kept
 // per pixel, and the three lists are compacted in pixel order.
@@ -25,6 +31,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "../../include/mvdr/crossview.h"
 #include "common.h"
@@ -140,30 +147,46 @@ __device__ inline float nearest_in_view(const CvFrame& f, const CvBuffers& b, ui
     const uint32_t x0 = (uint32_t)project_round<float>(q.x, q.z, f.fx[n], f.cx[n]) - (uint32_t)b.radius;
     const uint32_t y0 = (uint32_t)project_round<float>(q.y, q.z, f.fy[n], f.cy[n]) - (uint32_t)b.radius;
     const uint32_t lane = threadIdx.x & 63;
+    // tap t is the window's (t / side, t % side); 64 taps on by two additions
+    const uint32_t rows = 64 / side, columns = 64 - rows * side;
+    uint32_t iy = lane / side, ix = lane - iy * side;
     constexpr uint32_t kTaps = 4;  // a lane's taps in flight
-    for (uint32_t t0 = lane; t0 < taps; t0 += 64 * kTaps) {
-        uint32_t o[kTaps];
-        uint8_t e[kTaps];
+    const uint8_t* edge = f.edge[n];
+    const float4* vertex = f.vertex[n];
+    auto scan = [&](auto inside) {
+        for (uint32_t t0 = lane; t0 < taps; t0 += 64 * kTaps) {
+            uint32_t o[kTaps];
+            uint8_t e[kTaps];
+            float4 v[kTaps];
 #pragma unroll
-        for (uint32_t k = 0; k < kTaps; ++k) {
-            const uint32_t t = t0 + 64 * k, iy = t / side, ix = t - iy * side;
-            const uint32_t x = x0 + ix * (uint32_t)b.step, y = y0 + iy * (uint32_t)b.step;
-            const bool in = t < taps && x < f.W && y < f.H;  // negative coordinates wrap above both
-            o[k] = in ? y * f.W + x : 0u;
-            e[k] = in ? f.edge[n][o[k]] : 0;
-        }
+            for (uint32_t k = 0; k < kTaps; ++k) {
+                const uint32_t x = x0 + ix * (uint32_t)b.step, y = y0 + iy * (uint32_t)b.step;
+                // negative coordinates wrap above both sizes
+                const bool in = t0 + 64 * k < taps && (decltype(inside)::value || (x < f.W && y < f.H));
+                o[k] = in ? y * f.W + x : 0u;
+                e[k] = in ? edge[o[k]] : 0;
+                const uint32_t next = ix + columns;
+                ix = next < side ? next : next - side;
+                iy += next < side ? rows : rows + 1;
+            }
 #pragma unroll
-        for (uint32_t k = 0; k < kTaps; ++k) {
-            float4 v;
-            if (e[k] != 1 || !edge_vertex(f, n, o[k], v)) continue;
-            const float dx = v.x - q.x, dy = v.y - q.y, dz = v.z - q.z;
-            const float d2 = dx * dx + dy * dy + dz * dz;
-            if (d2 < best) {
-                best = d2;
-                at = t0 + 64 * k;
+            for (uint32_t k = 0; k < kTaps; ++k) {
+                v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (e[k] == 1) v[k] = vertex[o[k]];
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < kTaps; ++k) {
+                const float dx = v[k].x - q.x, dy = v[k].y - q.y, dz = v[k].z - q.z;
+                const float d2 = dx * dx + dy * dy + dz * dz;
+                const bool nearer = !zero_vertex(v[k]) && d2 < best;
+                best = nearer ? d2 : best;
+                at = nearer ? t0 + 64 * k : at;
             }
         }
-    }
+    };
+    const uint32_t last = (side - 1) * (uint32_t)b.step;
+    if (x0 < f.W && y0 < f.H && last < f.W - x0 && last < f.H - y0) scan(std::true_type{});
+    else scan(std::false_type{});
     // the smallest distance, and of equal ones the first in the scan
     unsigned long long key = ((unsigned long long)__float_as_uint(best) << 32) | at;
 #pragma unroll
@@ -174,9 +197,9 @@ __device__ inline float nearest_in_view(const CvFrame& f, const CvBuffers& b, ui
     best = __uint_as_float((uint32_t)(key >> 32));
     at = (uint32_t)key;
     if (at != 0xFFFFFFFFu) {
-        const uint32_t iy = at / side;
-        bx = x0 + (at - iy * side) * (uint32_t)b.step;
-        by = y0 + iy * (uint32_t)b.step;
+        const uint32_t row = at / side;
+        bx = x0 + (at - row * side) * (uint32_t)b.step;
+        by = y0 + row * (uint32_t)b.step;
     }
     return best;
 }
@@ -190,7 +213,7 @@ __global__ void __launch_bounds__(256) cv_candidates_kernel(CvFrame f, CvBuffers
     uint32_t w = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
     if (w >= count) return;
     do {
-        const uint32_t p = b.edges[w];
+        const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane((int)b.edges[w]);
         const uint32_t v = p / plane;
         float4 src;
         if (f.V < 2 || v >= f.V || !edge_vertex(f, v, p - v * plane, src)) continue;
