@@ -471,17 +471,20 @@ __device__ inline DQ dq_mul(const DQ& a, const DQ& b) {
 }
 
 // computeCorrespondenceGuidedNodesSE3 with computeSuitableCorrespondenceGuidedSe3
-// (NonRigidSolver.cu:100-138, :155-167): 32 lanes per node, one per pixel of the 5 x 5
+// (NonRigidSolver.cu:100-138, :155-167): 16 lanes per node for the 25 pixels of its 5 x 5
 // window (columns outer); the nearest of the suitable pixels wins, the first of equals.
-// Bound by two dependent reads (maps, then the winner's transform): 4018 nodes 7.6
-// us; a thread per node walked its 25 pixels one after another in 16 workgroups,
-// 33 us.
-constexpr uint32_t kCorrLanes = 32;
+// Few nodes are bound by dependent reads (maps, transforms near enough, the winner's
+// transform), many by the motion's arithmetic, which every lane of a node repeats.
+// 100 / 4018 / 16000 / 65535 nodes 7.2 / 7.0 / 10.8 / 28.3 us; with 32 lanes 6.7 / 7.5 /
+// 14.9 / 43.3, with 8 lanes 7.7 / 8.5 / 10.2 / 21.7; a thread per node 22.7 / 27.5 /
+// 25.6 / 28.5.
+constexpr uint32_t kCorrLanes = 16;
 __global__ void __launch_bounds__(256) correction_kernel(CorrViews r, const float4* __restrict__ nodes,
                                                          const float* __restrict__ error, uint32_t num_nodes,
                                                          DQ* __restrict__ correction) {
-    constexpr uint32_t kSide = 2 * kCorrHalfWindow + 1;
-    const uint32_t lane = threadIdx.x % kCorrLanes, first = threadIdx.x & (64 - kCorrLanes);  // first: in the wave
+    constexpr uint32_t kSide = 2 * kCorrHalfWindow + 1, kPixels = kSide * kSide;
+    constexpr uint32_t kRounds = (kPixels + kCorrLanes - 1) / kCorrLanes;
+    const uint32_t lane = threadIdx.x % kCorrLanes;
     for (uint32_t n = (blockIdx.x * blockDim.x + threadIdx.x) / kCorrLanes; n < num_nodes;
          n += gridDim.x * blockDim.x / kCorrLanes) {
         const float e = error[n];
@@ -498,35 +501,47 @@ __global__ void __launch_bounds__(256) correction_kernel(CorrViews r, const floa
             const bool room = r.W > 2 * kCorrHalfWindow && r.H > 2 * kCorrHalfWindow;  // the window fits the map
             if (room && !(u >= r.W - kCorrHalfWindow || u < kCorrHalfWindow || y >= r.H - kCorrHalfWindow ||
                           y < kCorrHalfWindow)) {
-                uint32_t mine = 0xFFFFFFFFu;  // squared distance (its bits) of a suitable pixel
-                Mat34 G = sel;
-                if (lane < kSide * kSide) {
-                    const uint32_t column = u - kCorrHalfWindow + lane / kSide, row = y - kCorrHalfWindow + lane % kSide;
-                    const size_t o = (size_t)row * r.W + column;
-                    const float4 pv = r.prev[v][o];
-                    const float* g = r.guided[v] + 12 * o;
-                    if (r.valid[v][o] == 1 && !is_zero_vertex(pv)) {
-                        G.c0 = mk(g[0], g[1], g[2]);
-                        G.c1 = mk(g[3], g[4], g[5]);
-                        G.c2 = mk(g[6], g[7], g[8]);
-                        G.t = mk(g[9], g[10], g[11]);
-                        const f3 d = c - xyz(pv);
-                        const float d2 = dot3(d, d);
-                        const f3 m = G.apply(c) - c;
-                        if (d2 < 1e-4f && dot3(m, m) < 4 * (kNodeRadius * kNodeRadius)) mine = __float_as_uint(d2);
+                // window pixel w is column w / 5, row w % 5
+                auto offset = [&](uint32_t w) {
+                    return (size_t)(y - kCorrHalfWindow + w % kSide) * r.W + (u - kCorrHalfWindow + w / kSide);
+                };
+                auto transform = [&](uint32_t w) {
+                    const float* g = r.guided[v] + 12 * offset(w);
+                    Mat34 G;
+                    G.c0 = mk(g[0], g[1], g[2]);
+                    G.c1 = mk(g[3], g[4], g[5]);
+                    G.c2 = mk(g[6], g[7], g[8]);
+                    G.t = mk(g[9], g[10], g[11]);
+                    return G;
+                };
+                float4 pv[kRounds];
+                uint8_t valid[kRounds];
+#pragma unroll
+                for (uint32_t k = 0; k < kRounds; ++k) {
+                    const uint32_t w = min(lane + kCorrLanes * k, kPixels - 1);
+                    pv[k] = r.prev[v][offset(w)];
+                    valid[k] = lane + kCorrLanes * k < kPixels ? r.valid[v][offset(w)] : 0;
+                }
+                uint32_t best = 0xFFFFFFFFu, at = kPixels;  // squared distance (its bits) and place of a suitable pixel
+#pragma unroll
+                for (uint32_t k = 0; k < kRounds; ++k) {
+                    const f3 d = c - xyz(pv[k]);
+                    const float d2 = dot3(d, d);
+                    if (valid[k] != 1 || is_zero_vertex(pv[k]) || !(d2 < 1e-4f)) continue;
+                    const f3 m = transform(lane + kCorrLanes * k).apply(c) - c;
+                    if (dot3(m, m) < 4 * (kNodeRadius * kNodeRadius) && __float_as_uint(d2) < best) {
+                        best = __float_as_uint(d2);
+                        at = lane + kCorrLanes * k;
                     }
                 }
-                uint32_t best = mine;
 #pragma unroll
-                for (uint32_t s = 1; s < kCorrLanes; s *= 2) best = min(best, (uint32_t)__shfl_xor((int)best, s, 64));
-                if (best != 0xFFFFFFFFu) {
-                    const uint64_t winners = __ballot(mine == best) >> first;
-                    const int from = (int)first + __builtin_ctz((uint32_t)winners);
-                    sel.c0 = mk(__shfl(G.c0.x, from, 64), __shfl(G.c0.y, from, 64), __shfl(G.c0.z, from, 64));
-                    sel.c1 = mk(__shfl(G.c1.x, from, 64), __shfl(G.c1.y, from, 64), __shfl(G.c1.z, from, 64));
-                    sel.c2 = mk(__shfl(G.c2.x, from, 64), __shfl(G.c2.y, from, 64), __shfl(G.c2.z, from, 64));
-                    sel.t = mk(__shfl(G.t.x, from, 64), __shfl(G.t.y, from, 64), __shfl(G.t.z, from, 64));
+                for (uint32_t s = 1; s < kCorrLanes; s *= 2) {
+                    const uint32_t d = (uint32_t)__shfl_xor((int)best, s, 64), w = (uint32_t)__shfl_xor((int)at, s, 64);
+                    const bool take = d < best || (d == best && w < at);
+                    best = take ? d : best;
+                    at = take ? w : at;
                 }
+                if (at < kPixels) sel = transform(at);
                 sel = compose(compose(compose(compose(r.w2c_inv[v], r.init[v]), sel), r.init_inv[v]), r.w2c[v]);
             }
             out = dq_scale(dq_from_mat34(sel), e);
