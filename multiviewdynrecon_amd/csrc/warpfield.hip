@@ -10,13 +10,21 @@
 //               box of its vertices, a lane per box; the nodes of a box pass through
 //               scalar registers (every lane looks at the same node; from LDS the
 //               reads alone took as long as the arithmetic), asked for one box ahead.
-//   nodes     : a wave per node, in the graph and in the skinning; a lane per box and
-//               then per node of the next eight near boxes; the few that beat the
-//               worst slot are inserted one after another.  (A thread per node filled
-//               16 workgroups of 256.)
+//   nodes     : a wave per node where there are few; a lane per box and then per node
+//               of the next eight near boxes; the few that beat the worst slot are
+//               inserted one after another.  (A thread per node filled 16 workgroups
+//               of 256.)  An insertion is the whole wave's then, so more nodes take
+//               eight lanes each, and most a thread each, as the vertices.
 // Bound by the chain of insertions and the arithmetic around it (the memory traffic
-// is 8 MB).  159k surfels and 4018 nodes of the body scene: skinning 441 -> 198 us,
-// graph 791 -> 90 us; surfels in no order, whose boxes exclude nothing, 540 -> 494 us.
+// is 8 MB).  How many there are depends on the order of the nodes; the most are
+// on a line that comes nearer, all of them.  us of a call, a thread per point -> here:
+//   body scene, 159k surfels, 4018 nodes: skinning 431 -> 195, graph 794 -> 89
+//     surfels in no order (their boxes exclude nothing) 533 -> 451, nodes in no order
+//     363 -> 154 and 759 -> 54, both 368 -> 261
+//   281k surfels in no order, 7500 nodes: skinning 1096 -> 1046
+//   20k points in no order and nodes on a line, 600 / 1000 / 2000 / 4000 / 8192 / 65535 nodes:
+//     skinning 87 / 143 / 283 / 559 / 1143 / 9013 -> 86 / 141 / 257 / 507 / 743 / 5964
+//     graph 162 / 272 / 533 / 1065 / 2236 / 17925 -> 66 / 107 / 210 / 492 / 1352 / 12579
 //
 // The warps are streaming passes bound by HBM (a 16-32 B read and write per point plus
 // the L2-resident warp-field gathers).
@@ -40,7 +48,7 @@ namespace {
 constexpr uint32_t kBoxNodes = 8;       // nodes per box
 constexpr uint32_t kBoxes = 512;        // boxes in LDS at a time (4096 nodes, 16 KB)
 constexpr int kGraphNeighbours = 8;     // nodesGraphNeigboursNum
-constexpr uint32_t kGraphWaves = 8;     // nodes per workgroup of the graph search
+constexpr uint32_t kGraphWaves = 8;     // waves per workgroup of the graph search
 
 // Squared distances are compared by their bits: at least +0, they are ordered alike (a
 // not-a-number comes last), and integer minima and maxima need no canonical operands.
@@ -96,8 +104,16 @@ __device__ inline uint32_t wave_max(uint32_t v) {
 // The boxes of nodes [base, base + n), n <= kBoxes * kBoxNodes, by the workgroup.
 struct NodeBoxes {
     float4 lo[kBoxes], hi[kBoxes];
+    __device__ void put(uint32_t, float4) {}
 };
-__device__ inline uint32_t build_boxes(const float4* __restrict__ nodes, uint32_t base, uint32_t n, NodeBoxes& x) {
+// The same of kTileNodes nodes at a time, and the nodes.
+constexpr uint32_t kTileNodes = 1024;
+struct NodeTile {
+    float4 lo[kTileNodes / kBoxNodes], hi[kTileNodes / kBoxNodes], node[kTileNodes];
+    __device__ void put(uint32_t k, float4 q) { node[k] = q; }
+};
+template <class Boxes>
+__device__ inline uint32_t build_boxes(const float4* __restrict__ nodes, uint32_t base, uint32_t n, Boxes& x) {
     const uint32_t boxes = (n + kBoxNodes - 1) / kBoxNodes;
     __syncthreads();
     for (uint32_t t = threadIdx.x; t < 2 * boxes; t += blockDim.x) {  // two lanes per box, four nodes each
@@ -105,6 +121,7 @@ __device__ inline uint32_t build_boxes(const float4* __restrict__ nodes, uint32_
 #pragma unroll
         for (uint32_t j = 0; j < kBoxNodes / 2; ++j) {
             const float4 q = nodes[base + min(t * (kBoxNodes / 2) + j, n - 1)];  // the last node repeats past the end
+            x.put(t * (kBoxNodes / 2) + j, q);
             l = j == 0 ? q : make_float4(fminf(l.x, q.x), fminf(l.y, q.y), fminf(l.z, q.z), 0.f);
             h = j == 0 ? q : make_float4(fmaxf(h.x, q.x), fmaxf(h.y, q.y), fmaxf(h.z, q.z), 0.f);
         }
@@ -202,6 +219,71 @@ __device__ inline void scan_for_point(const float4* __restrict__ nodes, uint32_t
     }
 }
 
+// The value of lane j of each eight lanes, in all of them.
+template <uint32_t j>
+__device__ inline float eight_lane(float v) {
+    const float own = dpp<(j % 4) * 0x55>(v), other = dpp<0x141>(own);  // of the lane's four, of the other four
+    return (threadIdx.x & 4) == (j & 4) ? own : other;
+}
+// The lane's eight lanes of a ballot.
+__device__ inline uint32_t eight_bits(bool p) { return (uint32_t)(__ballot(p) >> (threadIdx.x & 56)) & 0xFFu; }
+
+// Passes the nodes that may enter the slots of eight points, one to each eight lanes
+// (`me`), in index order: a lane per box, then per node of the point's next near box.
+//   slots.bound()             the farthest slot
+//   slots.distance(me, q)     slots.wants(d): whether a distance may be inserted
+//   slots.insert(k, d)        node k at distance d, where wanted; equal in the eight lanes
+template <class Slots>
+__device__ inline void scan_for_eight(const float4* __restrict__ nodes, uint32_t num_nodes, float4 me, NodeTile& tile,
+                                      Slots& slots) {
+    const uint32_t sub = threadIdx.x % kBoxNodes;
+    const float inf = __int_as_float(0x7f800000);
+    for (uint32_t base = 0; base < num_nodes; base += kTileNodes) {
+        const uint32_t n = min(kTileNodes, num_nodes - base), boxes = build_boxes(nodes, base, n, tile);
+        float4 lo = tile.lo[min(sub, boxes - 1)], hi = tile.hi[min(sub, boxes - 1)];
+        for (uint32_t b0 = 0; b0 < boxes; b0 += kBoxNodes) {
+            const float away = box_distance(me, me, lo, hi);
+            uint32_t near = eight_bits(b0 + sub < boxes && may_be_nearer(away, slots.bound()));
+            const uint32_t mine = min(b0 + kBoxNodes + sub, boxes - 1);  // the next step's box loads meanwhile
+            lo = tile.lo[mine];
+            hi = tile.hi[mine];
+            while (__any(near != 0)) {
+                // two boxes at a time
+                uint32_t k[2];
+                float d[2];
+#pragma unroll
+                for (uint32_t p = 0; p < 2; ++p) {
+                    k[p] = (b0 + (near ? (uint32_t)__builtin_ctz(near) : 0u)) * kBoxNodes;
+                    const float4 q = tile.node[k[p] + sub];
+                    d[p] = near != 0 && k[p] + sub < n ? slots.distance(me, q) : inf;
+                    near &= near - 1;
+                }
+                bool any = false;
+#pragma unroll
+                for (uint32_t p = 0; p < 2; ++p) {
+                    uint64_t hits = __ballot(slots.wants(d[p]));
+                    if (!hits) continue;
+                    any = true;
+                    hits |= hits >> 32;
+                    hits |= hits >> 16;
+                    hits |= hits >> 8;
+                    const uint32_t first = base + k[p];
+                    if (hits & 1) slots.insert(first, eight_lane<0>(d[p]));
+                    if (hits & 2) slots.insert(first + 1, eight_lane<1>(d[p]));
+                    if (hits & 4) slots.insert(first + 2, eight_lane<2>(d[p]));
+                    if (hits & 8) slots.insert(first + 3, eight_lane<3>(d[p]));
+                    if (hits & 16) slots.insert(first + 4, eight_lane<4>(d[p]));
+                    if (hits & 32) slots.insert(first + 5, eight_lane<5>(d[p]));
+                    if (hits & 64) slots.insert(first + 6, eight_lane<6>(d[p]));
+                    if (hits & 128) slots.insert(first + 7, eight_lane<7>(d[p]));
+                }
+                // a box passed over is no nearer than the farthest slot, which only gets nearer
+                if (any) near &= eight_bits(may_be_nearer(away, slots.bound()));
+            }
+        }
+    }
+}
+
 struct SkinSlots {
     uint32_t d[4], id[4] = {0, 0, 0, 0};
     __device__ SkinSlots() { d[0] = d[1] = d[2] = d[3] = bits(1e6f); }
@@ -242,30 +324,54 @@ __device__ inline void put_skin(float4 pt, const SkinSlots& slots, const float4*
 
 constexpr uint32_t kSkinWaves = 4;  // waves per workgroup of the skinning
 
-// The first workgroups skin 256 vertices each, the others a node per wave.  (64 nodes
-// in a row lie too far apart for boxes common to them.)  All waves are resident at
-// once, a few per SIMD, and the longest of them set the time: vertices before nodes
-// (198 us; nodes first 226) and four waves a workgroup (eight of them 219 nodes first,
-// one 202) spread them best.
+// Lanes of a node in the skinning.  64 nodes in a row lie too far apart for boxes common
+// to them, so lanes of its own serve a node better, until the insertions of all nodes
+// fill the chip: a wave up to kSkinWaveNodes, eight lanes up to kSkinEightNodes, a
+// thread above (us; the listed order / a line that comes nearer, as above):
+//   600 nodes  wave  40 /   86, eight  44 /   81, thread  54 /  60
+//   2000       wave 103 /  327, eight 109 /  257, thread 121 / 183
+//   4000       wave 190 /  891, eight 195 /  507, thread 194 / 361
+//   7500, 8192 wave 327 / 2917, eight 337 / 1082, thread 336 / 743
+// A line's insertions by waves pass a thread per node (start of the file) at ~1000 nodes,
+// by eight lanes at ~8000.
+constexpr uint32_t kNodeWave = 64, kNodeEight = kBoxNodes, kNodeThread = 1;
+constexpr uint32_t kSkinWaveNodes = 1024, kSkinEightNodes = 6144;
+
+// Workgroups of 256 vertices, then of nodes with lanes of their own; nodes by threads
+// come first, as the longest waves (4018 nodes 202 us, last 216).
+template <uint32_t kNodeLanes>
 __global__ void __launch_bounds__(64 * kSkinWaves)
-    skin_kernel(const float4* __restrict__ vertices, uint32_t num_vertices, const float4* __restrict__ nodes,
-                uint32_t num_nodes, float radius, ushort4* __restrict__ vknn, float4* __restrict__ vw,
-                ushort4* __restrict__ nknn, float4* __restrict__ nw) {
-    __shared__ NodeBoxes box;
+    skin_kernel(const float4* vertices, uint32_t num_vertices, const float4* nodes, uint32_t num_nodes, float radius,
+                ushort4* vknn, float4* vw, ushort4* nknn, float4* nw) {
+    __shared__ union {
+        NodeBoxes box;
+        NodeTile tile;
+    } shared;
+    NodeBoxes& box = shared.box;
     SkinSlots slots;
     const uint32_t vertex_blocks = (num_vertices + blockDim.x - 1) / blockDim.x, lane = threadIdx.x & 63;
-    if (blockIdx.x >= vertex_blocks) {
-        const uint32_t i = (blockIdx.x - vertex_blocks) * kSkinWaves + (threadIdx.x >> 6);
+    const uint32_t node_blocks = gridDim.x - vertex_blocks;
+    const bool is_node = kNodeLanes == kNodeThread ? blockIdx.x < node_blocks : blockIdx.x >= vertex_blocks;
+    uint32_t block = blockIdx.x;
+    if (is_node != (kNodeLanes == kNodeThread)) block -= is_node ? vertex_blocks : node_blocks;
+    if (kNodeLanes != kNodeThread && is_node) {
+        const uint32_t i = (block * blockDim.x + threadIdx.x) / kNodeLanes;
         const float4 me = nodes[min(i, num_nodes - 1)];
-        scan_for_point(nodes, num_nodes, me, box, slots);
-        if (i < num_nodes && lane == 0) put_skin(me, slots, nodes, radius, nknn + i, nw + i);
+        if constexpr (kNodeLanes == kNodeWave) scan_for_point(nodes, num_nodes, me, box, slots);
+        else scan_for_eight(nodes, num_nodes, me, shared.tile, slots);
+        if (i < num_nodes && threadIdx.x % kNodeLanes == 0) put_skin(me, slots, nodes, radius, nknn + i, nw + i);
         return;
     }
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (is_node) {  // as the vertices are
+        vertices = nodes;
+        num_vertices = num_nodes;
+        vknn = nknn;
+        vw = nw;
+    }
+    const uint32_t p = block * blockDim.x + threadIdx.x;
     const float4 pt = vertices[min(p, num_vertices - 1)];  // idle lanes repeat the last vertex
     const float4 whi = make_float4(wave_max(pt.x), wave_max(pt.y), wave_max(pt.z), 0.f);
     const float4 wlo = make_float4(-wave_max(-pt.x), -wave_max(-pt.y), -wave_max(-pt.z), 0.f);
-    float worst = 1e6f;  // the farthest fourth neighbour of the wave's points
     for (uint32_t base = 0; base < num_nodes; base += kBoxes * kBoxNodes) {
         const uint32_t n = min(kBoxes * kBoxNodes, num_nodes - base);
         build_boxes(nodes, base, n, box);
@@ -274,8 +380,10 @@ __global__ void __launch_bounds__(64 * kSkinWaves)
             const uint32_t mine = min(b0 + lane, whole - 1);
             const float coarse = box_distance(wlo, whi, box.lo[mine], box.hi[mine]);
             uint64_t left = b0 + 64 <= whole ? ~0ull : (1ull << (whole - b0)) - 1;  // boxes not yet passed
+            float worst = __uint_as_float(wave_max(slots.d[0]));  // the farthest fourth neighbour of the wave's points
             uint64_t near = left & __ballot(may_be_nearer(coarse, worst));
             if (!near) continue;
+            uint32_t vain = 0;  // last looks at the boxes that excluded none
             const float4* first = nodes + base + b0 * kBoxNodes;
             uint32_t x = (uint32_t)__builtin_ctzll(near);
             NodeGroup here, next;
@@ -286,9 +394,12 @@ __global__ void __launch_bounds__(64 * kSkinWaves)
                 near &= left;
                 const uint32_t y = near ? (uint32_t)__builtin_ctzll(near) : x;
                 next.load(first, y * kBoxNodes);
-                if (slots.pass(pt, here, base + (b0 + x) * kBoxNodes)) {
+                if (slots.pass(pt, here, base + (b0 + x) * kBoxNodes) && vain < 4) {
+                    // looked at again while that excludes boxes (points in no order: 1125 -> 1047 us)
                     worst = __uint_as_float(wave_max(slots.d[0]));
-                    near = left & __ballot(may_be_nearer(coarse, worst));
+                    const uint64_t again = near & __ballot(may_be_nearer(coarse, worst));
+                    vain = again == near ? vain + 1 : 0;
+                    near = again;
                 }
                 if (y == x) break;
                 x = y;
@@ -300,10 +411,11 @@ __global__ void __launch_bounds__(64 * kSkinWaves)
     if (p < num_vertices) put_skin(pt, slots, nodes, radius, vknn + p, vw + p);
 }
 
-// BuildNodesGraphKernel: 8 slots, the worst replaced (WarpField.cu:15-59).  Lane
-// j < 8 holds slot j.
+// BuildNodesGraphKernel: 8 slots, the worst replaced (WarpField.cu:15-59).  Lane j
+// of the node's holds slot j: of its wave (kWave, lanes 8 on hold none) or of its eight.
+template <bool kWave>
 struct GraphSlots {
-    float dist = (threadIdx.x & 63) < kGraphNeighbours ? 1e5f : 0.f;
+    float dist = !kWave || (threadIdx.x & 63) < kGraphNeighbours ? 1e5f : 0.f;
     int idx = -1;
     float worst_d = 1e5f;
     uint32_t worst = 0;
@@ -313,22 +425,36 @@ struct GraphSlots {
     }
     __device__ bool wants(float d) const { return d > 1e-6f && d < worst_d; }
     __device__ void insert(uint32_t k, float d) {
-        if ((threadIdx.x & 63) == worst) {
+        if ((kWave || wants(d)) && (threadIdx.x & (kWave ? 63 : 7)) == worst) {
             dist = d;
             idx = (int)k;
         }
-        // the new worst slot: the first of the largest 
-        worst_d = __int_as_float(__builtin_amdgcn_readfirstlane((int)eight_max(bits(dist))));
-        worst = (uint32_t)__builtin_ctzll(__ballot(dist == worst_d));
+        // the new worst slot: the first of the largest
+        const uint32_t m = eight_max(bits(dist));
+        worst_d = __uint_as_float(kWave ? (uint32_t)__builtin_amdgcn_readfirstlane((int)m) : m);
+        worst = kWave ? (uint32_t)__builtin_ctzll(__ballot(dist == worst_d)) : (uint32_t)__builtin_ctz(eight_bits(dist == worst_d));
     }
 };
+static_assert(kGraphNeighbours == (int)kBoxNodes, "a lane per slot and per node of a box");
+
+// A wave per node up to kGraphWaveNodes, eight lanes above (us; random order / a line that
+// comes nearer): 4000 nodes 57 / 492 and 137 / 447, 8192 165 / 1352 and 240 / 918,
+// 12000 316 / 2495 and 328 / 1341, 20000 781 / 5974 and 588 / 2398.
+constexpr uint32_t kGraphWaveNodes = 12288;
+template <bool kWave>
 __global__ void __launch_bounds__(64 * kGraphWaves)
     node_graph_kernel(const float4* __restrict__ nodes, uint32_t num_nodes, ushort2* __restrict__ graph) {
-    __shared__ NodeBoxes box;
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t i = blockIdx.x * kGraphWaves + (threadIdx.x >> 6);
-    GraphSlots slots;
-    scan_for_point(nodes, num_nodes, nodes[min(i, num_nodes - 1)], box, slots);
+    constexpr uint32_t kLanes = kWave ? 64 : kBoxNodes;
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / kLanes, lane = threadIdx.x % kLanes;
+    const float4 me = nodes[min(i, num_nodes - 1)];
+    GraphSlots<kWave> slots;
+    if constexpr (kWave) {
+        __shared__ NodeBoxes box;
+        scan_for_point(nodes, num_nodes, me, box, slots);
+    } else {
+        __shared__ NodeTile tile;
+        scan_for_eight(nodes, num_nodes, me, tile, slots);
+    }
     if (i < num_nodes && lane < (uint32_t)kGraphNeighbours)
         graph[(size_t)i * kGraphNeighbours + lane] = make_ushort2((uint16_t)i, (uint16_t)slots.idx);
 }
@@ -594,9 +720,13 @@ mvdr_status mvdr_warp_build_node_graph(const void* nodes, uint32_t num_nodes, vo
     if (num_nodes == 0) return MVDR_OK;
     if (!nodes || !graph) return MVDR_E_INVALID;
     if (num_nodes > 65535) return MVDR_E_SHAPE;
-    hipLaunchKernelGGL(node_graph_kernel, dim3((num_nodes + kGraphWaves - 1) / kGraphWaves), dim3(64 * kGraphWaves), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const float4*>(nodes), num_nodes,
-                       static_cast<ushort2*>(graph));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const float4* n = static_cast<const float4*>(nodes);
+    ushort2* g = static_cast<ushort2*>(graph);
+    const uint32_t per = num_nodes <= kGraphWaveNodes ? kGraphWaves : 64 * kGraphWaves / kBoxNodes;  // nodes per workgroup
+    const dim3 grid((num_nodes + per - 1) / per), wg(64 * kGraphWaves);
+    if (num_nodes <= kGraphWaveNodes) hipLaunchKernelGGL(node_graph_kernel<true>, grid, wg, 0, st, n, num_nodes, g);
+    else hipLaunchKernelGGL(node_graph_kernel<false>, grid, wg, 0, st, n, num_nodes, g);
     return hipGetLastError() == hipSuccess ? MVDR_OK : MVDR_E_HIP;
 }
 
@@ -609,8 +739,11 @@ mvdr_status mvdr_warp_skin(const void* vertices, uint32_t num_vertices, const vo
     const uint64_t total = (uint64_t)num_vertices + num_nodes;
     if (total > 0xFFFFFFFFull - 255) return MVDR_E_SHAPE;
     constexpr uint32_t kSkinThreads = 64 * kSkinWaves;
-    const uint32_t blocks = (num_vertices + kSkinThreads - 1) / kSkinThreads + (num_nodes + kSkinWaves - 1) / kSkinWaves;
-    hipLaunchKernelGGL(skin_kernel, dim3(blocks), dim3(kSkinThreads), 0, static_cast<hipStream_t>(stream),
+    const uint32_t lanes = num_nodes <= kSkinWaveNodes ? kNodeWave : num_nodes <= kSkinEightNodes ? kNodeEight : kNodeThread;
+    const uint32_t per = kSkinThreads / lanes;  // nodes per workgroup
+    const dim3 grid((num_vertices + kSkinThreads - 1) / kSkinThreads + (num_nodes + per - 1) / per);
+    auto* kernel = lanes == kNodeWave ? skin_kernel<kNodeWave> : lanes == kNodeEight ? skin_kernel<kNodeEight> : skin_kernel<kNodeThread>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kSkinThreads), 0, static_cast<hipStream_t>(stream),
                        static_cast<const float4*>(vertices), num_vertices, static_cast<const float4*>(nodes), num_nodes,
                        node_radius, static_cast<ushort4*>(vknn), static_cast<float4*>(vw), static_cast<ushort4*>(nknn),
                        static_cast<float4*>(nw));
