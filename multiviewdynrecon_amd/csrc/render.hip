@@ -8,7 +8,9 @@
 // 64 B of surfel attributes read per surfel, 8 B atomic per drawn surfel,
 // ~88 B written per pixel).  A workgroup draws one view (grid.y), whose camera and
 // addresses are scalars then.  159k surfels into three 640 x 480 views: clear 4 us, splat
-// 15.5 (the atomics: looking before them takes 17.6), resolve 19.3 (20.8 with plain stores).
+// 15.5 (the atomics: looking before them takes 17.6), resolve 20.8 (19.3 with streaming
+// stores, but the solve that reads the maps then finds none of them in a cache: maps and a
+// solve of 2k / 7.5k nodes 241 and 312 us, with streaming stores 244 and 315).
 #pragma clang fp contract(off)
 
 #include <hip/hip_runtime.h>
@@ -71,12 +73,6 @@ __device__ inline float4 decode_rgb(float4 ct) {
                        (float)(c & 0x000000FF) / 255.f, ct.y);
 }
 
-// The maps are 77 MB, no cache keeps them: streaming stores.
-__device__ inline void stream(float4* p, float4 v) {
-    typedef float vec4 __attribute__((ext_vector_type(4)));
-    __builtin_nontemporal_store(vec4{v.x, v.y, v.z, v.w}, reinterpret_cast<vec4*>(p));
-}
-
 __global__ void __launch_bounds__(256) resolve_kernel(RenderViews r, RenderMaps m) {
     const uint32_t pixels = r.W * r.H, v = blockIdx.y;
     for (uint32_t o = blockIdx.x * blockDim.x + threadIdx.x; o < pixels; o += gridDim.x * blockDim.x) {
@@ -93,12 +89,12 @@ __global__ void __launch_bounds__(256) resolve_kernel(RenderViews r, RenderMaps 
             wn = make_float4(d.x, d.y, d.z, 0.f);
             rgb = decode_rgb(r.color_time[idx]);
         }
-        stream(m.ref_v[v] + o, rv);
-        stream(m.ref_n[v] + o, rn);
-        stream(m.warp_v[v] + o, wv);
-        if (m.warp_n[v]) stream(m.warp_n[v] + o, wn);
-        __builtin_nontemporal_store(idx, m.index[v] + o);
-        if (m.rgb[v]) stream(m.rgb[v] + o, rgb);
+        m.ref_v[v][o] = rv;
+        m.ref_n[v][o] = rn;
+        m.warp_v[v][o] = wv;
+        if (m.warp_n[v]) m.warp_n[v][o] = wn;
+        m.index[v][o] = idx;
+        if (m.rgb[v]) m.rgb[v][o] = rgb;
     }
 }
 
