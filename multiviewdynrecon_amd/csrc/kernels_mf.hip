@@ -1190,10 +1190,21 @@ static void apply_fp32(const Batch& B, bool recompute, int src_epi, uint32_t k, 
 }
 
 // ------------------------------------------------ mixed mode
+// Workgroups of a term launch over all frames, six to a CU, shared by the frames of a
+// batch: a workgroup forms the iteration's scalars from all partials before its terms,
+// and a frame's 160k terms fill a few hundred of them.  A lone frame takes
+// 1024 (a term or two a thread: 300 nodes 1090 us a solve, 75 workgroups 1143).  Batches
+// with 1024 a frame, and with their share (stored / recomputed J, ms a solve, two
+// 320x240 views, 3 GN x 10 PCG): 32 frames of 600 nodes 5.12 / 6.28 and 4.15 / 4.79, 16 of
+// 2000 3.44 / 4.06 and 2.95 / 3.41, 4 of 8000 2.36 / 2.59 and 2.19 / 2.28.
+constexpr uint32_t kTermWorkgroups = 6 * 256;
+static uint32_t mixed_term_grid(const Batch& B) {
+    return std::max<uint32_t>(64, std::min<uint32_t>(1024, kTermWorkgroups / B.frames));
+}
 template <int kSrc, int kEpi>
 static void apply_mixed(const Batch& B, bool recompute, uint32_t k, const Penalty& pen, uint32_t which,
                         hipStream_t stream) {
-    const dim3 tg(std::max<uint32_t>(term_grid(B), 1024), B.frames), gg(gather_grid(B), B.frames), wg(256), ww(64 * kMfWaves);
+    const dim3 tg(mixed_term_grid(B), B.frames), gg(gather_grid(B), B.frames), wg(256), ww(64 * kMfWaves);
     if (recompute) {
         hipLaunchKernelGGL((mf_apply_terms_kernel<true, kSrc, kOutG>), tg, wg, 0, stream, B.dev, k, pen, which);
         hipLaunchKernelGGL((mf_apply_gather_kernel<true, kEpi>), gg, ww, 0, stream, B.dev, k, pen);
