@@ -32,3 +32,15 @@ def test_first_call_on_a_stream_beside_a_busy_null_stream():
     h.FindCrossViewEdgeMatchedPairs(stream=side.cuda_stream)
     side.synchronize()
     assert lists(h) == want
+
+
+def test_dense_frame_then_sparse_smaller_one():
+    """Lists, flags, candidates and tile counts of a frame leave nothing for the next."""
+    cfg = default_config(max_width=64, max_height=64, search_radius=4, search_step=1)
+    h = CrossViewEdgeCorrespondence(cfg)
+    for cv in (frame(1, 3, 64, 64, None), frame(2, 2, 37, 29, 60), frame(3, 3, 64, 64, 0), frame(4, 3, 50, 64, 700),
+               frame(5, 1, 64, 64, 300), frame(2, 2, 37, 29, 60)):
+        ci, keep = crossview_input(cv, device="cuda")
+        h.SetCrossViewMatchingInput(ci)
+        h.FindCrossViewEdgeMatchedPairs()
+        assert lists(h) == oracle_lists(cv, cfg)
