@@ -107,6 +107,18 @@ __device__ inline T wave_sum(T v) {
     return lanes_sum<64>(v);
 }
 
+// One step of a reduce-scatter of 2 kHalf values over a wave: the lane keeps the half
+// that its lane bit names and adds the other lane's copies of it.
+template <int kHalf, int kValues>
+__device__ inline void reduce_half(double (&v)[kValues]) {
+    const bool upper = (threadIdx.x & kHalf) != 0;
+#pragma unroll
+    for (int k = 0; k < kHalf; ++k) {
+        const double keep = upper ? v[k + kHalf] : v[k], send = upper ? v[k] : v[k + kHalf];
+        v[k] = keep + lane_xor<kHalf>(send);
+    }
+}
+
 template <typename T>
 __device__ inline T wave_max(T v) {
 #pragma unroll

@@ -50,16 +50,16 @@ __device__ inline MfLambda2 mf_lambda2(const Penalty& p) {
 // Term pass: u_t for every term.  kSrcDir forms the PCG direction
 // d = s + beta d_prev (beta from the previous launches' partials) on the fly
 // and stores it for the gather and the update.
-template <typename Acc, int kSrc>
+template <int kSrc>
 __global__ void __launch_bounds__(256) mf_terms_kernel(const Buffers* __restrict__ bs, uint32_t k, uint32_t cur, Penalty pen) {
     const Buffers b = frame_buffers(bs);
     const FrameDev& f = *b.frame;
     const Counts& c = *b.counts;
-    Acc beta = 0;
+    float beta = 0;
     if (kSrc == kSrcDir && k > 0) {
-        Acc num, den;
-        reduce_partials2<Acc>(slot_ptr(b, kSlotDelta + k), kVecBlocks, slot_ptr(b, kSlotDelta + k - 1), kVecBlocks, num, den);
-        beta = den != (Acc)0 ? num / den : (Acc)0;
+        float num, den;
+        reduce_partials2<float>(slot_ptr(b, kSlotDelta + k), kVecBlocks, slot_ptr(b, kSlotDelta + k - 1), kVecBlocks, num, den);
+        beta = den != (float)0 ? num / den : (float)0;
     }
     if (c.error) return;
     const float* __restrict__ prev = cur ? b.d1 : b.d0;
@@ -70,7 +70,7 @@ __global__ void __launch_bounds__(256) mf_terms_kernel(const Buffers* __restrict
         for (int a = 0; a < 6; ++a) {
             if (kSrc == kSrcDir) {
                 const float p = prev[6 * n + a];
-                v[a] = k > 0 ? (float)((Acc)b.s[6 * n + a] + beta * (Acc)p) : p;
+                v[a] = k > 0 ? (float)((float)b.s[6 * n + a] + beta * (float)p) : p;
             } else {
                 v[a] = vec[6 * n + a];
             }
@@ -157,14 +157,14 @@ __global__ void __launch_bounds__(256) mf_terms_kernel(const Buffers* __restrict
 
 // Gather pass: y_i over the Node2Term list of row i (kRowLanes lanes per row),
 // then the epilogue of the PCG step it serves.
-template <typename Acc, int kEpi>
+template <int kEpi>
 __global__ void __launch_bounds__(256) mf_gather_kernel(const Buffers* __restrict__ bs, uint32_t k, uint32_t cur, Penalty pen) {
     const Buffers b = frame_buffers(bs);
     const FrameDev& f = *b.frame;
     const Counts& c = *b.counts;
     const uint32_t sub = threadIdx.x % kRowLanes;
     const float* __restrict__ vec = kEpi == kEpiSpmv ? (cur ? b.d0 : b.d1) : (kEpi == kEpiResidual ? b.x : b.d1);
-    Acc acc = 0;
+    float acc = 0;
     if (!c.error) {
         const TermBounds tb(c);
         const MfLambda2 l2 = mf_lambda2(pen);
@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(256) mf_gather_kernel(const Buffers* __restric
         const uint32_t groups = gridDim.x * kRowsPerBlock;
         for (uint32_t base = blockIdx.x * kRowsPerBlock; base < f.N; base += groups) {
             const uint32_t i = base + threadIdx.x / kRowLanes;
-            Acc y[6] = {0, 0, 0, 0, 0, 0};
+            float y[6] = {0, 0, 0, 0, 0, 0};
             float vi[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             if (i < f.N) {
                 const float4 g = f.nodes[i];
@@ -232,7 +232,7 @@ __global__ void __launch_bounds__(256) mf_gather_kernel(const Buffers* __restric
                             float s = wi * u[r];
                             if (mult > 1) s -= (float)(mult - 1) * lam[r] * wi * wi * dot6(J[r], vi);
 #pragma unroll
-                            for (int a = 0; a < 6; ++a) y[a] += (Acc)(s * J[r][a]);
+                            for (int a = 0; a < 6; ++a) y[a] += (float)(s * J[r][a]);
                         }
                     }
                 }
@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(256) mf_gather_kernel(const Buffers* __restric
                                 bz = tv[3] * g.y - tv[4] * g.x;
                     const float damp[6] = {tv[0] + bx, tv[1] + by, tv[2] + bz, tv[3], tv[4], tv[5]};
 #pragma unroll
-                    for (int a = 0; a < 6; ++a) y[a] += (Acc)(1e-2f * damp[a]);
+                    for (int a = 0; a < 6; ++a) y[a] += (float)(1e-2f * damp[a]);
                 }
             }
 #pragma unroll
@@ -254,29 +254,29 @@ __global__ void __launch_bounds__(256) mf_gather_kernel(const Buffers* __restric
 #pragma unroll
                     for (int a = 0; a < 6; ++a) {
                         b.q[6 * i + a] = (float)y[a];
-                        acc += (Acc)vi[a] * y[a];
+                        acc += (float)vi[a] * y[a];
                     }
                 } else if (kEpi == kEpiResidual) {
                     float rr[6], z[6];
 #pragma unroll
                     for (int a = 0; a < 6; ++a) {
-                        rr[a] = (float)((Acc)b.jtr[6 * i + a] - y[a]);
+                        rr[a] = (float)((float)b.jtr[6 * i + a] - y[a]);
                         b.r[6 * i + a] = rr[a];
                     }
-                    apply_minv<Acc>(b, i, rr, z);
+                    apply_minv<float>(b, i, rr, z);
 #pragma unroll
                     for (int a = 0; a < 6; ++a) {
                         b.d1[6 * i + a] = z[a];
-                        acc += (Acc)rr[a] * (Acc)z[a];
+                        acc += (float)rr[a] * (float)z[a];
                     }
                 } else {
 #pragma unroll
-                    for (int a = 0; a < 6; ++a) acc += (Acc)vi[a] * y[a];
+                    for (int a = 0; a < 6; ++a) acc += (float)vi[a] * y[a];
                 }
             }
         }
     }
-    write_partial<Acc>(b, kEpi == kEpiSpmv ? kSlotDQ + k : (kEpi == kEpiResidual ? kSlotRefNum : kSlotRefDen), acc);
+    write_partial<float>(b, kEpi == kEpiSpmv ? kSlotDQ + k : (kEpi == kEpiResidual ? kSlotRefNum : kSlotRefDen), acc);
 }
 
 // ------------------------------------------ matrix-free apply, J recomputed
@@ -379,18 +379,18 @@ __global__ void __launch_bounds__(256) mf_entry_weights_kernel(const Buffers* __
     }
 }
 
-template <typename Acc, typename R, int kSrc, int kOut>
+template <int kSrc, int kOut>
 __global__ void __launch_bounds__(256) mfr_terms_kernel(const Buffers* __restrict__ bs, uint32_t k, uint32_t cur, Penalty pen,
                                                         uint32_t which) {
     const Buffers b = frame_buffers(bs);
     const FrameDev& f = *b.frame;
     const Counts& c = *b.counts;
     const DQ* __restrict__ se3 = which ? b.se3[1] : b.se3[0];
-    Acc beta = 0;
+    float beta = 0;
     if (kSrc == kSrcDir && k > 0) {
-        Acc num, den;
-        reduce_partials2<Acc>(slot_ptr(b, kSlotDelta + k), kVecBlocks, slot_ptr(b, kSlotDelta + k - 1), kVecBlocks, num, den);
-        beta = den != (Acc)0 ? num / den : (Acc)0;
+        float num, den;
+        reduce_partials2<float>(slot_ptr(b, kSlotDelta + k), kVecBlocks, slot_ptr(b, kSlotDelta + k - 1), kVecBlocks, num, den);
+        beta = den != (float)0 ? num / den : (float)0;
     }
     if (c.error) return;
     const float* __restrict__ prev = cur ? b.d1 : b.d0;
@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(256) mfr_terms_kernel(const Buffers* __restric
         for (int a = 0; a < 6; ++a) {
             if (kSrc == kSrcDir) {
                 const float p = prev[6 * n + a];
-                v[a] = k > 0 ? (float)((Acc)b.s[6 * n + a] + beta * (Acc)p) : p;
+                v[a] = k > 0 ? (float)((float)b.s[6 * n + a] + beta * (float)p) : p;
             } else {
                 v[a] = vec[6 * n + a];
             }
@@ -425,7 +425,7 @@ __global__ void __launch_bounds__(256) mfr_terms_kernel(const Buffers* __restric
         }
         if (type == kSmooth) {
             if (kSrc != kSrcRows) {
-                const SmoothRec sm = eval_smooth<R>(f, se3, kk);
+                const SmoothRec sm = eval_smooth<float>(f, se3, kk);
                 const uint32_t n1 = sm.ij & 0xFFFF, n2 = sm.ij >> 16;
                 float J1[3][6], J2[3][6], res[3], v[6], w1[6], w2[6];
                 smooth_rows(sm, true, J1, res);
@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(256) mfr_terms_kernel(const Buffers* __restric
             for (int r = 0; r < 3; ++r) g[r] = l * u[r];
         } else {
             float J[3][6], lam[3];
-            const int rows = knn_term_rows<R>(b, f, se3, type, kk, l2, density, J, lam);
+            const int rows = knn_term_rows<float>(b, f, se3, type, kk, l2, density, J, lam);
             if (kSrc != kSrcRows) {
                 ushort4 knn;
                 float4 wk;
@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(256) mfr_terms_kernel(const Buffers* __restric
     }
 }
 
-template <typename Acc, typename R, int kEpi>
+template <int kEpi>
 __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restrict__ bs, uint32_t k, uint32_t cur, Penalty pen,
                                                          uint32_t which) {
     const Buffers b = frame_buffers(bs);
@@ -497,7 +497,7 @@ __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restri
     const uint32_t sub = threadIdx.x % kRowLanes;
     const float* __restrict__ vec = kEpi == kEpiSpmv ? (cur ? b.d0 : b.d1) : (kEpi == kEpiResidual ? b.x : b.d1);
     constexpr bool correct = kEpi != kEpiAdjoint;
-    Acc acc = 0;
+    float acc = 0;
     if (!c.error) {
         const TermBounds tb(c);
         const MfLambda2 l2 = mf_lambda2(pen);
@@ -505,7 +505,7 @@ __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restri
         const uint32_t groups = gridDim.x * kRowsPerBlock;
         for (uint32_t base = blockIdx.x * kRowsPerBlock; base < f.N; base += groups) {
             const uint32_t i = base + threadIdx.x / kRowLanes;
-            Acc y[6] = {0, 0, 0, 0, 0, 0};   // reference coordinates until the row is complete
+            float y[6] = {0, 0, 0, 0, 0, 0};   // reference coordinates until the row is complete
             float vi[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             float4 gi = make_float4(0.f, 0.f, 0.f, 0.f);
             if (i < f.N) {
@@ -523,7 +523,7 @@ __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restri
                     const int type = type_of(tb, t, kk);
                     const float4 g0 = b.mf_g[2 * (size_t)t];
                     if (type == kSmooth) {
-                        const SmoothRec sm = eval_smooth<R>(f, se3, kk);
+                        const SmoothRec sm = eval_smooth<float>(f, se3, kk);
                         const uint32_t n1 = sm.ij & 0xFFFF, n2 = sm.ij >> 16;
                         float J[3][6], res[3];
                         smooth_rows(sm, i == n1, J, res);
@@ -534,7 +534,7 @@ __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restri
                             float s = u[r];
                             if (correct && mult > 1) s -= (float)(mult - 1) * l2.smooth * dot6(J[r], tvi);
 #pragma unroll
-                            for (int a = 0; a < 6; ++a) y[a] += (Acc)(s * J[r][a]);
+                            for (int a = 0; a < 6; ++a) y[a] += (float)(s * J[r][a]);
                         }
                     } else {
                         const float4 g1 = b.mf_g[2 * (size_t)t + 1];
@@ -542,18 +542,18 @@ __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restri
                         const float wi = fabsf(ws);
                         const float gv[6] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y};
 #pragma unroll
-                        for (int a = 0; a < 6; ++a) y[a] += (Acc)(wi * gv[a]);
+                        for (int a = 0; a < 6; ++a) y[a] += (float)(wi * gv[a]);
                         if (correct && signbit(ws)) {
                             ushort4 knn;
                             float4 wk;
                             term_knn(b, type, kk, knn, wk);
                             const uint32_t mult = (knn.x == i) + (knn.y == i) + (knn.z == i) + (knn.w == i);
                             float J[3][6], lam[3];
-                            const int rows = knn_term_rows<R>(b, f, se3, type, kk, l2, density, J, lam);
+                            const int rows = knn_term_rows<float>(b, f, se3, type, kk, l2, density, J, lam);
                             for (int r = 0; r < rows; ++r) {
                                 const float s = -(float)(mult - 1) * lam[r] * wi * wi * dot6(J[r], tvi);
 #pragma unroll
-                                for (int a = 0; a < 6; ++a) y[a] += (Acc)(s * J[r][a]);
+                                for (int a = 0; a < 6; ++a) y[a] += (float)(s * J[r][a]);
                             }
                         }
                     }
@@ -563,9 +563,9 @@ __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restri
             for (int a = 0; a < 6; ++a) y[a] = lanes_sum<kRowLanes>(y[a]);
             if (i < f.N && sub == 0) {
                 // to node-centred coordinates: T^T (a, b) = (a + b x g, b)
-                y[0] += y[4] * (Acc)gi.z - y[5] * (Acc)gi.y;
-                y[1] += y[5] * (Acc)gi.x - y[3] * (Acc)gi.z;
-                y[2] += y[3] * (Acc)gi.y - y[4] * (Acc)gi.x;
+                y[0] += y[4] * (float)gi.z - y[5] * (float)gi.y;
+                y[1] += y[5] * (float)gi.x - y[3] * (float)gi.z;
+                y[2] += y[3] * (float)gi.y - y[4] * (float)gi.x;
                 if (kEpi == kEpiAdjoint) {
 #pragma unroll
                     for (int a = 0; a < 6; ++a) b.q[6 * i + a] = (float)y[a];
@@ -578,35 +578,35 @@ __global__ void __launch_bounds__(256) mfr_gather_kernel(const Buffers* __restri
                             bz = tv[3] * gi.y - tv[4] * gi.x;
                 const float damp[6] = {tv[0] + bx, tv[1] + by, tv[2] + bz, tv[3], tv[4], tv[5]};
 #pragma unroll
-                for (int a = 0; a < 6; ++a) y[a] += (Acc)(1e-2f * damp[a]);
+                for (int a = 0; a < 6; ++a) y[a] += (float)(1e-2f * damp[a]);
                 if (kEpi == kEpiSpmv) {
 #pragma unroll
                     for (int a = 0; a < 6; ++a) {
                         b.q[6 * i + a] = (float)y[a];
-                        acc += (Acc)vi[a] * y[a];
+                        acc += (float)vi[a] * y[a];
                     }
                 } else if (kEpi == kEpiResidual) {
                     float rr[6], z[6];
 #pragma unroll
                     for (int a = 0; a < 6; ++a) {
-                        rr[a] = (float)((Acc)b.jtr[6 * i + a] - y[a]);
+                        rr[a] = (float)((float)b.jtr[6 * i + a] - y[a]);
                         b.r[6 * i + a] = rr[a];
                     }
-                    apply_minv<Acc>(b, i, rr, z);
+                    apply_minv<float>(b, i, rr, z);
 #pragma unroll
                     for (int a = 0; a < 6; ++a) {
                         b.d1[6 * i + a] = z[a];
-                        acc += (Acc)rr[a] * (Acc)z[a];
+                        acc += (float)rr[a] * (float)z[a];
                     }
                 } else {
 #pragma unroll
-                    for (int a = 0; a < 6; ++a) acc += (Acc)vi[a] * y[a];
+                    for (int a = 0; a < 6; ++a) acc += (float)vi[a] * y[a];
                 }
             }
         }
     }
     if (kEpi != kEpiAdjoint)
-        write_partial<Acc>(b, kEpi == kEpiSpmv ? kSlotDQ + k : (kEpi == kEpiResidual ? kSlotRefNum : kSlotRefDen), acc);
+        write_partial<float>(b, kEpi == kEpiSpmv ? kSlotDQ + k : (kEpi == kEpiResidual ? kSlotRefNum : kSlotRefDen), acc);
 }
 
 // Node-centred <-> reference coordinates of the debug products, in place on
@@ -971,18 +971,6 @@ __global__ void __launch_bounds__(256) mf_apply_terms_kernel(const Buffers* __re
     }
 }
 
-// One step of a wave's reduction of 2 kHalf values: the lane keeps the half
-// its lane bit names and adds the other lane's copies of it.
-template <int kHalf>
-__device__ inline void reduce_half(double (&v)[8]) {
-    const bool upper = (threadIdx.x & kHalf) != 0;
-#pragma unroll
-    for (int k = 0; k < kHalf; ++k) {
-        const double keep = upper ? v[k + kHalf] : v[k], send = upper ? v[k] : v[k + kHalf];
-        v[k] = keep + lane_xor<kHalf>(send);
-    }
-}
-
 // y_i over the Node2Term list of row i, then the epilogue: kEpiSpmv (v = d):
 // q and dot(d, q) of iteration k; kEpiResidual (v = x): r = b - A x, z = M^-1 r to
 // d1, (r, z); kEpiCurvature (v = z): (z, A z); kEpiAdjoint: the gather's sum to q.
@@ -1157,14 +1145,14 @@ static uint32_t gather_grid(const Batch& B) { return (mf_partials(B.nodes) + kXc
 static void mf_apply(const Batch& B, int src_epi, uint32_t k, uint32_t cur, const Penalty& pen, hipStream_t stream) {
     const dim3 tg(term_grid(B), B.frames), sg(row_group_grid(B.nodes), B.frames), wg(256);
     if (src_epi == 0) {
-        hipLaunchKernelGGL((mf_terms_kernel<float, kSrcDir>), tg, wg, 0, stream, B.dev, k, cur, pen);
-        hipLaunchKernelGGL((mf_gather_kernel<float, kEpiSpmv>), sg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_terms_kernel<kSrcDir>), tg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_gather_kernel<kEpiSpmv>), sg, wg, 0, stream, B.dev, k, cur, pen);
     } else if (src_epi == 1) {
-        hipLaunchKernelGGL((mf_terms_kernel<float, kSrcX>), tg, wg, 0, stream, B.dev, k, cur, pen);
-        hipLaunchKernelGGL((mf_gather_kernel<float, kEpiResidual>), sg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_terms_kernel<kSrcX>), tg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_gather_kernel<kEpiResidual>), sg, wg, 0, stream, B.dev, k, cur, pen);
     } else {
-        hipLaunchKernelGGL((mf_terms_kernel<float, kSrcZ>), tg, wg, 0, stream, B.dev, k, cur, pen);
-        hipLaunchKernelGGL((mf_gather_kernel<float, kEpiCurvature>), sg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_terms_kernel<kSrcZ>), tg, wg, 0, stream, B.dev, k, cur, pen);
+        hipLaunchKernelGGL((mf_gather_kernel<kEpiCurvature>), sg, wg, 0, stream, B.dev, k, cur, pen);
     }
 }
 
@@ -1172,14 +1160,14 @@ static void mfr_apply(const Batch& B, int src_epi, uint32_t k, uint32_t cur, con
                       hipStream_t stream) {
     const dim3 tg(term_grid(B), B.frames), sg(row_group_grid(B.nodes), B.frames), wg(256);
     if (src_epi == 0) {
-        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcDir, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
-        hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiSpmv>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_terms_kernel<kSrcDir, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_gather_kernel<kEpiSpmv>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
     } else if (src_epi == 1) {
-        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcX, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
-        hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiResidual>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_terms_kernel<kSrcX, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_gather_kernel<kEpiResidual>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
     } else {
-        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcZ, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
-        hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiCurvature>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_terms_kernel<kSrcZ, kOutG>), tg, wg, 0, stream, B.dev, k, cur, pen, which);
+        hipLaunchKernelGGL((mfr_gather_kernel<kEpiCurvature>), sg, wg, 0, stream, B.dev, k, cur, pen, which);
     }
 }
 
@@ -1288,11 +1276,11 @@ void launch_debug_jacobian(const Batch& B, bool fp64, bool transpose, uint32_t w
     }
     if (!transpose) {
         hipLaunchKernelGGL(mfr_coords_kernel, vg, wg, 0, stream, B.dev, 0);
-        hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcZ, kOutRows>), tg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
+        hipLaunchKernelGGL((mfr_terms_kernel<kSrcZ, kOutRows>), tg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
         return;
     }
-    hipLaunchKernelGGL((mfr_terms_kernel<float, float, kSrcRows, kOutG>), tg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
-    hipLaunchKernelGGL((mfr_gather_kernel<float, float, kEpiAdjoint>), sg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
+    hipLaunchKernelGGL((mfr_terms_kernel<kSrcRows, kOutG>), tg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
+    hipLaunchKernelGGL((mfr_gather_kernel<kEpiAdjoint>), sg, wg, 0, stream, B.dev, 0u, 0u, unit, which);
     hipLaunchKernelGGL(mfr_coords_kernel, vg, wg, 0, stream, B.dev, 1);
 }
 

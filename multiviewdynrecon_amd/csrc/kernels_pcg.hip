@@ -102,39 +102,29 @@ __device__ inline void row_apply(const Buffers& b, const BlockRow& row, const Ro
 #pragma unroll
     for (int a = 0; a < 6; ++a) y[a] = lanes_sum<kRowLanes>(y[a]);
 }
-// y = (A v)_i of a vector that is known.
-template <typename Acc>
-__device__ inline void row_apply(const Buffers& b, uint32_t i, uint32_t sub, const float* v, Acc y[6]) {
-    const BlockRow row(b, i);
-    RowEntry first;
-    first.load(b, row, sub, v, nullptr);
-    row_apply<Acc>(b, row, first, sub, v, nullptr, false, (Acc)0, y);
-}
-
 // r = b, d = M^-1 b, x = 0, partials of delta_0 = dot(r, d)
 // (blockPCGZeroInitKernel, BlockPCG.cuh:65-111, then cublasSdot).
-template <typename Acc>
 __global__ void __launch_bounds__(256) pcg_init_kernel(const Buffers* __restrict__ bs) {
     const Buffers b = frame_buffers(bs);
     const FrameDev& f = *b.frame;
-    Acc acc = 0;
+    float acc = 0;
     if (!b.counts->error) {
         const uint32_t stride = gridDim.x * blockDim.x;
         for (uint32_t n = blockIdx.x * blockDim.x + threadIdx.x; n < f.N; n += stride) {
             float rb[6], dv[6];
 #pragma unroll
             for (int a = 0; a < 6; ++a) rb[a] = b.jtr[6 * n + a];
-            apply_minv<Acc>(b, n, rb, dv);
+            apply_minv<float>(b, n, rb, dv);
 #pragma unroll
             for (int a = 0; a < 6; ++a) {
                 b.r[6 * n + a] = rb[a];
                 b.d0[6 * n + a] = dv[a];
                 b.x[6 * n + a] = 0.f;
-                acc += (Acc)rb[a] * (Acc)dv[a];
+                acc += (float)rb[a] * (float)dv[a];
             }
         }
     }
-    write_partial<Acc>(b, kSlotDelta + 0, acc);
+    write_partial<float>(b, kSlotDelta + 0, acc);
 }
 
 // Iteration k: q = A d with d = s + beta d_prev (k > 0); partials of dot(d, q).
@@ -243,73 +233,17 @@ __global__ void __launch_bounds__(256) pcg_update_kernel(const Buffers* __restri
     write_partial<Acc>(b, kSlotDelta + k + 1, acc);
 }
 
-// Residual refinement (mixed mode), one preconditioned steepest-descent step
-// on the true residual: r = b - A x, z = M^-1 r, num = dot(r, z) ...
-template <typename Acc>
-__global__ void __launch_bounds__(256) refine_residual_kernel(const Buffers* __restrict__ bs) {
-    const Buffers b = frame_buffers(bs);
-    const FrameDev& f = *b.frame;
-    const uint32_t sub = threadIdx.x % kRowLanes;
-    Acc acc = 0;
-    if (!b.counts->error) {
-        const uint32_t groups = gridDim.x * kRowsPerBlock;
-        for (uint32_t base = blockIdx.x * kRowsPerBlock; base < f.N; base += groups) {
-            const uint32_t i = base + threadIdx.x / kRowLanes;
-            Acc y[6];
-            row_apply<Acc>(b, i < f.N ? i : 0, sub, b.x, y);
-            if (i < f.N && sub == 0) {
-                float rr[6], z[6];
-#pragma unroll
-                for (int a = 0; a < 6; ++a) {
-                    rr[a] = (float)((Acc)b.jtr[6 * i + a] - y[a]);
-                    b.r[6 * i + a] = rr[a];
-                }
-                apply_minv<Acc>(b, i, rr, z);
-#pragma unroll
-                for (int a = 0; a < 6; ++a) {
-                    b.d1[6 * i + a] = z[a];
-                    acc += (Acc)rr[a] * (Acc)z[a];
-                }
-            }
-        }
-    }
-    write_partial<Acc>(b, kSlotRefNum, acc);
-}
-
-// ... den = dot(z, A z) ...
-template <typename Acc>
-__global__ void __launch_bounds__(256) refine_curvature_kernel(const Buffers* __restrict__ bs) {
-    const Buffers b = frame_buffers(bs);
-    const FrameDev& f = *b.frame;
-    const uint32_t sub = threadIdx.x % kRowLanes;
-    Acc acc = 0;
-    if (!b.counts->error) {
-        const uint32_t groups = gridDim.x * kRowsPerBlock;
-        for (uint32_t base = blockIdx.x * kRowsPerBlock; base < f.N; base += groups) {
-            const uint32_t i = base + threadIdx.x / kRowLanes;
-            Acc y[6];
-            row_apply<Acc>(b, i < f.N ? i : 0, sub, b.d1, y);
-            if (i < f.N && sub == 0) {
-#pragma unroll
-                for (int a = 0; a < 6; ++a) acc += (Acc)b.d1[6 * i + a] * y[a];
-            }
-        }
-    }
-    write_partial<Acc>(b, kSlotRefDen, acc);
-}
-
-// ... x += (num / den) z
-template <typename Acc>
+// x += (num / den) z of a refinement step (FP32 matrix-free solve).
 __global__ void __launch_bounds__(256) refine_step_kernel(const Buffers* __restrict__ bs, uint32_t spmv_blocks) {
     const Buffers b = frame_buffers(bs);
     const FrameDev& f = *b.frame;
-    Acc num, den;
-    reduce_partials2<Acc>(slot_ptr(b, kSlotRefNum), spmv_blocks, slot_ptr(b, kSlotRefDen), spmv_blocks, num, den);
+    float num, den;
+    reduce_partials2<float>(slot_ptr(b, kSlotRefNum), spmv_blocks, slot_ptr(b, kSlotRefDen), spmv_blocks, num, den);
     if (b.counts->error) return;
-    const Acc a = den > (Acc)0 ? num / den : (Acc)0;
+    const float a = den > (float)0 ? num / den : (float)0;
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 6 * f.N; i += stride)
-        b.x[i] = (float)((Acc)b.x[i] + a * (Acc)b.d1[i]);
+        b.x[i] = (float)((float)b.x[i] + a * (float)b.d1[i]);
 }
 
 // ------------------------------------------- fused CG (mixed precision mode)
@@ -770,7 +704,7 @@ __global__ void __launch_bounds__(256) cg_iter_kernel(const Buffers* __restrict_
 }
 
 // Residual refinement on the CG solution (preconditioned steepest descent on
-// the true residual, as refine_* above, in the A^ coordinates):
+// the true residual, in the A^ coordinates):
 // r^ = b^ - A^ x^, num = (r^, r^) ...
 __global__ void __launch_bounds__(256) cg_refine_residual_kernel(const Buffers* __restrict__ bs) {
     const WorkItem wi = frame_affine();
@@ -973,27 +907,17 @@ static uint32_t spmv_grid(uint32_t nodes) {
     return std::max<uint32_t>(kXcds, std::min<uint32_t>((g + kXcds - 1) / kXcds * kXcds, kPartialStride));
 }
 
-template <typename Acc>
-static void pcg_impl(const Batch& B, uint32_t iters, uint32_t refine, hipStream_t stream) {
+// Block-Jacobi PCG of the plain FP32 mode.
+void launch_pcg(const Batch& B, uint32_t iters, hipStream_t stream) {
     const uint32_t sg = spmv_grid(B.nodes);
     iters = std::min(iters, kMaxIters);
-    hipLaunchKernelGGL(pcg_init_kernel<Acc>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev);
+    hipLaunchKernelGGL(pcg_init_kernel, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev);
     uint32_t cur = 0;
     for (uint32_t k = 0; k < iters; ++k) {
-        hipLaunchKernelGGL(pcg_spmv_kernel<Acc>, dim3(sg, B.frames), dim3(256), 0, stream, B.dev, k, cur);
+        hipLaunchKernelGGL(pcg_spmv_kernel<float>, dim3(sg, B.frames), dim3(256), 0, stream, B.dev, k, cur);
         cur ^= 1;
-        hipLaunchKernelGGL(pcg_update_kernel<Acc>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, k, sg, cur);
+        hipLaunchKernelGGL(pcg_update_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, k, sg, cur);
     }
-    for (uint32_t r = 0; r < refine; ++r) {
-        hipLaunchKernelGGL(refine_residual_kernel<Acc>, dim3(sg, B.frames), dim3(256), 0, stream, B.dev);
-        hipLaunchKernelGGL(refine_curvature_kernel<Acc>, dim3(sg, B.frames), dim3(256), 0, stream, B.dev);
-        hipLaunchKernelGGL(refine_step_kernel<Acc>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, sg);
-    }
-}
-
-void launch_pcg(const Batch& B, uint32_t iters, uint32_t refine, bool fp64, hipStream_t stream) {
-    if (fp64) pcg_impl<double>(B, iters, refine, stream);
-    else pcg_impl<float>(B, iters, refine, stream);
 }
 
 // One ApplyJtJ (q = A d0, no direction update) for stage timing.
@@ -1083,7 +1007,7 @@ void launch_pair_blocks(const Batch& B, const Penalty& pen, hipStream_t stream) 
 
 // Steps of the FP32 matrix-free PCG.
 void launch_pcg_init(const Batch& B, hipStream_t stream) {
-    hipLaunchKernelGGL(pcg_init_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev);
+    hipLaunchKernelGGL(pcg_init_kernel, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev);
 }
 
 void launch_pcg_update(const Batch& B, uint32_t k, uint32_t spmv_blocks, uint32_t dsel, hipStream_t stream) {
@@ -1092,7 +1016,7 @@ void launch_pcg_update(const Batch& B, uint32_t k, uint32_t spmv_blocks, uint32_
 }
 
 void launch_refine_step(const Batch& B, uint32_t spmv_blocks, hipStream_t stream) {
-    hipLaunchKernelGGL(refine_step_kernel<float>, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, spmv_blocks);
+    hipLaunchKernelGGL(refine_step_kernel, dim3(kVecBlocks, B.frames), dim3(256), 0, stream, B.dev, spmv_blocks);
 }
 
 // The CG transform alone (launch tuning).

@@ -60,24 +60,12 @@ __device__ inline uint32_t pixel_u16(float u) {
 __device__ inline bool zero_vertex4(float4 v) { return fabsf(v.x) < 1e-3f && fabsf(v.y) < 1e-3f && fabsf(v.z) < 1e-3f; }
 
 // Wave sums of 32 values: lane l (and l + 32) returns the sum of value l & 31.
-// Each step halves the values a lane carries: it keeps the half its lane bit
-// names and adds the other lane's copies of it.
-template <int kHalf>
-__device__ inline void reduce_half(double (&v)[32], uint32_t lane) {
-    const bool upper = (lane & kHalf) != 0;
-#pragma unroll
-    for (int k = 0; k < kHalf; ++k) {
-        const double keep = upper ? v[k + kHalf] : v[k], send = upper ? v[k] : v[k + kHalf];
-        v[k] = keep + lane_xor<kHalf>(send);
-    }
-}
 __device__ inline double wave_sums32(double (&v)[32]) {
-    const uint32_t lane = threadIdx.x & 63;
-    reduce_half<16>(v, lane);
-    reduce_half<8>(v, lane);
-    reduce_half<4>(v, lane);
-    reduce_half<2>(v, lane);
-    reduce_half<1>(v, lane);
+    reduce_half<16>(v);
+    reduce_half<8>(v);
+    reduce_half<4>(v);
+    reduce_half<2>(v);
+    reduce_half<1>(v);
     return v[0] + lane_xor<32>(v[0]);
 }
 

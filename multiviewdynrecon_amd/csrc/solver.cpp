@@ -33,7 +33,7 @@ void launch_mf_update_once(const Batch& B, hipStream_t stream);
 void launch_spmv_once(const Batch& B, bool fp64, hipStream_t stream);
 void launch_pcg_update_once(const Batch& B, bool fp64, hipStream_t stream);
 uint32_t launch_cost(const Batch& B, const Penalty& pen, bool density_in_jtj, hipStream_t stream);
-void launch_pcg(const Batch& B, uint32_t iters, uint32_t refine, bool fp64, hipStream_t stream);
+void launch_pcg(const Batch& B, uint32_t iters, hipStream_t stream);
 void launch_apply_update(const Batch& B, uint32_t k, hipStream_t stream);
 void launch_cg_solve(const Batch& B, uint32_t iters, uint32_t refine, uint32_t k, const Penalty& pen,
                      hipStream_t stream);
@@ -211,7 +211,7 @@ void enqueue_batch(const Batch& B, const mvdr_solver_config& c, hipStream_t stre
         if (fp64) {
             launch_cg_solve(B, c.pcg_iterations, c.refine_steps, k, pen, stream);
         } else {
-            launch_pcg(B, c.pcg_iterations, 0, false, stream);
+            launch_pcg(B, c.pcg_iterations, stream);
             launch_apply_update(B, k, stream);
         }
     }
@@ -478,7 +478,9 @@ static size_t layout_buffers(const mvdr_solver_config& c, Buffers& b, FrameDev*&
     const bool factors64 = c.precision == MVDR_PRECISION_MIXED || mf;
     if (factors64) A(b.diag_inv64, 36 * (size_t)c.max_nodes);
     A(b.jtr, 6 * (size_t)c.max_nodes);
-    for (float** v : {&b.x, &b.r, &b.s, &b.q, &b.d0, &b.d1}) A(*v, 6 * (size_t)c.max_nodes);
+    for (float** v : {&b.x, &b.r, &b.q, &b.d1}) A(*v, 6 * (size_t)c.max_nodes);
+    if (!mf || !mixed)  // the mixed matrix-free solve has them in mf_rec
+        for (float** v : {&b.s, &b.d0}) A(*v, 6 * (size_t)c.max_nodes);
     if (factors64) A(b.linv64, kTri * (size_t)c.max_nodes);
     if (c.precision == MVDR_PRECISION_MIXED && !mf) {
         A(b.offhat, 36 * (size_t)b.cap_pairs);

@@ -41,6 +41,7 @@
 
 #include "../../include/mvdr/warpfield.h"
 #include "common.h"
+#include "device_util.h"
 
 namespace mvdr {
 namespace {
@@ -78,7 +79,7 @@ __device__ inline void heap_update(uint32_t d[4], uint32_t id[4], uint32_t idx, 
 // Maximum over each eight lanes, and over the wave (from lane 63, without LDS).
 template <int kCtrl, int kRows = 0xF>
 __device__ inline float dpp(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), kCtrl, kRows, 0xF, false));
+    return __uint_as_float(lane_dpp<kCtrl, kRows>(__float_as_uint(v), __float_as_uint(v)));
 }
 __device__ inline float wave_max(float v) {
     v = fmaxf(v, dpp<0xB1>(v));        // lane ^ 1
@@ -93,7 +94,7 @@ __device__ inline float wave_max(float v) {
 // The same for the bits of squared distances (one instruction a step).
 template <int kCtrl, int kRows = 0xF>
 __device__ inline uint32_t max_dpp(uint32_t v) {
-    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xF, false));
+    return max(v, lane_dpp<kCtrl, kRows>(v));
 }
 __device__ inline uint32_t eight_max(uint32_t v) { return max_dpp<0x141>(max_dpp<0x4E>(max_dpp<0xB1>(v))); }
 __device__ inline uint32_t wave_max(uint32_t v) {
