@@ -12,7 +12,7 @@
 // nearest tap by a minimum of (squared-distance bits, scan position), which is
 // the first strict minimum of the scan).  With one thread per pixel the few
 // edge pixels of a wave walked 2 x 441 taps each in a chain, at one or two
-// active lanes: 493 us for three 640x480 views, 29 us now (all passes 525 -> 60 us).
+// active lanes: 493 us for three 640x480 views, 17 us now (all passes 525 -> 49 us).
 // With many edges the taps' arithmetic bounds it: the pixel and its views are the
 // wave's (scalars), a tap's place follows from the last one's by additions, and a
 // window inside the image needs no bounds.  All passes, 2 / 10 / 50 / 100 % edge

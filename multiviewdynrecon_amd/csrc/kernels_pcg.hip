@@ -971,8 +971,8 @@ uint32_t transform_workgroups_for(uint32_t nodes, uint32_t frames) { return tran
 
 // Workgroups of a CG launch up to which all of them run at once with the deep reads'
 // registers, three to a CU (4k nodes: 6 frames 12.4 -> 12.1 us, 8 frames 12.3 -> 14.6).
-// Only one pass of rows is read ahead: launches of more (a tuned grid) gain nothing (8
-// frames of 64 workgroups 13.8 -> 14.6).
+// Only one pass of rows is read ahead: launches of more (a tuned grid) gain nothing (back
+// to back, 64 workgroups a frame: a lone frame 8.16 -> 8.36 us, 8 frames 12.85 -> 13.0).
 constexpr uint32_t kCgDeepWorkgroups = 3 * 256;
 static void launch_cg_iter(const Batch& B, uint32_t i, uint32_t grid, hipStream_t stream) {
     if (grid >= cg_partials(B.nodes) && (uint64_t)grid * B.frames <= kCgDeepWorkgroups)
