@@ -24,7 +24,9 @@ def lib():
 
 def mat34(m):
     out = _abi.Mat34()
-    v = m.tolist() if getattr(m, "ndim", 0) == 1 else [float(x) for x in m[:12]]  # flat arrays in one step
+    # flat arrays of real numbers in one step
+    flat = getattr(m, "ndim", 0) == 1 and getattr(getattr(m, "dtype", None), "kind", "f") in "fiub"
+    v = m.tolist() if flat else [float(x) for x in m[:12]]
     out.rot[:] = v[:9]
     out.trans[:] = v[9:12]
     return out
