@@ -15,10 +15,11 @@
 // active lanes: 493 us for three 640x480 views, 17 us now (all passes 525 -> 49 us).
 // With many edges the taps' arithmetic bounds it: the pixel and its views are the
 // wave's (scalars), a tap's place follows from the last one's by additions, and a
-// window inside the image needs no bounds.  All passes, 2 / 10 / 50 / 100 % edge
-// pixels of three 640x480 views: 70 / 192 / 773 / 1557 us; a division per tap and
-// addresses per lane 87 / 297 / 1291 / 2442; a thread per pixel 641 / 1129 / 1469 /
-// 1436 (its taps lie side by side, a wave's lie `step` apart: from ~90 % on it wins).
+// window inside the image needs no bounds.  A frame of almost nothing but edge pixels
+// takes a thread per pixel again.  All passes, 2 / 10 / 50 / 100 % edge pixels of three
+// 640x480 views, every second tap: 70 / 192 / 780 / 909 us (by waves alone 1560); a
+// division per tap and addresses per lane 87 / 297 / 1291 / 2442; a thread per pixel
+// throughout 636 / 1135 / 1485 / 1433.
 // The list's order is arbitrary and no result depends on it: candidates and the
 // per-target 64-bit minimum (squared-distance bits << 32 | source pixel) are kept
 // per pixel, and the three lists are compacted in pixel order.
@@ -204,39 +205,83 @@ __device__ inline float nearest_in_view(const CvFrame& f, const CvBuffers& b, ui
     return best;
 }
 
-// Stage 1: one candidate per listed edge pixel, one wave each; the per-target
-// minimum.
-__global__ void __launch_bounds__(256) cv_candidates_kernel(CvFrame f, CvBuffers b) {
-    const uint32_t plane = f.W * f.H;
-    const uint32_t count = min(*b.num_edges, b.cap_edges);
-    const uint32_t waves = gridDim.x * (blockDim.x / 64);
-    uint32_t w = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
-    if (w >= count) return;
-    do {
-        const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane((int)b.edges[w]);
-        const uint32_t v = p / plane;
-        float4 src;
-        if (f.V < 2 || v >= f.V || !edge_vertex(f, v, p - v * plane, src)) continue;
-        const f3 world = f.init[v].apply(xyz(src));
-        float best = __int_as_float(0x7f800000);
-        uint2 cand = make_uint2(kNoCandidate, 0u);
-        const uint32_t next = (v + 1) % f.V, last = (v + f.V - 1) % f.V;
-        for (int k = 0; k < 2; ++k) {
-            const uint32_t n = k == 0 ? next : last;
-            if (k == 1 && last == next) break;
-            uint32_t bx, by;
-            const float d2 = nearest_in_view(f, b, n, f.init_inv[n].apply(world), bx, by);
+// The same by one thread for a frame of mostly edge pixels: the taps of neighbouring
+// threads lie side by side, a wave's taps `step` apart.
+__device__ inline float nearest_by_thread(const CvFrame& f, const CvBuffers& b, uint32_t n, f3 q, uint32_t& bx, uint32_t& by) {
+    float best = __int_as_float(0x7f800000);
+    bx = by = 0;
+    if (!(q.z > 0.f)) return best;
+    const uint32_t side = 2 * (uint32_t)b.radius / (uint32_t)b.step + 1;
+    const uint32_t x0 = (uint32_t)project_round<float>(q.x, q.z, f.fx[n], f.cx[n]) - (uint32_t)b.radius;
+    const uint32_t y0 = (uint32_t)project_round<float>(q.y, q.z, f.fy[n], f.cy[n]) - (uint32_t)b.radius;
+    const uint8_t* edge = f.edge[n];
+    const float4* vertex = f.vertex[n];
+    for (uint32_t iy = 0, y = y0; iy < side; ++iy, y += (uint32_t)b.step)
+        for (uint32_t ix = 0, x = x0; ix < side; ++ix, x += (uint32_t)b.step) {
+            if (x >= f.W || y >= f.H || edge[y * f.W + x] != 1) continue;  // negative coordinates wrap above both sizes
+            const float4 v = vertex[y * f.W + x];
+            if (zero_vertex(v)) continue;
+            const float dx = v.x - q.x, dy = v.y - q.y, dz = v.z - q.z;
+            const float d2 = dx * dx + dy * dy + dz * dz;
             if (d2 < best) {
                 best = d2;
-                cand = make_uint2(bx | (by << 16), n);
+                bx = x;
+                by = y;
             }
         }
-        if (!(best < b.max_d2)) continue;
-        if ((threadIdx.x & 63) == 0) {
-            b.cand[p] = cand;
-            const uint32_t t = cand.y * plane + (cand.x >> 16) * f.W + (cand.x & 0xFFFF);
-            atomicMin(&b.best[t], ((unsigned long long)__float_as_uint(best) << 32) | p);
+    return best;
+}
+
+// The candidate of source pixel p (at vertex src of view v) and the per-target minimum.
+template <bool kWave>
+__device__ inline void find_candidate(const CvFrame& f, const CvBuffers& b, uint32_t p) {
+    const uint32_t plane = f.W * f.H, v = p / plane;
+    float4 src;
+    if (f.V < 2 || v >= f.V || !edge_vertex(f, v, p - v * plane, src)) return;
+    const f3 world = f.init[v].apply(xyz(src));
+    float best = __int_as_float(0x7f800000);
+    uint2 cand = make_uint2(kNoCandidate, 0u);
+    const uint32_t next = (v + 1) % f.V, last = (v + f.V - 1) % f.V;
+    for (int k = 0; k < 2; ++k) {
+        const uint32_t n = k == 0 ? next : last;
+        if (k == 1 && last == next) break;
+        uint32_t bx, by;
+        const f3 q = f.init_inv[n].apply(world);
+        const float d2 = kWave ? nearest_in_view(f, b, n, q, bx, by) : nearest_by_thread(f, b, n, q, bx, by);
+        if (d2 < best) {
+            best = d2;
+            cand = make_uint2(bx | (by << 16), n);
         }
+    }
+    if (!(best < b.max_d2)) return;
+    if (!kWave || (threadIdx.x & 63) == 0) {
+        b.cand[p] = cand;
+        const uint32_t t = cand.y * plane + (cand.x >> 16) * f.W + (cand.x & 0xFFFF);
+        atomicMin(&b.best[t], ((unsigned long long)__float_as_uint(best) << 32) | p);
+    }
+}
+
+// Stage 1: one candidate per edge pixel, one wave each from the list; where more than
+// 7/8 of the pixels are edges, a thread per pixel of the frame (100 %: 909 us against
+// 1560 with every second tap, 3230 against 3773 with every tap, where the two meet at
+// about 85 %; 70 % by waves 1080 and 2640).  Eight waves to a SIMD: left to itself the
+// compiler gives the two paths other registers, and 2 % edges take 75 us in place of 70.
+__global__ void __launch_bounds__(kCvThreads, 8) cv_candidates_kernel(CvFrame f, CvBuffers b) {
+    const uint32_t count = min(*b.num_edges, b.cap_edges), pixels = f.V * f.W * f.H;
+    if (count > pixels - pixels / 8) {
+        uint32_t p = blockIdx.x * kCvThreads + threadIdx.x;
+        if (p >= pixels) return;
+        do {
+            const uint32_t v = p / (f.W * f.H);
+            if (f.edge[v][p - v * (f.W * f.H)] == 1) find_candidate<false>(f, b, p);
+        } while (cv_step(p, gridDim.x * kCvThreads, pixels));
+        return;
+    }
+    const uint32_t waves = gridDim.x * (kCvThreads / 64);
+    uint32_t w = blockIdx.x * (kCvThreads / 64) + (threadIdx.x >> 6);
+    if (w >= count) return;
+    do {
+        find_candidate<true>(f, b, (uint32_t)__builtin_amdgcn_readfirstlane((int)b.edges[w]));
     } while (cv_step(w, waves, count));
 }
 

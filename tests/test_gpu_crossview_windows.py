@@ -35,3 +35,20 @@ def test_wide_windows(radius, step):
     h.FindCrossViewEdgeMatchedPairs()
     want = oracle_lists(cv, cfg)
     assert lists(h) == want and len(want[0]) > 0
+
+
+@pytest.mark.parametrize("spare", [255, 256, 257])
+@pytest.mark.parametrize("step", [1, 2])
+def test_mostly_edges(step, spare):
+    """Either side of 7/8 edge pixels, where threads take over from waves."""
+    W, H = 32, 32
+    cv = frame(7, 2, W, H, None)
+    for view, n in zip(cv.views, (spare // 2, spare - spare // 2)):
+        view.maps["edge_mask"].reshape(-1)[n:2 * n] = 0
+    assert sum(int((v.maps["edge_mask"] == 1).sum()) for v in cv.views) == 2 * W * H - spare
+    cfg = default_config(max_width=W, max_height=H, search_radius=4, search_step=step)
+    h = CrossViewEdgeCorrespondence(cfg)
+    ci, keep = crossview_input(cv, device="cuda")
+    h.SetCrossViewMatchingInput(ci)
+    h.FindCrossViewEdgeMatchedPairs()
+    assert lists(h) == oracle_lists(cv, cfg)
