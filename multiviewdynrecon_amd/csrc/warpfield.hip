@@ -10,21 +10,22 @@
 //               box of its vertices, a lane per box; the nodes of a box pass through
 //               scalar registers (every lane looks at the same node; from LDS the
 //               reads alone took as long as the arithmetic), asked for one box ahead.
-//   nodes     : a wave per node where there are few; a lane per box and then per node
-//               of the next eight near boxes; the few that beat the worst slot are
-//               inserted one after another.  (A thread per node filled 16 workgroups
-//               of 256.)  An insertion is the whole wave's then, so more nodes take
-//               eight lanes each, and most a thread each, as the vertices.
+//   nodes     : lanes of its own to a node, a lane per box and then per node of the
+//               next near boxes; the few that beat the worst slot are inserted one after
+//               another.  (A thread per node filled 16 workgroups of 256.)  The lanes of
+//               a node repeat its insertions, so the more nodes, the fewer lanes each:
+//               a wave or a row of 16 in the graph, a row or a thread, as the vertices,
+//               in the skinning.
 // Bound by the chain of insertions and the arithmetic around it (the memory traffic
 // is 8 MB).  How many there are depends on the order of the nodes; the most are
 // on a line that comes nearer, all of them.  us of a call, a thread per point -> here:
-//   body scene, 159k surfels, 4018 nodes: skinning 431 -> 195, graph 794 -> 89
-//     surfels in no order (their boxes exclude nothing) 533 -> 451, nodes in no order
-//     363 -> 154 and 759 -> 54, both 368 -> 261
-//   281k surfels in no order, 7500 nodes: skinning 1096 -> 1046
+//   body scene, 159k surfels, 4018 nodes: skinning 431 -> 185, graph 796 -> 88
+//     surfels in no order (their boxes exclude nothing) 533 -> 454, nodes in no order
+//     364 -> 154 and 757 -> 53, both 368 -> 262
+//   281k surfels in no order, 7500 nodes: skinning 1099 -> 1052
 //   20k points in no order and nodes on a line, 600 / 1000 / 2000 / 4000 / 8192 / 65535 nodes:
-//     skinning 87 / 143 / 283 / 559 / 1143 / 9013 -> 86 / 141 / 257 / 507 / 743 / 5964
-//     graph 162 / 272 / 533 / 1065 / 2236 / 17925 -> 66 / 107 / 210 / 492 / 1352 / 12579
+//     skinning 87 / 143 / 284 / 556 / 1146 / 8988 -> 52 / 82 / 157 / 330 / 772 / 5931
+//     graph 161 / 274 / 531 / 1069 / 2226 / 17970 -> 67 / 107 / 210 / 486 / 1345 / 17427
 //
 // The warps are streaming passes bound by HBM (a 16-32 B read and write per point plus
 // the L2-resident warp-field gathers).
@@ -49,7 +50,7 @@ namespace {
 constexpr uint32_t kBoxNodes = 8;       // nodes per box
 constexpr uint32_t kBoxes = 512;        // boxes in LDS at a time (4096 nodes, 16 KB)
 constexpr int kGraphNeighbours = 8;     // nodesGraphNeigboursNum
-constexpr uint32_t kGraphWaves = 8;     // waves per workgroup of the graph search
+constexpr uint32_t graph_threads(uint32_t lanes) { return lanes == 64 ? 512 : 256; }  // per workgroup of the graph search
 
 // Squared distances are compared by their bits: at least +0, they are ordered alike (a
 // not-a-number comes last), and integer minima and maxima need no canonical operands.
@@ -220,66 +221,52 @@ __device__ inline void scan_for_point(const float4* __restrict__ nodes, uint32_t
     }
 }
 
-// The value of lane j of each eight lanes, in all of them.
+// The value of lane j of each row of 16 lanes, in all of them, and their bits of a ballot.
 template <uint32_t j>
-__device__ inline float eight_lane(float v) {
-    const float own = dpp<(j % 4) * 0x55>(v), other = dpp<0x141>(own);  // of the lane's four, of the other four
-    return (threadIdx.x & 4) == (j & 4) ? own : other;
-}
-// The lane's eight lanes of a ballot.
-__device__ inline uint32_t eight_bits(bool p) { return (uint32_t)(__ballot(p) >> (threadIdx.x & 56)) & 0xFFu; }
+__device__ inline float row_lane(float v) { return dpp<0x150 + j>(v); }
+__device__ inline uint32_t row_bits(bool p) { return (uint32_t)(__ballot(p) >> (threadIdx.x & 48)) & 0xFFFFu; }
 
-// Passes the nodes that may enter the slots of eight points, one to each eight lanes
-// (`me`), in index order: a lane per box, then per node of the point's next near box.
+// Inserts where a row may have a hit: lane j's node is first + j for j < 8, second + j - 8 after.
+template <uint32_t j = 0, class Slots>
+__device__ inline void insert_hits(Slots& slots, uint32_t hits, uint32_t first, uint32_t second, float d) {
+    if (hits & (1u << j)) slots.insert(j < kBoxNodes ? first + j : second + j - kBoxNodes, row_lane<j>(d));
+    if constexpr (j < 15) insert_hits<j + 1>(slots, hits, first, second, d);
+}
+
+// Passes the nodes that may enter the slots of four points, one to each row of 16 lanes
+// (`me`), in index order: a lane per box, then per node of the point's next two near boxes.
 //   slots.bound()             the farthest slot
 //   slots.distance(me, q)     slots.wants(d): whether a distance may be inserted
-//   slots.insert(k, d)        node k at distance d, where wanted; equal in the eight lanes
+//   slots.insert(k, d)        node k at distance d, where wanted; equal in the row
 template <class Slots>
-__device__ inline void scan_for_eight(const float4* __restrict__ nodes, uint32_t num_nodes, float4 me, NodeTile& tile,
-                                      Slots& slots) {
-    const uint32_t sub = threadIdx.x % kBoxNodes;
-    const float inf = __int_as_float(0x7f800000);
+__device__ inline void scan_for_row(const float4* __restrict__ nodes, uint32_t num_nodes, float4 me, NodeTile& tile,
+                                    Slots& slots) {
+    const uint32_t lane = threadIdx.x & 15;
     for (uint32_t base = 0; base < num_nodes; base += kTileNodes) {
         const uint32_t n = min(kTileNodes, num_nodes - base), boxes = build_boxes(nodes, base, n, tile);
-        float4 lo = tile.lo[min(sub, boxes - 1)], hi = tile.hi[min(sub, boxes - 1)];
-        for (uint32_t b0 = 0; b0 < boxes; b0 += kBoxNodes) {
+        float4 lo = tile.lo[min(lane, boxes - 1)], hi = tile.hi[min(lane, boxes - 1)];
+        for (uint32_t b0 = 0; b0 < boxes; b0 += 16) {
             const float away = box_distance(me, me, lo, hi);
-            uint32_t near = eight_bits(b0 + sub < boxes && may_be_nearer(away, slots.bound()));
-            const uint32_t mine = min(b0 + kBoxNodes + sub, boxes - 1);  // the next step's box loads meanwhile
+            uint32_t near = row_bits(b0 + lane < boxes && may_be_nearer(away, slots.bound()));
+            const uint32_t mine = min(b0 + 16 + lane, boxes - 1);  // the next step's box loads meanwhile
             lo = tile.lo[mine];
             hi = tile.hi[mine];
             while (__any(near != 0)) {
-                // two boxes at a time
-                uint32_t k[2];
-                float d[2];
-#pragma unroll
-                for (uint32_t p = 0; p < 2; ++p) {
-                    k[p] = (b0 + (near ? (uint32_t)__builtin_ctz(near) : 0u)) * kBoxNodes;
-                    const float4 q = tile.node[k[p] + sub];
-                    d[p] = near != 0 && k[p] + sub < n ? slots.distance(me, q) : inf;
-                    near &= near - 1;
-                }
-                bool any = false;
-#pragma unroll
-                for (uint32_t p = 0; p < 2; ++p) {
-                    uint64_t hits = __ballot(slots.wants(d[p]));
-                    if (!hits) continue;
-                    any = true;
-                    hits |= hits >> 32;
-                    hits |= hits >> 16;
-                    hits |= hits >> 8;
-                    const uint32_t first = base + k[p];
-                    if (hits & 1) slots.insert(first, eight_lane<0>(d[p]));
-                    if (hits & 2) slots.insert(first + 1, eight_lane<1>(d[p]));
-                    if (hits & 4) slots.insert(first + 2, eight_lane<2>(d[p]));
-                    if (hits & 8) slots.insert(first + 3, eight_lane<3>(d[p]));
-                    if (hits & 16) slots.insert(first + 4, eight_lane<4>(d[p]));
-                    if (hits & 32) slots.insert(first + 5, eight_lane<5>(d[p]));
-                    if (hits & 64) slots.insert(first + 6, eight_lane<6>(d[p]));
-                    if (hits & 128) slots.insert(first + 7, eight_lane<7>(d[p]));
-                }
+                const uint32_t rest = near & (near - 1);
+                const uint32_t first = (b0 + (near ? (uint32_t)__builtin_ctz(near) : 0u)) * kBoxNodes;
+                const uint32_t second = (b0 + (rest ? (uint32_t)__builtin_ctz(rest) : 0u)) * kBoxNodes;
+                const uint32_t k = (lane < kBoxNodes ? first : second) + lane % kBoxNodes;
+                const bool live = (lane < kBoxNodes ? near : rest) != 0 && k < n;
+                near = rest & (rest - 1);
+                const float4 q = tile.node[k];
+                const float d = live ? slots.distance(me, q) : __int_as_float(0x7f800000);
+                uint64_t hits = __ballot(slots.wants(d));
+                if (!hits) continue;
+                hits |= hits >> 32;
+                hits |= hits >> 16;
+                insert_hits(slots, (uint32_t)hits, base + first, base + second, d);
                 // a box passed over is no nearer than the farthest slot, which only gets nearer
-                if (any) near &= eight_bits(may_be_nearer(away, slots.bound()));
+                near &= row_bits(may_be_nearer(away, slots.bound()));
             }
         }
     }
@@ -325,18 +312,16 @@ __device__ inline void put_skin(float4 pt, const SkinSlots& slots, const float4*
 
 constexpr uint32_t kSkinWaves = 4;  // waves per workgroup of the skinning
 
-// Lanes of a node in the skinning.  64 nodes in a row lie too far apart for boxes common
-// to them, so lanes of its own serve a node better, until the insertions of all nodes
-// fill the chip: a wave up to kSkinWaveNodes, eight lanes up to kSkinEightNodes, a
-// thread above (us; the listed order / a line that comes nearer, as above):
-//   600 nodes  wave  40 /   86, eight  44 /   81, thread  54 /  60
-//   2000       wave 103 /  327, eight 109 /  257, thread 121 / 183
-//   4000       wave 190 /  891, eight 195 /  507, thread 194 / 361
-//   7500, 8192 wave 327 / 2917, eight 337 / 1082, thread 336 / 743
-// A line's insertions by waves pass a thread per node (start of the file) at ~1000 nodes,
-// by eight lanes at ~8000.
-constexpr uint32_t kNodeWave = 64, kNodeEight = kBoxNodes, kNodeThread = 1;
-constexpr uint32_t kSkinWaveNodes = 1024, kSkinEightNodes = 6144;
+// 16 lanes to a node up to kSkinRowNodes, a thread above: 64 nodes in a row lie too far
+// apart for boxes common to them, so lanes of its own serve a node better, until the
+// insertions of all nodes fill the chip.  us; listed order / a line that comes nearer:
+//   600 nodes   16 lanes  40 /   51, thread  54 /   60, wave  40 /   85
+//   2000                 100 /  154,        121 /  183,      102 /  327
+//   4000                 186 /  326,        194 /  361,      188 /  888
+//   7500, 8192           312 /  766,        336 /  743,      323 / 2914
+//   12000 (no order)     455 / 1285,        468 / 1073,      468 / 5842
+constexpr uint32_t kNodeRow = 16, kNodeThread = 1;
+constexpr uint32_t kSkinRowNodes = 8192;
 
 // Workgroups of 256 vertices, then of nodes with lanes of their own; nodes by threads
 // come first, as the longest waves (4018 nodes 202 us, last 216).
@@ -358,8 +343,7 @@ __global__ void __launch_bounds__(64 * kSkinWaves)
     if (kNodeLanes != kNodeThread && is_node) {
         const uint32_t i = (block * blockDim.x + threadIdx.x) / kNodeLanes;
         const float4 me = nodes[min(i, num_nodes - 1)];
-        if constexpr (kNodeLanes == kNodeWave) scan_for_point(nodes, num_nodes, me, box, slots);
-        else scan_for_eight(nodes, num_nodes, me, shared.tile, slots);
+        scan_for_row(nodes, num_nodes, me, shared.tile, slots);
         if (i < num_nodes && threadIdx.x % kNodeLanes == 0) put_skin(me, slots, nodes, radius, nknn + i, nw + i);
         return;
     }
@@ -412,11 +396,11 @@ __global__ void __launch_bounds__(64 * kSkinWaves)
     if (p < num_vertices) put_skin(pt, slots, nodes, radius, vknn + p, vw + p);
 }
 
-// BuildNodesGraphKernel: 8 slots, the worst replaced (WarpField.cu:15-59).  Lane j
-// of the node's holds slot j: of its wave (kWave, lanes 8 on hold none) or of its eight.
-template <bool kWave>
+// BuildNodesGraphKernel: 8 slots, the worst replaced (WarpField.cu:15-59).  Lane j of
+// the node's wave or row of 16 lanes holds slot j; the lanes from 8 on hold none.
+template <uint32_t kLanes>
 struct GraphSlots {
-    float dist = !kWave || (threadIdx.x & 63) < kGraphNeighbours ? 1e5f : 0.f;
+    float dist = threadIdx.x % kLanes < kGraphNeighbours ? 1e5f : 0.f;
     int idx = -1;
     float worst_d = 1e5f;
     uint32_t worst = 0;
@@ -426,35 +410,40 @@ struct GraphSlots {
     }
     __device__ bool wants(float d) const { return d > 1e-6f && d < worst_d; }
     __device__ void insert(uint32_t k, float d) {
-        if ((kWave || wants(d)) && (threadIdx.x & (kWave ? 63 : 7)) == worst) {
+        // (the scan of a wave passes only wanted ones)
+        if ((kLanes == 64 || wants(d)) && threadIdx.x % kLanes == worst) {
             dist = d;
             idx = (int)k;
         }
         // the new worst slot: the first of the largest
-        const uint32_t m = eight_max(bits(dist));
-        worst_d = __uint_as_float(kWave ? (uint32_t)__builtin_amdgcn_readfirstlane((int)m) : m);
-        worst = kWave ? (uint32_t)__builtin_ctzll(__ballot(dist == worst_d)) : (uint32_t)__builtin_ctz(eight_bits(dist == worst_d));
+        const float m = __uint_as_float(eight_max(bits(dist)));
+        if constexpr (kLanes == 64) {
+            worst_d = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(m)));
+            worst = (uint32_t)__builtin_ctzll(__ballot(dist == worst_d));
+        } else {
+            worst_d = row_lane<0>(m);
+            worst = (uint32_t)__builtin_ctz(row_bits(dist == worst_d));
+        }
     }
 };
-static_assert(kGraphNeighbours == (int)kBoxNodes, "a lane per slot and per node of a box");
 
-// A wave per node up to kGraphWaveNodes, eight lanes above (us; random order / a line that
-// comes nearer): 4000 nodes 57 / 492 and 137 / 447, 8192 165 / 1352 and 240 / 918,
-// 12000 316 / 2495 and 328 / 1341, 20000 781 / 5974 and 588 / 2398.
-constexpr uint32_t kGraphWaveNodes = 12288;
-template <bool kWave>
-__global__ void __launch_bounds__(64 * kGraphWaves)
+// A wave per node up to kGraphWaveNodes, 16 lanes above.  us; random order / a line that
+// comes nearer: 4000 nodes 57 / 492 and 89 / 342, 8192 165 / 1379 and 161 / 740, 12000
+// 317 / 2555 and 239 / 1172, 65535 7106 / 54884 and 3671 / 17515 (listed order: 7500
+// nodes 161 and 204).  Workgroups of four waves with rows (of eight 159 / 779 at 8192).
+constexpr uint32_t kGraphWaveNodes = 8192;
+template <uint32_t kLanes>
+__global__ void __launch_bounds__(graph_threads(kLanes))
     node_graph_kernel(const float4* __restrict__ nodes, uint32_t num_nodes, ushort2* __restrict__ graph) {
-    constexpr uint32_t kLanes = kWave ? 64 : kBoxNodes;
     const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / kLanes, lane = threadIdx.x % kLanes;
     const float4 me = nodes[min(i, num_nodes - 1)];
-    GraphSlots<kWave> slots;
-    if constexpr (kWave) {
+    GraphSlots<kLanes> slots;
+    if constexpr (kLanes == 64) {
         __shared__ NodeBoxes box;
         scan_for_point(nodes, num_nodes, me, box, slots);
     } else {
         __shared__ NodeTile tile;
-        scan_for_eight(nodes, num_nodes, me, tile, slots);
+        scan_for_row(nodes, num_nodes, me, tile, slots);
     }
     if (i < num_nodes && lane < (uint32_t)kGraphNeighbours)
         graph[(size_t)i * kGraphNeighbours + lane] = make_ushort2((uint16_t)i, (uint16_t)slots.idx);
@@ -724,10 +713,10 @@ mvdr_status mvdr_warp_build_node_graph(const void* nodes, uint32_t num_nodes, vo
     hipStream_t st = static_cast<hipStream_t>(stream);
     const float4* n = static_cast<const float4*>(nodes);
     ushort2* g = static_cast<ushort2*>(graph);
-    const uint32_t per = num_nodes <= kGraphWaveNodes ? kGraphWaves : 64 * kGraphWaves / kBoxNodes;  // nodes per workgroup
-    const dim3 grid((num_nodes + per - 1) / per), wg(64 * kGraphWaves);
-    if (num_nodes <= kGraphWaveNodes) hipLaunchKernelGGL(node_graph_kernel<true>, grid, wg, 0, st, n, num_nodes, g);
-    else hipLaunchKernelGGL(node_graph_kernel<false>, grid, wg, 0, st, n, num_nodes, g);
+    const uint32_t lanes = num_nodes <= kGraphWaveNodes ? 64 : 16, threads = graph_threads(lanes);
+    const dim3 grid((num_nodes + threads / lanes - 1) / (threads / lanes)), wg(threads);
+    if (lanes == 64) hipLaunchKernelGGL(node_graph_kernel<64>, grid, wg, 0, st, n, num_nodes, g);
+    else hipLaunchKernelGGL(node_graph_kernel<16>, grid, wg, 0, st, n, num_nodes, g);
     return hipGetLastError() == hipSuccess ? MVDR_OK : MVDR_E_HIP;
 }
 
@@ -740,10 +729,10 @@ mvdr_status mvdr_warp_skin(const void* vertices, uint32_t num_vertices, const vo
     const uint64_t total = (uint64_t)num_vertices + num_nodes;
     if (total > 0xFFFFFFFFull - 255) return MVDR_E_SHAPE;
     constexpr uint32_t kSkinThreads = 64 * kSkinWaves;
-    const uint32_t lanes = num_nodes <= kSkinWaveNodes ? kNodeWave : num_nodes <= kSkinEightNodes ? kNodeEight : kNodeThread;
-    const uint32_t per = kSkinThreads / lanes;  // nodes per workgroup
+    const bool row = num_nodes <= kSkinRowNodes;
+    const uint32_t per = kSkinThreads / (row ? kNodeRow : kNodeThread);  // nodes per workgroup
     const dim3 grid((num_vertices + kSkinThreads - 1) / kSkinThreads + (num_nodes + per - 1) / per);
-    auto* kernel = lanes == kNodeWave ? skin_kernel<kNodeWave> : lanes == kNodeEight ? skin_kernel<kNodeEight> : skin_kernel<kNodeThread>;
+    auto* kernel = row ? skin_kernel<kNodeRow> : skin_kernel<kNodeThread>;
     hipLaunchKernelGGL(kernel, grid, dim3(kSkinThreads), 0, static_cast<hipStream_t>(stream),
                        static_cast<const float4*>(vertices), num_vertices, static_cast<const float4*>(nodes), num_nodes,
                        node_radius, static_cast<ushort4*>(vknn), static_cast<float4*>(vw), static_cast<ushort4*>(nknn),

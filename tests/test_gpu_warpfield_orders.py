@@ -1,8 +1,8 @@
-"""Node graph and skinning on the GPU around the node counts where a node's lanes change
-(a wave, eight, one: 1024, 6144; graph 12288) and the tiles of 1024 nodes, with nodes in
-no order, on a line that comes nearer (every node enters the slots) and on one that goes
-away; coincident nodes and nodes that are not finite.  Indices bit for bit against the
-oracle, weights within 1e-6 of it."""
+"""Node graph and skinning on the GPU around the node count where a node's lanes change
+(8192: a wave and 16 lanes in the graph, 16 lanes and one in the skinning) and the tiles
+of 1024 nodes, with nodes in no order, on a line that comes nearer (every node enters
+the slots) and on one that goes away; coincident nodes and nodes that are not finite.
+Indices bit for bit against the oracle, weights within 1e-6 of it."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("order", ["none", "nearer", "away"])
-@pytest.mark.parametrize("n", [1023, 1024, 1025, 1031, 2048, 2053, 6144, 6145, 12288, 12291])
+@pytest.mark.parametrize("n", [3, 17, 1023, 1024, 1025, 1031, 2048, 2053, 6144, 6145, 8191, 8192, 8193, 8201, 9217, 12288, 12291])
 def test_orders(n, order):
     rng = np.random.default_rng(n)
     nodes, pts = cloud(rng, n), cloud(rng, 131)
